@@ -44,7 +44,7 @@ class Sim2D(C.Structure):
                 ("src_add", vp), ("src_mul", vp), ("signal", vp), ("power", vp),
                 ("snap_x0", i32), ("snap_y0", i32), ("snap_sx", i32), ("snap_sy", i32), ("snap", vp),
                 ("stg", vp), ("stg_x0", i32), ("stg_y0", i32), ("stg_sx", i32), ("stg_sy", i32), ("coef", vp),
-                ("src_sel", vp), ("src_sig_len", i32)]
+                ("src_sel", vp), ("src_sig_len", i32), ("gc", vp)]
 
 
 class Adj2D(C.Structure):
@@ -54,7 +54,9 @@ class Adj2D(C.Structure):
                 ("src_mul", vp), ("box_x0", i32), ("box_y0", i32), ("box_sx", i32), ("box_sy", i32),
                 ("snap", vp), ("snap_step0", i32), ("grad", vp),
                 ("inj_x0", i32), ("inj_y0", i32), ("inj_sx", i32), ("inj_sy", i32), ("inj_w", vp), ("phasor", vp), ("nf", i32),
-                ("coef", vp), ("l2hist", vp), ("inj_tab", vp)]
+                ("coef", vp), ("l2hist", vp), ("inj_tab", vp), ("gc", vp)]
+
+TILE_ANCHORED = 0x40000000     # BZ_TILE_ANCHORED
 
 # name -> argtypes (restype is int unless listed in _RESTYPE)
 SIGNATURES = {

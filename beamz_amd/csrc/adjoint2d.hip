@@ -29,6 +29,8 @@
 // the forward step.
 #include "common.h"
 
+#include <type_traits>
+
 // No multiply-add contraction: the one-step and the two-step kernels round every operation alike, so a
 // pair of reverse steps gives the bits of two single steps.
 #pragma clang fp contract(off)
@@ -103,6 +105,19 @@ __device__ __forceinline__ void grad_at(const bz_adj2d& A, const Coef& c, int i,
     }
 }
 
+// The reverse update of every kernel below, in one arithmetic (the same bits in each): the y-spacing folded into
+// the coefficients (gb = fb * rdy, gc = cb * rdy, as in the forward kernels), r = rdx / rdy (exactly 1 on square
+// cells, where its products are exact):
+//   U   = gc lE''                               (0 off the interior)
+//   muX = lHx + (U(j,i+1) - U),  muY = lHy + r (U - U(j+1,i))
+//   lE  = ca lE'' + (gb muX - (gb muX)(j,i-1)) + r ((gb muY)(j-1,i) - gb muY),  lH = fa mu
+// Without conductivity fa = ca = 1 and the K-step kernel leaves those products out (11 operations per cell and
+// step instead of 14; with the spacings as separate products it took 18).
+__device__ __forceinline__ float mu_y(float r, float ly, float u, float ud) { return fmaf(r, u - ud, ly); }
+__device__ __forceinline__ float lam_e(float r, float cl2, float fmx, float fmxl, float fmyu, float fmy) {
+    return cl2 + fmaf(r, fmyu - fmy, fmx - fmxl);
+}
+
 template <int SEG>
 __global__ __launch_bounds__(LANES* WPG) void k_adj2d(const bz_adj2d* __restrict__ adjs, const int* __restrict__ tiles,
                                                      int ntiles, int n, int flip) {
@@ -122,6 +137,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d(const bz_adj2d* __restrict
     c.ke = A.ke;
     c.kbe = A.kbe;
     const float rdx = A.rdx, rdy = A.rdy;
+    const float rxy = rdx / rdy;
     const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
     const bool xin = i >= 1 && i <= nx - 2;
 
@@ -152,7 +168,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d(const bz_adj2d* __restrict
         const int j = j0 - 1 + r;
         l2[r] = src_mul_at(A, i, j) * le[r];
         e_coef(sg[r], ee[r], c, ca_[r], cb_[r]);
-        w[r] = (xin && j >= 1 && j <= ny - 2) ? cb_[r] * l2[r] : 0.0f;
+        w[r] = (xin && j >= 1 && j <= ny - 2) ? (cb_[r] * rdy) * l2[r] : 0.0f;
     }
     // fb muY on rows j0-1 .. j0+SEG-1, fb muX on rows j0 .. j0+SEG-1 (zero where the H entry does not exist)
     float fmy[SEG + 1], fmx[SEG + 1], fmxl[SEG + 1], my[SEG + 1], mx[SEG + 1], fa_[SEG + 1];
@@ -163,11 +179,12 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d(const bz_adj2d* __restrict
         float fa, fb;
         h_coef(sg[r], c, fa, fb);
         fa_[r] = fa;
-        my[r] = (j >= 0 && j <= ny - 2) ? ly[r] + (w[r] - w[r + 1]) * rdx : 0.0f;
-        fmy[r] = fb * my[r];
+        const float gb = fb * rdy;
+        my[r] = (j >= 0 && j <= ny - 2) ? mu_y(rxy, ly[r], w[r], w[r + 1]) : 0.0f;
+        fmy[r] = gb * my[r];
         const float wR = __shfl_down(w[r], 1, LANES);
-        mx[r] = hxok ? lx[r] + (wR - w[r]) * rdy : 0.0f;
-        fmx[r] = fb * mx[r];
+        mx[r] = hxok ? lx[r] + (wR - w[r]) : 0.0f;
+        fmx[r] = gb * mx[r];
         const float left = __shfl_up(fmx[r], 1, LANES);
         fmxl[r] = i >= 1 ? left : 0.0f;
     }
@@ -182,7 +199,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d(const bz_adj2d* __restrict
         if (out && j < ny) {
             const float ca = ca_[r], cb = cb_[r];
             const bool in = xin && j >= 1 && j <= ny - 2;
-            float lnew = (in ? ca * l2[r] : l2[r]) + (fmx[r] - fmxl[r]) * rdy + (fmy[r - 1] - fmy[r]) * rdx;
+            float lnew = lam_e(rxy, in ? ca * l2[r] : l2[r], fmx[r], fmxl[r], fmy[r - 1], fmy[r]);
             inject_at(A, lnew, i, j, n);
             put(ole, ro[r], lnew);
             put(olx, ro[r], fa_[r] * mx[r]);
@@ -227,6 +244,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
     c.ke = A.ke;
     c.kbe = A.kbe;
     const float rdx = A.rdx, rdy = A.rdy;
+    const float rxy = rdx / rdy;
     const bool xin = i >= 1 && i <= nx - 2;
     const bool hxok = i <= nx - 2;
     const bool out = l >= 2 && l <= LANES - 3 && i < nx;
@@ -239,14 +257,14 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
     float l2_0 = src_mul_at(A, i, rstart) * at(gle, off(rstart));
     float ca0, cb0;
     e_coef(sg0, ee0, c, ca0, cb0);
-    float w0 = interior(rstart) ? cb0 * l2_0 : 0.0f;
+    float w0 = interior(rstart) ? (cb0 * rdy) * l2_0 : 0.0f;
     // loads one row ahead: lE, sigma, eps of row r+1 and lHx, lHy of row r
     float nle = at(gle, off(rstart + 1)), nsg = at(A.sig, off(rstart + 1)), nee = at(A.eps, off(rstart + 1));
     float nlx = at(glx, off(rstart)), nly = at(gly, off(rstart));
     // carried from row r-1: fb muY of step n; step n's outputs there and its cell's coefficients for step n-1
     float fmy_p = 0.0f;
     float l2b_p = 0.0f, wb_p = 0.0f, lxn_p = 0.0f, lyn_p = 0.0f, fmyb_p = 0.0f;
-    float fa_p = 0.0f, fb_p = 0.0f, ca_p = 1.0f, cb_p = 0.0f, sg_p = 0.0f, ee_p = 1.0f;
+    float fa_p = 0.0f, gb_p = 0.0f, ca_p = 1.0f, cb_p = 0.0f, sg_p = 0.0f, ee_p = 1.0f;
     for (int r = rstart; r <= j1; ++r) {
         const float le1 = nle, sg1 = nsg, ee1 = nee, lx0 = nlx, ly0 = nly;
         {
@@ -261,36 +279,37 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
         const float l2_1 = src_mul_at(A, i, r + 1) * le1;
         float ca1, cb1;
         e_coef(sg1, ee1, c, ca1, cb1);
-        const float w1 = interior(r + 1) ? cb1 * l2_1 : 0.0f;
+        const float w1 = interior(r + 1) ? (cb1 * rdy) * l2_1 : 0.0f;
 
         // ---- reverse step n on row r ----
         float fa0, fb0;
         h_coef(sg0, c, fa0, fb0);
         const float wR = __shfl_down(w0, 1, LANES);
-        const float mx = hxok ? lx0 + (wR - w0) * rdy : 0.0f;
-        const float my = (r >= 0 && r <= ny - 2) ? ly0 + (w0 - w1) * rdx : 0.0f;
-        const float fmx = fb0 * mx, fmy = fb0 * my;
+        const float gb0 = fb0 * rdy;
+        const float mx = hxok ? lx0 + (wR - w0) : 0.0f;
+        const float my = (r >= 0 && r <= ny - 2) ? mu_y(rxy, ly0, w0, w1) : 0.0f;
+        const float fmx = gb0 * mx, fmy = gb0 * my;
         const float left = __shfl_up(fmx, 1, LANES);
         const float fmxl = i >= 1 ? left : 0.0f;
         const bool in0 = interior(r);
-        float lnew = (in0 ? ca0 * l2_0 : l2_0) + (fmx - fmxl) * rdy + (fmy_p - fmy) * rdx;
+        float lnew = lam_e(rxy, in0 ? ca0 * l2_0 : l2_0, fmx, fmxl, fmy_p, fmy);
         inject_at(A, lnew, i, r, n);
         const float lxn = fa0 * mx, lyn = fa0 * my;
         if (A.grad && out && in0 && r >= j0 && r < j1) grad_at(A, c, i, r, n, l2_0, ee0, sg0, cb0, rdx, rdy);
         // lam_n-side quantities of row r for step n-1 (same cell coefficients)
         const float l2b = src_mul_at(A, i, r) * lnew;
-        const float wbv = in0 ? cb0 * l2b : 0.0f;
+        const float wbv = in0 ? (cb0 * rdy) * l2b : 0.0f;
 
         // ---- reverse step n-1 on row m = r-1 ----
         const int m = r - 1;
         const float wbR = __shfl_down(wb_p, 1, LANES);
-        const float mx2 = hxok ? lxn_p + (wbR - wb_p) * rdy : 0.0f;
-        const float my2 = (m >= 0 && m <= ny - 2) ? lyn_p + (wb_p - wbv) * rdx : 0.0f;
-        const float fmx2 = fb_p * mx2, fmy2 = fb_p * my2;
+        const float mx2 = hxok ? lxn_p + (wbR - wb_p) : 0.0f;
+        const float my2 = (m >= 0 && m <= ny - 2) ? mu_y(rxy, lyn_p, wb_p, wbv) : 0.0f;
+        const float fmx2 = gb_p * mx2, fmy2 = gb_p * my2;
         const float left2 = __shfl_up(fmx2, 1, LANES);
         const float fmxl2 = i >= 1 ? left2 : 0.0f;
         const bool inm = interior(m);
-        float lnew2 = (inm ? ca_p * l2b_p : l2b_p) + (fmx2 - fmxl2) * rdy + (fmyb_p - fmy2) * rdx;
+        float lnew2 = lam_e(rxy, inm ? ca_p * l2b_p : l2b_p, fmx2, fmxl2, fmyb_p, fmy2);
         if (out && m >= j0 && m < j1) {
             inject_at(A, lnew2, i, m, n - 1);
             const uint32_t om = off(m);
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
         ca_p = ca0;
         cb_p = cb0;
         fa_p = fa0;
-        fb_p = fb0;
+        gb_p = gb0;
         sg_p = sg0;
         ee_p = ee0;
         l2b_p = l2b;
@@ -329,8 +348,15 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
 // n_top-K+1 on the whole region; the cells within K of its edge go stale one ring per step, the inner ones
 // are stored. w = cb lE'' plays Ez (muY needs w of the next row, muX w of the next column) and fb mu plays H
 // (lE needs fb muY of the previous row, fb muX of the previous column): right and left neighbours by DPP
-// wave shifts, band edges through LDS. Each inner cell is owned by one tile, which injects the objective
-// and accumulates its gradient, step by step in the one-step order. Reads buffer rb, writes rb ^ 1.
+// wave shifts; across band edges, w of the next band's first row and of the previous band's last row come through
+// LDS, and the previous band's last muY is kept by this wave too: one barrier per step, on alternating LDS slots.
+// Regions, their windows of stored cells (anchored tiles) and the waves without conductivity as in the forward
+// kernel. Each stored cell is owned by one tile, which accumulates its gradient, step by step in the one-step
+// order. Reads buffer rb, writes rb ^ 1.
+// Measured: the gradient of 16 designs of 600 x 600 cells, 3000 steps (reverse sweep, gradient pass, tables)
+// 39.1 -> 25.3 ms with one barrier per step, 11 instead of 18 operations per cell without conductivity, anchored
+// regions and the injection values of a launch staged in LDS. 99 registers: the gradient terms added in the sweep
+// (without l2hist) would spill at the 80 of the forward kernel.
 __device__ __forceinline__ float from_right(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, false));
 }
@@ -338,174 +364,289 @@ __device__ __forceinline__ float from_left(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, false));
 }
 
+// The part of the injection box inside a region.
+struct InjBox {
+    int x0, y0, sx, sy;
+};
+constexpr int INJ_LDS = 2048;   // injection values of a launch a workgroup holds (64 cells x 31 steps)
+
+// The lambda history of the design box (bz_adj2d.l2hist).
+struct HistBox {
+    int x0, y0, sx, sy, step0;
+};
+
 template <int B, int KW>
-__global__ __launch_bounds__(LANES* KW) void k_adj2d_tbk(const bz_adj2d* __restrict__ adjs,
+__global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_adj2d_tbk(const bz_adj2d* __restrict__ adjs,
                                                         const int* __restrict__ tiles, int ntiles, int K, int n_top,
                                                         int rb) {
     constexpr int RH = KW * B;
-    __shared__ float w_top[KW][LANES];
-    __shared__ float fmy_bot[KW][LANES];
-    __shared__ int ibox[4];     // the injection box (x0, y0, sx, sy), read after the first barrier
+    __shared__ float xw[2][2][KW][LANES];   // [step parity][first, last row of a band]: its w
+    __shared__ HistBox hbox;
+    __shared__ InjBox ibox;
+    __shared__ float injv[INJ_LDS];
     const int t = blockIdx.x;
     if (t >= ntiles) return;
-    const int s = tiles[3 * t];
-    if (s < 0) return;   // padding entry of a reordered tile list (uniform over the workgroup)
-    const bz_adj2d& A = adjs[s];
+    const int se = tiles[3 * t];
+    if (se < 0) return;   // padding entry of a reordered tile list (uniform over the workgroup)
+    const bool anch = se & BZ_TILE_ANCHORED;
+    const bz_adj2d& A = adjs[se & ~BZ_TILE_ANCHORED];
     const int tx = tiles[3 * t + 1], ty = tiles[3 * t + 2];
     const int nx = A.nx, ny = A.ny, ld = A.ld;
     const int l = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int rx0 = tx * (LANES - 2 * K) - K;
+    // region origin, and its window of stored cells [cx0, cx1) x [cy0, cy1)
+    const int rx0 = tx * (LANES - 2 * K) - (anch ? 0 : K), ry0 = ty * (RH - 2 * K) - (anch ? 0 : K);
+    const bool top = anch && ty == 0, bottom = anch && ry0 + RH >= ny;
+    const int cx0 = anch && tx == 0 ? 0 : K, cx1 = anch && rx0 + LANES >= nx ? LANES : LANES - K;
+    const int cy0 = top ? 0 : K, cy1 = bottom ? RH : RH - K;
     const int i = rx0 + l;
-    const int jb = ty * (RH - 2 * K) - K + w * B;
-    const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
-    Coef c;
-    c.kh = A.kh;
-    c.kbh = A.kbh;
-    c.ke = A.ke;
-    c.kbe = A.kbe;
-    const float rdx = A.rdx, rdy = A.rdy;
+    const int jb = ry0 + w * B;
+    const float rdy = A.rdy;
+    const float rxy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(A.rdx / rdy)));
     const bool xin = i >= 1 && i <= nx - 2;
     const bool hxok = i <= nx - 2;
-    const bool lane_inner = l >= K && l < LANES - K;
-    // uniform over the wave: does it meet the source box, the injection box, the design box (inner cells)
+    const bool lane_out = l >= cx0 && l < cx1 && i < nx;
+    // live steps of the wave and its edge class, as in the forward kernel
+    int klive = K;
+    if (!top) klive = min(klive, w * B + B - 1);
+    if (!bottom) klive = min(klive, RH - 1 - w * B);
+    if (jb >= ny || jb + B <= 0) klive = 0;
+    // uniform over the wave: does it meet the source box, the injection box, the design box (stored cells)
     const bool src_band = A.src_mul && jb < A.src_y0 + A.src_sy && jb + B > A.src_y0 && rx0 < A.src_x0 + A.src_sx &&
                           rx0 + LANES > A.src_x0;
     const bool inj_band = A.inj_w && jb < A.inj_y0 + A.inj_sy && jb + B > A.inj_y0 &&
                           rx0 < A.inj_x0 + A.inj_sx && rx0 + LANES > A.inj_x0;
-    // with the injection table, the next step's injection values are loaded one step ahead (their latency
-    // hides behind a whole step); the box comes from LDS, so it adds no registers
-    const float* __restrict__ itab = A.inj_tab;
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        ibox[0] = A.inj_x0;
-        ibox[1] = A.inj_y0;
-        ibox[2] = A.inj_sx;
-        ibox[3] = A.inj_sy;
-    }
-    float injv[B];
-    auto inj_fetch = [&](int nn) {       // values of step nn (0 outside the box or for nn < 1)
-#pragma unroll
-        for (int r = 0; r < B; ++r) {
-            const int a = i - ibox[0], bb = jb + r - ibox[1];
-            injv[r] = (nn >= 1 && a >= 0 && a < ibox[2] && bb >= 0 && bb < ibox[3])
-                          ? itab[(long)nn * ibox[2] * ibox[3] + (long)bb * ibox[2] + a]
-                          : 0.0f;
-        }
-    };
     const bool grad_band = A.grad && jb < A.box_y0 + A.box_sy && jb + B > A.box_y0 &&
-                           rx0 + K < A.box_x0 + A.box_sx && rx0 + LANES - K > A.box_x0;
-    const bool inner = jb >= 1 && jb + B - 1 <= ny - 2 && rx0 >= 1 && rx0 + LANES - 1 <= nx - 2;
-
-    float le[B], lx[B], ly[B], fa[B], fb[B], ca[B], cb[B];
+                           rx0 + cx0 < A.box_x0 + A.box_sx && rx0 + cx1 > A.box_x0;
+    // edge rules as in the forward kernel; the general form (2) also has the source's multiplier, the injection
+    // and the gradient terms added in the sweep
+    const bool xedge = rx0 < 1 || rx0 + LANES - 1 > nx - 2;
+    const int edge = jb < 1 || jb + B - 1 > ny - 2 || rxy != 1.0f || !A.coef || src_band || inj_band ||
+                             (grad_band && !A.l2hist)
+                         ? 2
+                         : (xedge ? 1 : 0);
+    // the design box, and the part of the injection box inside the region with its K steps' table values (sx 0:
+    // without the table or with more than INJ_LDS values the general form sums the injection itself), all written
+    // before the first barrier and read after it: from LDS they add no registers and no memory latency to a step
     {
+        const int x0 = max(A.inj_x0, rx0), x1 = min(A.inj_x0 + A.inj_sx, rx0 + LANES);
+        const int y0 = max(A.inj_y0, ry0), y1 = min(A.inj_y0 + A.inj_sy, ry0 + RH);
+        const bool meets = A.inj_w && A.inj_tab && x0 < x1 && y0 < y1;
+        const int sx = meets && (long)K * (x1 - x0) * (y1 - y0) <= INJ_LDS ? x1 - x0 : 0, sy = y1 - y0;
+        if (threadIdx.x == 0 && threadIdx.y == 0) ibox = InjBox{x0, y0, sx, sy};
+        for (int q = w * LANES + l; q < K * sx * sy; q += LANES * KW) {
+            const int k = q / (sx * sy), c = q - k * (sx * sy), n = n_top - k;
+            const long cell = (long)(y0 + c / sx - A.inj_y0) * A.inj_sx + (x0 + c % sx - A.inj_x0);
+            injv[q] = n >= 1 ? A.inj_tab[(long)n * A.inj_sx * A.inj_sy + cell] : 0.0f;
+        }
+    }
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        hbox = HistBox{A.box_x0, A.box_y0, A.box_sx, A.box_sy, A.snap_step0};
+    }
+
+    // the adjoint state, lHy of the row above the band (lyg), and gc = cb * rdy of cells without conductivity
+    float le[B], lx[B], ly[B], gc[B], lyg = 0.0f;
+    const float gb0 = A.kbh * rdy;                  // gb = fb * rdy of such a cell
+    bool lossy = true;
+#pragma unroll
+    for (int r = 0; r < B; ++r) le[r] = lx[r] = ly[r] = gc[r] = 0.0f;
+    const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
+    auto off = [&](int j) { return ((uint32_t)min(max(j, 0), ny - 1) * (uint32_t)ld + ic) * 4u; };
+    if (klive > 0) {
         const float* __restrict__ gle = A.le[rb];
         const float* __restrict__ glx = A.lhx[rb];
         const float* __restrict__ gly = A.lhy[rb];
-        const float* __restrict__ cf = A.coef;
-        uint32_t o[B];
+        const float* __restrict__ gcp = A.gc;
+        const bool one = edge == 0 && gcp;
+        float m = 0.0f;
+        if (one) {
+            m = at(gcp, off(jb - 1));
+#pragma unroll
+            for (int r = 0; r < B; ++r) gc[r] = at(gcp, off(jb + r));
+        }
 #pragma unroll
         for (int r = 0; r < B; ++r) {
-            o[r] = ((uint32_t)min(max(jb + r, 0), ny - 1) * (uint32_t)ld + ic) * 4u;
-            le[r] = at(gle, o[r]);
-            lx[r] = at(glx, o[r]);
-            ly[r] = at(gly, o[r]);
+            le[r] = at(gle, off(jb + r));
+            lx[r] = at(glx, off(jb + r));
+            ly[r] = at(gly, off(jb + r));
         }
-        if (cf) {
+        lyg = at(gly, off(jb - 1));
+        if (one) {
 #pragma unroll
             for (int r = 0; r < B; ++r) {
-                const float4 q = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(cf) + 4u * o[r]);
-                fa[r] = q.x;
-                fb[r] = q.y;
-                ca[r] = q.z;
-                cb[r] = q.w;
+                m = fminf(m, gc[r]);
+                gc[r] *= rdy;
             }
-        } else {
-#pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const float sg = at(A.sig, o[r]);
-                h_coef(sg, c, fa[r], fb[r]);
-                e_coef(sg, at(A.eps, o[r]), c, ca[r], cb[r]);
-            }
+            lossy = __ballot(m < 0.0f) != 0;
         }
     }
 
-    for (int k = 0; k < K; ++k) {
-        const int n = n_top - k;
-        // lE'' = M lE (kept in le) and w = cb lE'' on the interior
-        if (src_band) {
+    const int wd = min(w + 1, KW - 1), wu = max(w - 1, 0);   // edge waves read their own slot (stale rows)
+    auto steps = [&](auto lossy_c, auto edge_c) {
+        constexpr bool L = decltype(lossy_c)::value;
+        constexpr int E = decltype(edge_c)::value;
+        const float r1 = E == 2 ? rxy : 1.0f;
+        // the four coefficients of every cell, and fa, gb of the row above
+        float fa[B], gb[B], ca[B], gcl[B], fag = 1.0f, gbg = 0.0f;
+        if (L) {
+            const float* __restrict__ cf = A.coef;
+            if (E < 2 || cf) {
+                auto at4 = [&](uint32_t o) {
+                    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(cf) + o);
+                };
+                const float4 g4 = at4(4u * off(jb - 1));
+                fag = g4.x;
+                gbg = g4.y * rdy;
 #pragma unroll
-            for (int r = 0; r < B; ++r) le[r] = src_mul_at(A, i, jb + r) * le[r];
-        }
-        float wv[B];
+                for (int r = 0; r < B; ++r) {
+                    const float4 v = at4(4u * off(jb + r));
+                    fa[r] = v.x;
+                    gb[r] = v.y * rdy;
+                    ca[r] = v.z;
+                    gcl[r] = v.w * rdy;
+                }
+            } else {
+                Coef c;
+                c.kh = A.kh;
+                c.kbh = A.kbh;
+                c.ke = A.ke;
+                c.kbe = A.kbe;
 #pragma unroll
-        for (int r = 0; r < B; ++r) {
-            const int j = jb + r;
-            wv[r] = (inner || (xin && j >= 1 && j <= ny - 2)) ? cb[r] * le[r] : 0.0f;
-        }
-        // mu: muY of the band's last row needs w of the next band's first row
-        w_top[w][l] = wv[0];
-        __syncthreads();
-        if (itab && inj_band && k == 0) inj_fetch(n);     // the first step's values (ibox is written by now)
-        const float wb = w < KW - 1 ? w_top[w + 1][l] : wv[B - 1];
-        float fmx[B], fmy[B];
-#pragma unroll
-        for (int r = 0; r < B; ++r) {
-            const int j = jb + r;
-            const float wR = from_right(wv[r]);
-            const float wd = r < B - 1 ? wv[r + 1] : wb;
-            const float mx = (inner || hxok) ? lx[r] + (wR - wv[r]) * rdy : 0.0f;
-            const float my = (inner || (j >= 0 && j <= ny - 2)) ? ly[r] + (wv[r] - wd) * rdx : 0.0f;
-            fmx[r] = fb[r] * mx;
-            fmy[r] = fb[r] * my;
-            lx[r] = fa[r] * mx;
-            ly[r] = fa[r] * my;
-        }
-        // lE: the band's first row needs fb muY of the previous band's last row
-        fmy_bot[w][l] = fmy[B - 1];
-        __syncthreads();
-        const float fu = w > 0 ? fmy_bot[w - 1][l] : fmy[0];
-#pragma unroll
-        for (int r = 0; r < B; ++r) {
-            const int j = jb + r;
-            const float left = from_left(fmx[r]);
-            const float fmxl = (inner || i >= 1) ? left : 0.0f;
-            const float fmyu = r > 0 ? fmy[r - 1] : fu;
-            const bool in = inner || (xin && j >= 1 && j <= ny - 2);
-            const float l2 = le[r];
-            float lnew = (in ? ca[r] * l2 : l2) + (fmx[r] - fmxl) * rdy + (fmyu - fmy[r]) * rdx;
-            if (inj_band) {
-                if (itab) {
-                    const int a = i - ibox[0], bb = j - ibox[1];
-                    if (n >= 1 && a >= 0 && a < ibox[2] && bb >= 0 && bb < ibox[3]) lnew += injv[r];
-                } else {
-                    inject_at(A, lnew, i, j, n);
+                for (int r = -1; r < B; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);      // one row after the other: few registers at a time
+                    const float sg = at(A.sig, off(jb + r));
+                    float a, b, d, e;
+                    h_coef(sg, c, a, b);
+                    e_coef(sg, at(A.eps, off(jb + r)), c, d, e);
+                    if (r < 0) {
+                        fag = a;
+                        gbg = b * rdy;
+                    } else {
+                        fa[r] = a;
+                        gb[r] = b * rdy;
+                        ca[r] = d;
+                        gcl[r] = e * rdy;
+                    }
                 }
             }
-            const int rr = w * B + r;
-            if (grad_band && in && lane_inner && rr >= K && rr < RH - K) {
-                if (A.l2hist) {
-                    const int a = i - A.box_x0, bb = j - A.box_y0;
-                    if (a >= 0 && a < A.box_sx && bb >= 0 && bb < A.box_sy)
-                        A.l2hist[(long)(n - A.snap_step0) * A.box_sx * A.box_sy + (long)bb * A.box_sx + a] = l2;
-                } else {
-                    const uint32_t o = ((uint32_t)min(max(j, 0), ny - 1) * (uint32_t)ld + ic) * 4u;
-                    grad_at(A, c, i, j, n, l2, at(A.eps, o), at(A.sig, o), cb[r], rdx, rdy);
+        }
+        for (int k = 0; k < K; ++k) {
+            const int n = n_top - k;
+            float(*x)[KW][LANES] = xw[k & 1];
+            // lE'' = M lE (kept in le) and w = gc lE'' on the interior
+            float wv[B];
+            auto interior = [&](int r) { return E == 0 || (xin && (E < 2 || (jb + r >= 1 && jb + r <= ny - 2))); };
+            if (E == 2 && src_band) {
+#pragma unroll
+                for (int r = 0; r < B; ++r) le[r] = src_mul_at(A, i, jb + r) * le[r];
+            }
+            if (E == 2 && grad_band && !A.l2hist && k < klive) {     // gradient terms added in the sweep
+                Coef c;
+                c.kh = A.kh;
+                c.kbh = A.kbh;
+                c.ke = A.ke;
+                c.kbe = A.kbe;
+#pragma unroll
+                for (int r = 0; r < B; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int rr = w * B + r, j = jb + r;
+                    if (lane_out && rr >= cy0 && rr < cy1 && interior(r)) {
+                        const float sg = at(A.sig, off(j)), ee = at(A.eps, off(j));
+                        float ca1, cb1;
+                        e_coef(sg, ee, c, ca1, cb1);
+                        grad_at(A, c, i, j, n, le[r], ee, sg, cb1, A.rdx, rdy);
+                    }
                 }
             }
-            le[r] = lnew;
+#pragma unroll
+            for (int r = 0; r < B; ++r) {
+                const float u = (L ? gcl[r] : gc[r]) * le[r];
+                wv[r] = interior(r) ? u : 0.0f;
+            }
+            x[0][w][l] = wv[0];
+            x[1][w][l] = wv[B - 1];
+            __syncthreads();
+            if (k >= klive) continue;
+            const float wb = x[0][wd][l], wg = x[1][wu][l];
+            // lambda of the design cells into the history (a uniform base and 32-bit offsets)
+            if (grad_band && (E < 2 || A.l2hist)) {
+                const HistBox h = hbox;
+                const int hx0 = __builtin_amdgcn_readfirstlane(h.x0), hsx = __builtin_amdgcn_readfirstlane(h.sx);
+                const int hy0 = __builtin_amdgcn_readfirstlane(h.y0), hsy = __builtin_amdgcn_readfirstlane(h.sy);
+                float* hp = A.l2hist + (long)(n - __builtin_amdgcn_readfirstlane(h.step0)) * hsx * hsy;
+                const int a = i - hx0;
+                if (lane_out && a >= 0 && a < hsx)
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        const int rr = w * B + r, bb = jb + r - hy0;
+                        if (rr >= cy0 && rr < cy1 && bb >= 0 && bb < hsy) put(hp, (uint32_t)(bb * hsx + a) * 4u, le[r]);
+                    }
+            }
+            // the row above the band (its muY only), then the band: mu, lH and fb mu
+            float fmyu = 0.0f;
+            if (E < 2 || (jb >= 1 && jb <= ny - 1)) {
+                const float myg = mu_y(r1, lyg, wg, wv[0]);
+                fmyu = (L ? gbg : gb0) * myg;
+                lyg = L ? fag * myg : myg;
+            }
+#pragma unroll
+            for (int r = 0; r < B; ++r) {
+                const int j = jb + r;
+                const float wR = from_right(wv[r]);
+                const float wdn = r < B - 1 ? wv[r + 1] : wb;
+                float mx = lx[r] + (wR - wv[r]);
+                if (E > 0) mx = hxok ? mx : 0.0f;
+                float my = mu_y(r1, ly[r], wv[r], wdn);
+                if (E == 2) my = j >= 0 && j <= ny - 2 ? my : 0.0f;
+                const float g = L ? gb[r] : gb0;
+                const float fmx = g * mx, fmy = g * my;
+                lx[r] = L ? fa[r] * mx : mx;
+                ly[r] = L ? fa[r] * my : my;
+                float fmxl = from_left(fmx);
+                if (E > 0) fmxl = i >= 1 ? fmxl : 0.0f;
+                const float l2 = le[r];
+                float cl2 = l2;
+                if (L) {
+                    const float v = ca[r] * l2;
+                    cl2 = interior(r) ? v : l2;
+                }
+                le[r] = lam_e(r1, cl2, fmx, fmxl, fmyu, fmy);
+                fmyu = fmy;
+            }
+            if (E == 2 && inj_band && n >= 1) {
+                const InjBox h = ibox;
+#pragma unroll
+                for (int r = 0; r < B; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int a = i - h.x0, bb = jb + r - h.y0;
+                    if (h.sx == 0) inject_at(A, le[r], i, jb + r, n);
+                    else if (a >= 0 && a < h.sx && bb >= 0 && bb < h.sy) le[r] += injv[(k * h.sy + bb) * h.sx + a];
+                }
+            }
         }
-        if (itab && inj_band && k + 1 < K) inj_fetch(n - 1);   // the next step's values load during this one
-    }
+    };
+    // One form runs (tests of separate copies of its number, as in the forward kernel)
+    const int form = klive == 0 || (lossy && edge == 2) ? 3 : (lossy ? 1 + edge : 0);
+    auto is = [&](int f) {
+        int v = form;
+        asm volatile("" : "+s"(v));
+        return v == f;
+    };
+    using std::bool_constant;
+    if (is(0)) steps(bool_constant<false>{}, std::integral_constant<int, 0>{});
+    if (is(1)) steps(bool_constant<true>{}, std::integral_constant<int, 0>{});
+    if (is(2)) steps(bool_constant<true>{}, std::integral_constant<int, 1>{});
+    if (is(3)) steps(bool_constant<true>{}, std::integral_constant<int, 2>{});
 
-    // the inner cells hold lam_{n_top-K+1}
-    if (!lane_inner || i >= nx) return;
+    // the region's window holds lam_{n_top-K+1}
+    if (!lane_out) return;
     float* __restrict__ ole = A.le[rb ^ 1];
     float* __restrict__ olx = A.lhx[rb ^ 1];
     float* __restrict__ oly = A.lhy[rb ^ 1];
 #pragma unroll
     for (int r = 0; r < B; ++r) {
         const int rr = w * B + r, j = jb + r;
-        if (rr >= K && rr < RH - K && j < ny) {
+        if (rr >= cy0 && rr < cy1 && j < ny) {
             const uint32_t o = ((uint32_t)j * (uint32_t)ld + (uint32_t)i) * 4u;
             put(ole, o, le[r]);
             put(olx, o, lx[r]);

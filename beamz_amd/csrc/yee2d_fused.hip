@@ -98,22 +98,22 @@ __device__ __forceinline__ float box_amp(const bz_sim2d& S, long rr, int n, floa
 
 // The (Ez, Hx, Hy) updates of every kernel below, in one arithmetic: the y-spacing folded into the cell's
 // coefficients (gb = fb * rdy, gc = cb * rdy, each rounded once), r = rdx / rdy (exactly 1 on square cells,
-// where its products are exact), explicit fused multiply-adds. 11 to 12 vector operations per cell instead
-// of 18, and the same bits in every kernel.
+// where its products are exact), explicit fused multiply-adds, the same bits in every kernel.
 //   Hx' = fa Hx - gb (Ez[i+1] - Ez)            (= fa Hx - fb dEz/dy)
 //   Hy' = fa Hy + gb r (Ez[j+1] - Ez)          (= fa Hy + fb dEz/dx)
 //   Ez' = ca Ez + gc (r (Hy - Hy[j-1]) - (Hx - Hx[i-1]))
-// The field's own term is the multiply of the last fused multiply-add: a separate product (fa Hx) needs no
-// neighbour, so the compiler hoists it above the step's branches and holds it in registers.
+// The curl term is the multiply of the last fused multiply-add and the field's own product is rounded before
+// it: where fa = ca = 1 (no conductivity) that product is the field itself, so the K-step kernel leaves it out
+// there (8 vector operations per cell and step instead of 11) and still gives these bits.
 __device__ __forceinline__ float upd_hx(float fa, float gb, float hx, float ezR, float ez) {
-    return fmaf(fa, hx, -(gb * (ezR - ez)));
+    return fmaf(-gb, ezR - ez, fa * hx);
 }
 __device__ __forceinline__ float upd_hy(float fa, float gb, float r, float hy, float ed, float ez) {
-    return fmaf(fa, hy, gb * (r * (ed - ez)));
+    return fmaf(gb, r * (ed - ez), fa * hy);
 }
 __device__ __forceinline__ float upd_ez(float ca, float gc, float r, float ez, float hx, float hxl, float hy,
                                         float hu) {
-    return fmaf(ca, ez, gc * fmaf(r, hy - hu, -(hx - hxl)));
+    return fmaf(gc, fmaf(r, hy - hu, -(hx - hxl)), ca * ez);
 }
 
 // Monitor sample p of step n, read from the buffer step n wrote.
@@ -597,20 +597,29 @@ int run(const bz_sim2d* sims, const int* tiles, int ntiles, int* step, int nstep
 
 // ---------------- K steps per pass ----------------
 // A workgroup of KW waves takes one tile: a region of 64 columns x KW*B rows, wave w holding rows
-// w*B .. w*B+B-1 of it in registers (lane l = column), with the H and E coefficients of its cells computed
-// once. It advances the whole region K steps; the cells within K of the region's edge go stale one ring
-// per step (they lack neighbours outside the region), so after K steps the inner (64-2K) x (KW*B-2K) cells
-// hold step n+K and are stored. Tiles overlap by 2K cells, so one pass over HBM serves K steps.
-// Neighbours along a row come from wave shuffles, neighbours across band edges through LDS (two barriers
-// per step). Cells outside the grid compute garbage that never reaches a cell inside it: the update rules
-// read only in-grid neighbours for every updated in-grid entry. Monitor samples of each step are copied
-// from the owning tile to staging slot q & 1 of launch q, stage[q & 1][k][point], and accumulated into the
-// FP64 DFT in step order by extra workgroups of the next launch (by k_gather2d_k after the last one).
+// w*B .. w*B+B-1 of it in registers (lane l = column), with the H and E coefficients of its cells. It advances
+// the whole region K steps; the cells within K of a region edge inside the grid go stale one ring per step (they
+// lack neighbours outside the region), so after K steps the cells further in hold step n+K and are stored. Tiles
+// overlap by 2K cells, so one pass over HBM serves K steps. A region that starts or ends at the grid's edge
+// loses nothing there: an anchored tile list (BZ_TILE_ANCHORED) starts its first region at cell 0 and stores up
+// to the edge, so 256 cells take 5 regions of 64 (K = 8) instead of 6. Waves whose rows have all gone stale, or lie
+// outside the grid, only keep the barriers.
+// Neighbours along a row come from wave shifts; across band edges, Ez of the next band's first row and of the
+// previous band's last row come through LDS, and the previous band's last Hy (which Ez of the first row needs)
+// is kept by this wave too and advanced from those: one barrier per step, on alternating LDS slots, instead of
+// one before H and one before E.
+// A wave whose cells (and the row above them) have no conductivity reads one coefficient per cell (bz_sim2d.gc)
+// instead of four and runs the update without the fa and ca products.
+// Cells outside the grid compute garbage that never reaches a cell inside it: the update rules read only
+// in-grid neighbours for every updated in-grid entry. Monitor samples of each step are copied from the owning
+// tile to staging slot q & 1 of launch q, stage[q & 1][k][point], and accumulated into the FP64 DFT in step
+// order by extra workgroups of the next launch (by k_gather2d_k after the last one).
 // Reads buffer rd, writes rd ^ 1.
 // Update coefficients of every cell: blockIdx.y is the simulation, the x blocks stride over its cells.
 __global__ __launch_bounds__(256) void k_coef2d(const bz_sim2d* __restrict__ sims) {
     const bz_sim2d& S = sims[blockIdx.y];
     float* __restrict__ cf = S.coef;
+    float* __restrict__ gc = S.gc;
     if (!cf) return;
     Coef c;
     c.kh = S.kh;
@@ -623,6 +632,7 @@ __global__ __launch_bounds__(256) void k_coef2d(const bz_sim2d* __restrict__ sim
         h_coef(S.sig[o], c, fa, fb);
         e_coef(S.sig[o], S.eps[o], c, ca, cb);
         reinterpret_cast<float4*>(cf)[o] = make_float4(fa, fb, ca, cb);
+        if (gc) gc[o] = fa == 1.0f && ca == 1.0f && fb == c.kbh && cb > 0.0f ? cb : -1.0f;
     }
 }
 
@@ -673,20 +683,29 @@ __global__ void k_gather2d_k(Gather2D G, const float* __restrict__ stage, const 
     gather_k(G, stage, *step + K * q, K, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
+constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further ones are read again every step)
+
 // SEL: some simulation's source box holds several sources (bz_sim2d.src_sel); without it the per-cell
-// source lookup is compiled out, which keeps the kernel at the register count of four waves per SIMD.
+// source lookup is compiled out.
+// What bounds it: on many grids the load phase of a region beside vector issue (8 waves x 8 rows in 80 registers
+// let three workgroups of a CU overlap those; with 128 registers it was two), on one small grid the chain of a
+// step (LDS round trip, barrier, six dependent operations) and the launch itself. Measured, with 4-value
+// coefficients, two barriers per step, unanchored regions and 128 registers before: 64 grids of 256 x 256 cells
+// 7.3 -> 4.95 us/step, 16 grids of 600 x 600 cells 8.6 -> 5.8, twelve of 256..1024 a side 6.3 -> 4.5, one grid of
+// 800 x 400 cells with a 16-frequency line 1.33 (K = 12) -> 1.09 (K = 16).
 template <int B, int KW, bool SEL>
-__global__ __launch_bounds__(LANES* KW) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
+__global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                                                         const int* __restrict__ tiles, int ntiles, int K,
                                                         const int* __restrict__ step, int q, int rd,
                                                         const int* __restrict__ ent_start,
                                                         const int* __restrict__ ents, float* __restrict__ stage_all,
                                                         Gather2D G) {
     constexpr int RH = KW * B;
-    __shared__ float ez_top[KW][LANES];
-    __shared__ float hy_bot[KW][LANES];
-    __shared__ float amps[32];          // the signal's K <= 31 samples of this launch
-    extern __shared__ float smp[];      // [3][RH][LANES] when there are monitor points (launch-sized)
+    __shared__ float xe[2][2][KW][LANES];   // [step parity][first, last row of a band]: its Ez
+    __shared__ float amps[32];              // the signal's K <= 31 samples of this launch
+    __shared__ float wsrc[KW][B][LANES];    // source weights of the cells of the waves that meet the box
+    __shared__ SnapBox snq;
+    extern __shared__ float smp_all[];      // with monitor points: samples [KW][B][LANES], entries [KW][ELIST][2]
     const int npts = G.npts;
     const int t = blockIdx.x;
     if (t >= ntiles) {
@@ -696,192 +715,321 @@ __global__ __launch_bounds__(LANES* KW) void k_yee2d_tbk(const bz_sim2d* __restr
                  (long)(t - ntiles) * (LANES * KW) + threadIdx.y * LANES + threadIdx.x);
         return;
     }
-    float* __restrict__ stage = stage_all + (long)(q & 1) * K * npts;
-    const int s = tiles[3 * t];
-    if (s < 0) return;   // padding entry of a reordered tile list (uniform over the workgroup)
-    const bz_sim2d& S = sims[s];
+    const int se = tiles[3 * t];
+    if (se < 0) return;   // padding entry of a reordered tile list (uniform over the workgroup)
+    const bool anch = se & BZ_TILE_ANCHORED;
+    const bz_sim2d& S = sims[se & ~BZ_TILE_ANCHORED];
     const int tx = tiles[3 * t + 1], ty = tiles[3 * t + 2];
     const int nx = S.nx, ny = S.ny, ld = S.ld;
     const int l = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int i = tx * (LANES - 2 * K) - K + l;
-    const int jb = ty * (RH - 2 * K) - K + w * B;   // grid row of the wave's first register row
-    const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
+    // region origin, and its window of stored cells [cx0, cx1) x [cy0, cy1)
+    const int rx0 = tx * (LANES - 2 * K) - (anch ? 0 : K), ry0 = ty * (RH - 2 * K) - (anch ? 0 : K);
+    const bool top = anch && ty == 0, bottom = anch && ry0 + RH >= ny;
+    const int cx0 = anch && tx == 0 ? 0 : K, cx1 = anch && rx0 + LANES >= nx ? LANES : LANES - K;
+    const int cy0 = top ? 0 : K, cy1 = bottom ? RH : RH - K;
+    const int i = rx0 + l;
+    const int jb = ry0 + w * B;                     // grid row of the wave's first register row
     const int wr = rd ^ 1;
     const int n0 = *step + K * q;
-    Coef c;
-    c.kh = S.kh;
-    c.kbh = S.kbh;
-    c.ke = S.ke;
-    c.kbe = S.kbe;
-    const float rdx = S.rdx, rdy = S.rdy;
+    const float rdy = S.rdy;
     // 1 on square cells; uniform, so kept in a scalar register
-    const float rxy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(rdx / rdy)));
+    const float rxy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(S.rdx / rdy)));
     const bool hxok = i < nx - 1;
     const bool xin = i >= 1 && i <= nx - 2;
-    // the source box, held in registers (the step loop stores to memory, so fields read through S would be
-    // reloaded on every row)
-    const int sx0 = S.src_x0, sy0 = S.src_y0, ssx = S.src_sx, ssy = S.src_sy;
-    const float* __restrict__ sadd = S.src_add;
-    const float* __restrict__ smul = S.src_mul;
-    const float* __restrict__ sgl = S.signal;
-    const bool src_col = ssx > 0 && i >= sx0 && i < sx0 + ssx;
-    // does the source box meet this wave's rows and this region's columns (uniform over the wave)
-    const int rx0 = tx * (LANES - 2 * K) - K;
-    const bool src_band = ssx > 0 && jb < sy0 + ssy && jb + B > sy0 && rx0 < sx0 + ssx && rx0 + LANES > sx0;
-    // every row of the wave and every column of the region is interior to the grid (the usual case): no edge
-    // rules per row or per lane
-    const bool inner = jb >= 1 && jb + B - 1 <= ny - 2 && rx0 >= 1 && rx0 + LANES - 1 <= nx - 2;
-    // does the snapshot box meet this wave's rows and this region's inner columns (uniform over the wave)
-    // the snapshot box in LDS (written before the first barrier, read after it): in registers it would add
-    // scalar spills to every wave
-    __shared__ SnapBox snq;
-    if (threadIdx.x == 0 && threadIdx.y == 0) snq = snap_box(S);
+    const bool lane_out = l >= cx0 && l < cx1 && i < nx;
+    // the steps this wave has a live row for: after step k a band next to an open region edge holds valid rows
+    // from row k + 1 (up to row RH - 2 - k) on; none if every row lies outside the grid
+    int klive = K;
+    if (!top) klive = min(klive, w * B + B - 1);
+    if (!bottom) klive = min(klive, RH - 1 - w * B);
+    if (jb >= ny || jb + B <= 0) klive = 0;
+    // uniform over the wave: do the source box, and the snapshot box, meet its rows and this region's columns
+    const bool src_band = S.src_sx > 0 && jb < S.src_y0 + S.src_sy && jb + B > S.src_y0 &&
+                          rx0 < S.src_x0 + S.src_sx && rx0 + LANES > S.src_x0;
     const bool snap_band = S.snap && jb < S.snap_y0 + S.snap_sy && jb + B > S.snap_y0 &&
-                           rx0 + K < S.snap_x0 + S.snap_sx && rx0 + LANES - K > S.snap_x0;
-    const bool lane_inner = l >= K && l < LANES - K;
+                           rx0 + cx0 < S.snap_x0 + S.snap_sx && rx0 + cx1 > S.snap_x0;
+    // edge rules: 0 every row and column of the wave is interior to the grid (the usual case), 1 some column is
+    // not, 2 the general form: some row is not, the cells are not square (only this form has the r products), or
+    // there are no coefficient arrays (or, below, the wave has a source or monitor cells)
+    const bool xedge = rx0 < 1 || rx0 + LANES - 1 > nx - 2;
+    int edge = jb < 1 || jb + B - 1 > ny - 2 || rxy != 1.0f || !S.coef ? 2 : (xedge ? 1 : 0);
+    if (threadIdx.x == 0 && threadIdx.y == 0) snq = snap_box(S);   // written before the first barrier, read after it
+    // the launch's signal samples, staged in LDS and read after the step's barrier: a vector load inside the
+    // step loop would wait behind the snapshot and staging stores of the previous step (the vector memory
+    // counter retires in order)
+    const int tid = w * LANES + l;
+    if (tid < K) amps[tid] = S.signal ? gload(S.signal, n0 + tid) : 0.0f;
 
-    // fb and cb hold fb * rdy and cb * rdy (upd_hx, upd_hy, upd_ez)
-    float ez[B], hx[B], hy[B], fa[B], fb[B], ca[B], cb[B];
-    {
+    // the monitor entries of the tile whose rows are this wave's, compacted into its LDS list: (sample slot,
+    // (row * LANES + column) | comp << 16)
+    const int e0 = ent_start ? ent_start[t] : 0, e1 = ent_start ? ent_start[t + 1] : 0;
+    float* __restrict__ smp = smp_all + w * (B * LANES);
+    int2* __restrict__ list = reinterpret_cast<int2*>(smp_all + RH * LANES) + w * ELIST;
+    int nmine = 0;
+    auto entries = [&](auto use) {          // use(position among the wave's entries, slot, code) on its lane
+        int seen = 0;
+        for (int eb = e0; eb < e1; eb += LANES) {
+            const int e = eb + l;
+            const int code = e < e1 ? ents[2 * e + 1] : 0;
+            const bool m = e < e1 && (code >> 10) / B == w;
+            const unsigned long long mask = __ballot(m);
+            const int pos = seen + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+            if (m) use(pos, ents[2 * e], (((code >> 10) - w * B) * LANES + ((code >> 2) & 255)) | ((code & 3) << 16));
+            seen += __popcll(mask);
+        }
+        return seen;
+    };
+    if (e1 > e0)
+        nmine = entries([&](int pos, int pnt, int loc) {
+            if (pos < ELIST) list[pos] = make_int2(pnt, loc);
+        });
+    if (src_band || nmine > 0) edge = 2;    // the general form of the step samples and adds the source
+
+    // the fields, Hy of the row above the band (hyg), and gc = cb * rdy of cells without conductivity
+    float ez[B], hx[B], hy[B], gc[B], hyg = 0.0f;
+    const float gb0 = S.kbh * rdy;                  // gb = fb * rdy of such a cell
+    bool lossy = true;
+#pragma unroll
+    for (int r = 0; r < B; ++r) ez[r] = hx[r] = hy[r] = gc[r] = 0.0f;
+    const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
+    auto off = [&](int j) { return ((uint32_t)min(max(j, 0), ny - 1) * (uint32_t)ld + ic) * 4u; };
+    if (klive > 0) {
         const float* __restrict__ gez = S.ez[rd];
         const float* __restrict__ ghx = S.hx[rd];
         const float* __restrict__ ghy = S.hy[rd];
-        const float* __restrict__ cf = S.coef;
-        uint32_t o[B];
+        const float* __restrict__ gcp = S.gc;
+        const bool one = edge == 0 && gcp;
+        float m = 0.0f;
+        if (one) {
+            m = at(gcp, off(jb - 1));
+#pragma unroll
+            for (int r = 0; r < B; ++r) gc[r] = at(gcp, off(jb + r));
+        }
 #pragma unroll
         for (int r = 0; r < B; ++r) {
-            o[r] = ((uint32_t)min(max(jb + r, 0), ny - 1) * (uint32_t)ld + ic) * 4u;
-            ez[r] = at(gez, o[r]);
-            hx[r] = at(ghx, o[r]);
-            hy[r] = at(ghy, o[r]);
+            ez[r] = at(gez, off(jb + r));
+            hx[r] = at(ghx, off(jb + r));
+            hy[r] = at(ghy, off(jb + r));
         }
-        if (cf) {
-            // precomputed by k_coef2d (the same roundings), one 16-byte (fa, fb, ca, cb) per cell
+        hyg = at(ghy, off(jb - 1));
+        if (one) {
 #pragma unroll
             for (int r = 0; r < B; ++r) {
-                const float4 q = at4(cf, 4u * o[r]);
-                fa[r] = q.x;
-                fb[r] = q.y * rdy;
-                ca[r] = q.z;
-                cb[r] = q.w * rdy;
+                m = fminf(m, gc[r]);
+                gc[r] *= rdy;
             }
-        } else {
-#pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const float sg = at(S.sig, o[r]);
-                h_coef(sg, c, fa[r], fb[r]);
-                e_coef(sg, at(S.eps, o[r]), c, ca[r], cb[r]);
-                fb[r] *= rdy;
-                cb[r] *= rdy;
-            }
+            lossy = __ballot(m < 0.0f) != 0;
         }
     }
-    const int e0 = ent_start ? ent_start[t] : 0, e1 = ent_start ? ent_start[t + 1] : 0;
-    const int tid = w * LANES + l;
-    // the tile's monitor entries: thread tid stages entries e0 + tid, e0 + tid + LANES*KW, ...; the first one
-    // is read here, once for all K steps
-    const int ef = e0 + tid;
-    const int epnt = ef < e1 ? ents[2 * ef] : -1;
-    const int ecode = ef < e1 ? ents[2 * ef + 1] : 0;
 
-    // the launch's signal samples, staged in LDS and read after the step's barriers: a vector load inside the
-    // step loop would wait behind the snapshot and staging stores of the previous step (the vector memory
-    // counter retires in order)
-    if (sgl && tid < K) amps[tid] = gload(sgl, n0 + tid);
-    for (int k = 0; k < K; ++k) {
-        // H of step n0+k+1: Hy of the band's last row needs Ez of the next band's first row
-        ez_top[w][l] = ez[0];
-        __syncthreads();
-        const float ezb = w < KW - 1 ? ez_top[w + 1][l] : ez[B - 1];
-        auto h_rows = [&](auto check) {
-            constexpr bool C = decltype(check)::value;
+    const int wd = min(w + 1, KW - 1), wu = max(w - 1, 0);   // edge waves read their own slot (stale rows)
+    auto steps = [&](auto lossy_c, auto edge_c) {
+        constexpr bool L = decltype(lossy_c)::value;
+        constexpr int E = decltype(edge_c)::value;
+        // the four coefficients of every cell, and fa, gb of the row above
+        float fa[B], gb[B], ca[B], gcl[B], fag = 1.0f, gbg = 0.0f;
+        if (L) {
+            const float* __restrict__ cf = S.coef;
+            if (E < 2 || cf) {
+                // precomputed by k_coef2d (the same roundings), one 16-byte (fa, fb, ca, cb) per cell
+                const float4 g4 = at4(cf, 4u * off(jb - 1));
+                fag = g4.x;
+                gbg = g4.y * rdy;
 #pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const int j = jb + r;
-                const float ezR = from_right(ez[r]);
-                const float ed = r < B - 1 ? ez[r + 1] : ezb;
-                if (C) {
-                    const float hn = computed(upd_hx(fa[r], fb[r], hx[r], ezR, ez[r]));
-                    hx[r] = hxok ? hn : hx[r];
-                } else {
-                    hx[r] = upd_hx(fa[r], fb[r], hx[r], ezR, ez[r]);
+                for (int r = 0; r < B; ++r) {
+                    const float4 v = at4(cf, 4u * off(jb + r));
+                    fa[r] = v.x;
+                    gb[r] = v.y * rdy;
+                    ca[r] = v.z;
+                    gcl[r] = v.w * rdy;
                 }
-                if (!C || j < ny - 1) hy[r] = upd_hy(fa[r], fb[r], rxy, hy[r], ed, ez[r]);
-            }
-        };
-        if (inner) h_rows(std::false_type{});
-        else h_rows(std::true_type{});
-        // snapshot of call-relative step q*K+k at the inner cells: the Ez this step reads, the Hx, Hy it wrote
-        if (snap_band) {
+            } else {
+                Coef c;
+                c.kh = S.kh;
+                c.kbh = S.kbh;
+                c.ke = S.ke;
+                c.kbe = S.kbe;
 #pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const int rr = w * B + r;
-                if (rr >= K && rr < RH - K && lane_inner) snap_put(snq, q * K + k, i, jb + r, ez[r], hx[r], hy[r]);
-            }
-        }
-        // E: Ez of the band's first row needs the new Hy of the previous band's last row
-        hy_bot[w][l] = hy[B - 1];
-        __syncthreads();
-        const float hya = w > 0 ? hy_bot[w - 1][l] : hy[0];
-        auto e_rows = [&](auto check) {
-            constexpr bool C = decltype(check)::value;
-#pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const int j = jb + r;
-                const float hxl = from_left(hx[r]);
-                const float hu = r > 0 ? hy[r - 1] : hya;
-                if (!C) {
-                    ez[r] = upd_ez(ca[r], cb[r], rxy, ez[r], hx[r], hxl, hy[r], hu);
-                } else if (j >= 1 && j <= ny - 2) {
-                    const float en = computed(upd_ez(ca[r], cb[r], rxy, ez[r], hx[r], hxl, hy[r], hu));
-                    ez[r] = xin ? en : ez[r];
-                }
-            }
-        };
-        if (inner) e_rows(std::false_type{});
-        else e_rows(std::true_type{});
-        // the source box, after E (it touches only the Ez of its own cells)
-        if (src_band) {
-#pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const int j = jb + r;
-                if (j >= sy0 && j < sy0 + ssy && src_col) {
-                    const long rr = (long)(j - sy0) * ssx + (i - sx0);
-                    const float amp = sgl ? amps[k] : 0.0f;        // written before the first barrier
-                    const float a = SEL ? box_amp(S, rr, n0 + k, amp) : amp;
-                    ez[r] = (smul ? gload(smul, rr) : 1.0f) * ez[r] + gload(sadd, rr) * a;
+                for (int r = -1; r < B; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);      // one row after the other: few registers at a time
+                    const float sg = at(S.sig, off(jb + r));
+                    float a, b, d, e;
+                    h_coef(sg, c, a, b);
+                    e_coef(sg, at(S.eps, off(jb + r)), c, d, e);
+                    if (r < 0) {
+                        fag = a;
+                        gbg = b * rdy;
+                    } else {
+                        fa[r] = a;
+                        gb[r] = b * rdy;
+                        ca[r] = d;
+                        gcl[r] = e * rdy;
+                    }
                 }
             }
         }
-        // monitor samples of step n0+k owned by this tile, all three components behind one barrier. The next
-        // step's writes to smp come after its two barriers, which every thread reaches only after these reads.
-        if (e1 > e0) {
+        // the source's weights of this wave's cells (0 outside its box), loaded once, in LDS
+        const bool plain_src = E == 2 && src_band && !SEL && !S.src_mul;
+        auto src_cell = [&](int r) {
+            const int a = i - S.src_x0, b = jb + r - S.src_y0;
+            return a >= 0 && a < S.src_sx && b >= 0 && b < S.src_sy ? (long)b * S.src_sx + a : -1L;
+        };
+        if (E == 2 && src_band) {
 #pragma unroll
             for (int r = 0; r < B; ++r) {
-                const int o = (w * B + r) * LANES + l;
-                smp[o] = ez[r];
-                smp[RH * LANES + o] = hx[r];
-                smp[2 * RH * LANES + o] = hy[r];
+                const long o = src_cell(r);
+                wsrc[w][r][l] = o >= 0 ? gload(S.src_add, o) : 0.0f;
             }
+        }
+        for (int k = 0; k < K; ++k) {
+            float(*x)[KW][LANES] = xe[k & 1];
+            x[0][w][l] = ez[0];
+            x[1][w][l] = ez[B - 1];
             __syncthreads();
-            // code = (region row << 10) | (region column << 2) | component
-            auto sample = [&](int code) { return smp[((code & 3) * RH + (code >> 10)) * LANES + ((code >> 2) & 255)]; };
-            if (epnt >= 0) gstore(stage, (long)k * npts + epnt, sample(ecode));
-            for (int e = ef + LANES * KW; e < e1; e += LANES * KW)
-                gstore(stage, (long)k * npts + ents[2 * e], sample(ents[2 * e + 1]));
+            if (k < klive) {
+                const float ezb = x[0][wd][l], ezg = x[1][wu][l];
+                // what the source adds at the end of this step: with few rows per wave (the small grids' shapes, where
+                // a step's latency counts) read and multiplied here, off the step's chain
+                float add[B], amp = 0.0f;
+                // (four LDS reads at a time, then selects: no wait for each read in turn)
+                auto src_adds = [&](int r0) {
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = wsrc[w][r0 + r][l];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float a = computed(v[r] * amp);
+                        add[r0 + r] = v[r] != 0.0f ? a : 0.0f;
+                    }
+                };
+                if (E == 2 && src_band) amp = amps[k];
+                if (plain_src && B <= 4) src_adds(0);
+                // H: the row above the band (its Hy only), then the band
+                hyg = L ? upd_hy(fag, gbg, E == 2 ? rxy : 1.0f, hyg, ez[0], ezg) : fmaf(gb0, ez[0] - ezg, hyg);
+#pragma unroll
+                for (int r = 0; r < B; ++r) {
+                    const float ezR = from_right(ez[r]);
+                    const float ed = r < B - 1 ? ez[r + 1] : ezb;
+                    if (!L) {
+                        hx[r] = fmaf(-gb0, ezR - ez[r], hx[r]);
+                        hy[r] = fmaf(gb0, ed - ez[r], hy[r]);
+                    } else {
+                        const float hn = computed(upd_hx(fa[r], gb[r], hx[r], ezR, ez[r]));
+                        hx[r] = E == 0 || hxok ? hn : hx[r];
+                        if (E < 2 || jb + r < ny - 1)
+                            hy[r] = upd_hy(fa[r], gb[r], E == 2 ? rxy : 1.0f, hy[r], ed, ez[r]);
+                    }
+                }
+                // snapshot of call-relative step q*K+k at the stored cells: the Ez this step reads, the Hx, Hy it
+                // wrote
+                if (snap_band) {        // a uniform base per plane and 32-bit offsets
+                    const SnapBox sn = snq;
+                    const int qx0 = __builtin_amdgcn_readfirstlane(sn.x0), qsx = __builtin_amdgcn_readfirstlane(sn.sx);
+                    const int qy0 = __builtin_amdgcn_readfirstlane(sn.y0), qsy = __builtin_amdgcn_readfirstlane(sn.sy);
+                    float* p0 = S.snap + (long)(q * K + k) * 3 * qsx * qsy;
+                    float* p1 = p0 + (long)qsx * qsy;
+                    float* p2 = p1 + (long)qsx * qsy;
+                    const int a = i - qx0;
+                    if (lane_out && a >= 0 && a < qsx)
+#pragma unroll
+                        for (int r = 0; r < B; ++r) {
+                            const int rr = w * B + r, b = jb + r - qy0;
+                            if (rr >= cy0 && rr < cy1 && b >= 0 && b < qsy) {
+                                const uint32_t o = (uint32_t)(b * qsx + a) * 4u;
+                                put(p0, o, ez[r]);
+                                put(p1, o, hx[r]);
+                                put(p2, o, hy[r]);
+                            }
+                        }
+                }
+                // E
+#pragma unroll
+                for (int r = 0; r < B; ++r) {
+                    const float hxl = from_left(hx[r]);
+                    const float hu = r > 0 ? hy[r - 1] : hyg;
+                    if (!L) {
+                        ez[r] = fmaf(gc[r], (hy[r] - hu) - (hx[r] - hxl), ez[r]);
+                    } else if (E < 2 || (jb + r >= 1 && jb + r <= ny - 2)) {
+                        const float en =
+                            computed(upd_ez(ca[r], gcl[r], E == 2 ? rxy : 1.0f, ez[r], hx[r], hxl, hy[r], hu));
+                        ez[r] = E == 0 || xin ? en : ez[r];
+                    }
+                }
+                // the source box, after E (it touches only the Ez of its own cells)
+                if (plain_src) {
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        if (B > 4 && r % 4 == 0) src_adds(r);
+                        ez[r] += add[r];
+                    }
+                } else if (E == 2 && src_band) {
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        const long o = src_cell(r);
+                        if (o >= 0)
+                            ez[r] = (S.src_mul ? gload(S.src_mul, o) : 1.0f) * ez[r] +
+                                    wsrc[w][r][l] * (SEL ? box_amp(S, o, n0 + k, amp) : amp);
+                    }
+                }
+            }
+            // monitor samples of step n0+k: the wave's rows of one component after the other go through its own LDS
+            // rows, and the lanes read their entries' cells back between them (no workgroup barrier and no wait in
+            // between: a wave's LDS operations complete in order)
+            if (E == 2 && nmine > 0) {
+                float* __restrict__ stage = stage_all + ((long)(q & 1) * K + k) * npts;
+                for (int eb = 0; eb < min(nmine, ELIST); eb += LANES) {
+                    const int2 ent = list[min(eb + l, nmine - 1)];
+                    float val = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+                        for (int r = 0; r < B; ++r) smp[r * LANES + l] = c == 0 ? ez[r] : (c == 1 ? hx[r] : hy[r]);
+                        __builtin_amdgcn_wave_barrier();
+                        const float v = smp[ent.y & 0xffff];
+                        val = (ent.y >> 16) == c ? v : val;
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                    if (eb + l < nmine) gstore(stage, ent.x, val);
+                }
+                // the entries beyond the list
+                for (int c = 0; c < 3 && nmine > ELIST; ++c) {
+#pragma unroll
+                    for (int r = 0; r < B; ++r) smp[r * LANES + l] = c == 0 ? ez[r] : (c == 1 ? hx[r] : hy[r]);
+                    __builtin_amdgcn_wave_barrier();
+                    entries([&](int pos, int pnt, int loc) {
+                        if (pos >= ELIST && (loc >> 16) == c) gstore(stage, pnt, smp[loc & 0xffff]);
+                    });
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
         }
-    }
+    };
+    // One form runs. Written as tests of separate copies of its number, not as an else chain: the compiler lays
+    // divergent code out in sequence, and a chain's later forms would keep their inputs, the 3 B field registers,
+    // alive beside an earlier form's results (98 instead of 72 registers at B = 8).
+    const int form = klive == 0 || (lossy && edge == 2) ? 3 : (lossy ? 1 + edge : 0);
+    auto is = [&](int f) {
+        int v = form;
+        asm volatile("" : "+s"(v));
+        return v == f;
+    };
+    using std::bool_constant;
+    if (is(0)) steps(bool_constant<false>{}, std::integral_constant<int, 0>{});
+    if (is(1)) steps(bool_constant<true>{}, std::integral_constant<int, 0>{});
+    if (is(2)) steps(bool_constant<true>{}, std::integral_constant<int, 1>{});
+    if (is(3)) steps(bool_constant<true>{}, std::integral_constant<int, 2>{});
 
-    // the inner cells of the region hold step n0+K
-    if (l < K || l >= LANES - K || i >= nx) return;
+    // the region's window holds step n0+K
+    if (!lane_out) return;
     float* __restrict__ oez = S.ez[wr];
     float* __restrict__ ohx = S.hx[wr];
     float* __restrict__ ohy = S.hy[wr];
 #pragma unroll
     for (int r = 0; r < B; ++r) {
         const int rr = w * B + r, j = jb + r;
-        if (rr >= K && rr < RH - K && j < ny) {
+        if (rr >= cy0 && rr < cy1 && j < ny) {
             const uint32_t o = ((uint32_t)j * (uint32_t)ld + (uint32_t)i) * 4u;
             put(oez, o, ez[r]);
             put(ohx, o, hx[r]);
@@ -894,8 +1042,8 @@ template <int B, int KW>
 int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int K, int* step, int rd0, int nlaunch,
          const int* ent_start, const int* ents, float* stage, const Gather2D& G, bool sel, hipStream_t st) {
     const dim3 b(LANES, KW);
-    // sample staging in LDS, [3][KW*B][LANES] floats, only when there are monitor points
-    const size_t lds = G.npts > 0 ? 3u * KW * B * LANES * sizeof(float) : 0;
+    // sample staging and entry lists in LDS, only when there are monitor points
+    const size_t lds = G.npts > 0 ? (size_t)KW * (B * LANES * sizeof(float) + ELIST * sizeof(int2)) : 0;
     const long gather_threads = (long)G.npts * (G.nfreq > 0 ? G.nfreq : 1);
     const int gather_blocks = (int)((gather_threads + LANES * KW - 1) / (LANES * KW));
     // the gather of launch q-1 runs as extra workgroups of launch q; the last launch's gets a launch of its own

@@ -268,6 +268,7 @@ class AdjointProblem2D:
             eng = self.fwd if self.full else self.rec
             cf = eng.coefs[b] if eng.kstep and eng.coefs is not None else None
             d.coef = cf.data_ptr() if cf is not None else None
+            d.gc = eng.gcs[b].data_ptr() if cf is not None else None
             descs.append(d)
         return descs
 

@@ -611,14 +611,21 @@ class Grid:
         return True
 
 
+def anchored_regions(n, size, K):
+    """Regions of ``size`` cells that cover an axis of n cells in K-step passes: a region loses K cells at each
+    end inside the grid and none at the grid's own edges (BZ_TILE_ANCHORED), so the first and the last store
+    size - K cells and those between size - 2K."""
+    return max(1, -(-(n - 2 * K) // (size - 2 * K)))
+
+
 def kstep_owner_tables(tiles, pts, dims, K, rh):
     """Monitor-point owner tables of the K-step kernel (bz_yee2d_runk).
 
     tiles: (ntiles, 3) = (sim, x-tile, y-tile) in units of the inner size (64 - 2K) x (rh - 2K), sim < 0 for
-    padding; pts: (npts, 3) = (sim, comp, offset into [ny][ld]); dims: (nsims, 3) = (nx, ny, ld). Each point
-    belongs to the tile whose inner cells hold it. Returns (start, ents): start[t] .. start[t+1]-1 index the
-    rows of ents that tile t owns, sorted by component, ents[e] = (point index, (region row << 10) |
-    (region column << 2) | comp)."""
+    padding, sim | TILE_ANCHORED for regions that start at the grid's cell 0; pts: (npts, 3) = (sim, comp,
+    offset into [ny][ld]); dims: (nsims, 3) = (nx, ny, ld). Each point belongs to the tile that stores it.
+    Returns (start, ents): start[t] .. start[t+1]-1 index the rows of ents that tile t owns, sorted by
+    component, ents[e] = (point index, (region row << 10) | (region column << 2) | comp)."""
     tiles = np.asarray(tiles, np.int64).reshape(-1, 3)
     pts = np.asarray(pts, np.int64).reshape(-1, 3)
     ix, iy = 64 - 2 * K, rh - 2 * K
@@ -628,10 +635,20 @@ def kstep_owner_tables(tiles, pts, dims, K, rh):
     j, i = np.divmod(pts[:, 2], lds)
     if np.any(i >= nxs) or np.any(j >= nys):
         raise ValueError("a monitor point lies outside its grid")
-    tx, ty = i // ix, j // iy
-    index = {(int(a), int(b), int(c)): q for q, (a, b, c) in enumerate(tiles) if a >= 0}
+    real = tiles[:, 0] >= 0
+    of = np.where(real, tiles[:, 0] & ~N.TILE_ANCHORED, -1)
+    anchored = np.zeros(len(dims), bool)
+    anchored[of[real & (tiles[:, 0] & N.TILE_ANCHORED != 0)]] = True
+    # anchored regions: cells below K belong to region 0, those of the last region's far edge to it
+    anc = anchored[sim]
+    gx = np.maximum(1, -(-(nxs - 2 * K) // ix))
+    gy = np.maximum(1, -(-(nys - 2 * K) // iy))
+    tx = np.where(anc, np.clip((i - K) // ix, 0, gx - 1), i // ix)
+    ty = np.where(anc, np.clip((j - K) // iy, 0, gy - 1), j // iy)
+    index = {(int(a), int(b), int(c)): q for q, (a, (_, b, c)) in enumerate(zip(of, tiles)) if a >= 0}
     t = np.array([index.get((int(a), int(b), int(c)), -1) for a, b, c in zip(sim, tx, ty)], np.int64)
-    code = ((j - (ty * iy - K)) << 10) | ((i - (tx * ix - K)) << 2) | comp
+    low = np.where(anc, 0, K)
+    code = ((j - (ty * iy - low)) << 10) | ((i - (tx * ix - low)) << 2) | comp
     own = np.nonzero(t >= 0)[0]
     order = own[np.lexsort((comp[own], t[own]))]
     ents = np.stack([order, code[order]], axis=1).astype(np.int32)
@@ -790,7 +807,7 @@ class Fused2D:
         self._pts_host = pts if plans else None
         self.kstep, self.krows, self.kwaves = 0, 8, 8
         self.tilesk = self.ent_start = self.ents = self.stagek = None
-        self.coefs = None
+        self.coefs = self.gcs = None
         self._coef_done = False
         if kstep is None and self.kstep_applies():
             kstep, r, w = self.auto_kstep()
@@ -908,21 +925,20 @@ class Fused2D:
         self.ntiles2 = len(tiles)
 
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
-    # (K, rows, waves) candidates of tune_kstep; the automatic shapes were the fastest measured on 64 members
-    # of 256..1024 cells a side (30 M cells: 0.051 ms/step for (8, 8, 8)) and on one 800 x 400 grid with a
-    # 16-wavelength DFT line (1.43 us/step for (12, 4, 16), against 1.51 for (8, 4, 8) and 1.80 for (8, 8, 8));
-    # 64 x 128 regions, (8, 8, 16), fewer recomputed halo cells but one workgroup per CU: 0.057 ms/step on the
-    # 64 members against 0.043 for (8, 8, 8)
-    KCANDIDATES = ((8, 8, 8), (6, 8, 8), (8, 8, 4), (8, 4, 8), (12, 4, 16))
+    # (K, rows, waves) candidates of tune_kstep. Forward sweeps: 64 grids of 256 x 256 cells 4.95 / 5.05 us/step
+    # for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 4.49 / 4.45; 16 grids of 600 x 600 cells
+    # 5.81 / 5.79 against 6.47 for (12, 4, 16); one 800 x 400 grid 1.16 for (16, 4, 16), 1.42 for (8, 4, 8), 1.33
+    # for (12, 4, 16); one 256 x 256 grid 1.07 for (12, 4, 8), 1.11 for (16, 4, 16), 1.28 for (16, 8, 8)
+    KCANDIDATES = ((8, 8, 8), (12, 8, 8), (8, 4, 8), (12, 4, 8), (16, 4, 16))
 
     def kstep_applies(self):
         return all(g.power is None for g in self.grids)
 
     def auto_kstep(self):
         """(K, rows, waves): 64 x 64 regions of 8 waves x 8 rows from PAIR_MIN_CELLS cells on; below, 64 x 64
-        regions of 16 waves x 4 rows and 12 steps per pass, which halve each wave's rows and the launches."""
+        regions of 16 waves x 4 rows and 16 steps per pass, which halve each wave's rows and the launches."""
         big = sum(g.nx * g.ny for g in self.grids) >= self.PAIR_MIN_CELLS
-        return (8, 8, 8) if big else (12, 4, 16)
+        return (8, 8, 8) if big else (16, 4, 16)
 
     def tune_kstep(self, n0=0, steps=16, candidates=None):
         """Time every (K, rows, waves) of `candidates` (default KCANDIDATES) on about `steps` steps from step
@@ -932,10 +948,14 @@ class Fused2D:
         if not self.kstep:
             raise ValueError("tune_kstep needs an engine that runs K steps per pass")
         timings = {}
+        avail = min(self.signal_lens.values(), default=n0 + (1 << 30)) - n0     # steps the sources have samples for
+        kept = (self.kstep, self.krows, self.kwaves)
         for shape in candidates or self.KCANDIDATES:
             K, rows, waves = shape
+            n = min(max(1, steps // K), avail // K - 1) * K                   # after K steps of warm-up
+            if n <= 0:
+                continue
             self.set_kstep(K, rows, waves)
-            n = max(1, steps // K) * K
             self.run(n0, K)                                   # warm-up
             e0, e1 = T.cuda.Event(enable_timing=True), T.cuda.Event(enable_timing=True)
             e0.record()
@@ -943,15 +963,15 @@ class Fused2D:
             e1.record()
             T.cuda.synchronize(self.dev)
             timings[shape] = e0.elapsed_time(e1) / n
-        best = min(timings, key=timings.get)
+        best = min(timings, key=timings.get) if timings else kept
         self.set_kstep(*best)
         return best, timings
 
     def set_kstep(self, K, rows=8, waves=8):
         """Tile list, monitor-owner tables and sample staging of the K-steps-per-pass kernel (K 0: off).
 
-        A tile's region is 64 columns x rows*waves rows; its inner (64-2K) x (rows*waves-2K) cells tile the
-        grid, and each monitor point is sampled by the tile whose inner cells hold it."""
+        A tile's region is 64 columns x rows*waves rows, at multiples of (64-2K) x (rows*waves-2K) cells from the
+        grid's cell 0 (anchored tiles); each monitor point is sampled by the tile that stores it."""
         T = self.torch
         K = int(K or 0)
         if not K:
@@ -962,14 +982,13 @@ class Fused2D:
             raise ValueError(f"K steps per pass need (rows, waves) in {self.KSHAPES} and 2K < min(64, rows*waves)")
         if any(g.power is not None for g in self.grids):
             raise ValueError("K steps per pass do not accumulate grid power")
-        ix, iy = 64 - 2 * K, rows * waves - 2 * K
         parts = []
         for s, g in enumerate(self.grids):
             if not self.is_active(s):
                 continue
-            gx, gy = -(-g.nx // ix), -(-g.ny // iy)
+            gx, gy = anchored_regions(g.nx, 64, K), anchored_regions(g.ny, rows * waves, K)
             t = np.stack(np.meshgrid(np.arange(gx), np.arange(gy), indexing="xy"), -1).reshape(-1, 2)
-            parts.append(np.concatenate([np.full((len(t), 1), s), t], axis=1))
+            parts.append(np.concatenate([np.full((len(t), 1), s | N.TILE_ANCHORED), t], axis=1))
         tiles = np.concatenate(parts).astype(np.int32)
         if self.xcd:
             tiles = xcd_order(tiles, per_wg=1)
@@ -981,8 +1000,12 @@ class Fused2D:
             # with 32-bit byte offsets; a grid too large for that keeps coef NULL and the kernels divide.
             self.coefs = [T.empty((g.ny, g.ld, 4), dtype=T.float32, device=self.dev)
                           if 16 * g.ny * g.ld < 2 ** 32 else None for g in self.grids]
-            for d, c in zip(self.descs, self.coefs):
+            # and the one coefficient that cells without conductivity need
+            self.gcs = [None if c is None else T.empty(c.shape[:2], dtype=T.float32, device=self.dev)
+                        for c in self.coefs]
+            for d, c, h in zip(self.descs, self.coefs, self.gcs):
                 d.coef = c.data_ptr() if c is not None else None
+                d.gc = h.data_ptr() if h is not None else None
             self.shift = None
             self._desc_cache = {}
         self.tilesk = T.from_numpy(tiles.ravel()).to(self.dev)

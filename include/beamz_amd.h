@@ -203,7 +203,17 @@ typedef struct bz_sim2d {
                                            * belongs to: several sources on disjoint cells in one box, whose
                                            * amplitude at step n is signal[src_sel[cell] * src_sig_len + n] */
     int src_sig_len;                      /* samples per source in signal when src_sel is set */
+    float* gc;                            /* NULL, or [ny][ld] FP32, with coef: cb of the cells without conductivity
+                                           * (fa = ca = 1, cb > 0), -1 elsewhere, as bz_yee2d_coef writes it;
+                                           * bz_yee2d_runk then reads one coefficient per such cell, not four */
 } bz_sim2d;
+
+/* Flag of a tile's sim entry in the lists of bz_yee2d_runk and bz_adj2d_runk (sim | BZ_TILE_ANCHORED): the
+ * regions of that simulation start at its cell 0, x-tile tx at column tx * (64 - 2 ksteps) and y-tile ty at row
+ * ty * (waves * rows - 2 ksteps), and every region stores up to a grid edge it reaches. A list of anchored tiles
+ * holds max(1, ceil((n - 2 ksteps) / (size - 2 ksteps))) regions along an axis of n cells. Without the flag, region
+ * origins lie ksteps cells lower and only the inner cells are stored. */
+#define BZ_TILE_ANCHORED 0x40000000
 
 int bz_yee2d_run(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int seg, int* step, int nsteps,
                  const int* pts, int npts, const int* slot, const int* grp, int nslot, int nrow, float* series,
@@ -294,6 +304,7 @@ typedef struct bz_adj2d {
     float* inj_tab;                       /* NULL, or [num_steps][inj_sy][inj_sx]: the objective's injection
                                            * value of each cell at step n >= 1, as bz_adj2d_injtab computes it;
                                            * bz_adj2d_runk then reads it instead of summing inj_w * phasor */
+    const float* gc;                      /* NULL, or bz_sim2d.gc of the same materials (read with coef) */
 } bz_adj2d;
 
 /* Reverse steps n = n_hi-1 down to n_hi-nsteps of every adjoint described in `adjs` (device
