@@ -30,6 +30,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <string>
 #include <type_traits>
 
 // No multiply-add contraction: the one-step and two-step kernels then round identically, so a run gives
@@ -114,6 +115,20 @@ __device__ __forceinline__ float upd_hy(float fa, float gb, float r, float hy, f
 __device__ __forceinline__ float upd_ez(float ca, float gc, float r, float ez, float hx, float hxl, float hy,
                                         float hu) {
     return fmaf(gc, fmaf(r, hy - hu, -(hx - hxl)), ca * ez);
+}
+
+// The (Hz, Ex, Ey) updates, likewise one arithmetic for its two kernels:
+//   Hz' = fa Hz - gb (r (Ey[i+1] - Ey) - (Ex[j+1] - Ex)),  Ex' = ca Ex + gc (Hz - Hz[j-1]),
+//   Ey' = ca Ey - gc r (Hz - Hz[i-1])
+__device__ __forceinline__ float upd_hz(float fa, float gb, float r, float hz, float eyR, float ey, float exN,
+                                        float ex) {
+    return fmaf(-gb, fmaf(r, eyR - ey, -(exN - ex)), fa * hz);
+}
+__device__ __forceinline__ float upd_ex(float ca, float gc, float ex, float hz, float hzU) {
+    return fmaf(gc, hz - hzU, ca * ex);
+}
+__device__ __forceinline__ float upd_ey(float ca, float gc, float r, float ey, float hz, float hzL) {
+    return fmaf(-gc, r * (hz - hzL), ca * ey);
 }
 
 // Monitor sample p of step n, read from the buffer step n wrote.
@@ -288,6 +303,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
     c.ke = S.ke;
     c.kbe = S.kbe;
     const float rdx = S.rdx, rdy = S.rdy;
+    const float rxy = rdx / rdy;   // 1 on square cells
     const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
     // register row r = row j0-1+r, clamped into the grid
     uint32_t ro[SEG + 2];
@@ -316,7 +332,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
         float fa, fb;
         h_coef(sg[r], c, fa, fb);
         const float eyR = __shfl_down(ey[r], 1, LANES);
-        hzn[r] = (hzx && j < ny - 1) ? fa * hz[r] - fb * ((eyR - ey[r]) * rdx - (ex[r + 1] - ex[r]) * rdy) : hz[r];
+        hzn[r] = (hzx && j < ny - 1) ? upd_hz(fa, fb * rdy, rxy, hz[r], eyR, ey[r], ex[r + 1], ex[r]) : hz[r];
         hzl[r] = __shfl_up(hzn[r], 1, LANES);
     }
     // Ex, Ey of rows j0 .. j0+SEG-1, the source on Hz, stores
@@ -331,9 +347,9 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
         if (out && j < ny) {
             float ca, cb;
             e_coef(sg[r], ee[r], c, ca, cb);
-            const float exn = (j >= 1 && j <= ny - 2 && hzx) ? ca * ex[r] + cb * ((hzn[r] - hzn[r - 1]) * rdy) : ex[r];
-            const float eyn = (j <= ny - 2 && i >= 1 && i <= nx - 2) ? ca * ey[r] + cb * (-((hzn[r] - hzl[r]) * rdx))
-                                                                     : ey[r];
+            const float gc = cb * rdy;
+            const float exn = (j >= 1 && j <= ny - 2 && hzx) ? upd_ex(ca, gc, ex[r], hzn[r], hzn[r - 1]) : ex[r];
+            const float eyn = (j <= ny - 2 && i >= 1 && i <= nx - 2) ? upd_ey(ca, gc, rxy, ey[r], hzn[r], hzl[r]) : ey[r];
             float hzo = hzn[r];
             const int a = i - S.src_x0, b = j - S.src_y0;
             if (a >= 0 && a < S.src_sx && b >= 0 && b < S.src_sy) {
@@ -693,17 +709,22 @@ constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further 
 // coefficients, two barriers per step, unanchored regions and 128 registers before: 64 grids of 256 x 256 cells
 // 7.3 -> 4.95 us/step, 16 grids of 600 x 600 cells 8.6 -> 5.8, twelve of 256..1024 a side 6.3 -> 4.5, one grid of
 // 800 x 400 cells with a 16-frequency line 1.33 (K = 12) -> 1.09 (K = 16).
-template <int B, int KW, bool SEL>
-__global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
+// HZ: the (Hz, Ex, Ey) polarisation in the slots of (Ez, Hx, Hy). Its H update reads Ex of the next row and Ey of
+// the next column, its E update Hz of the previous row and column: the bands exchange Ex of the first row and Ex,
+// Ey of the last, and each keeps the Hz of the row above (with its source, which this family adds to Hz).
+template <int B, int KW, bool SEL, bool HZ>
+__global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                                                         const int* __restrict__ tiles, int ntiles, int K,
                                                         const int* __restrict__ step, int q, int rd,
                                                         const int* __restrict__ ent_start,
                                                         const int* __restrict__ ents, float* __restrict__ stage_all,
                                                         Gather2D G) {
     constexpr int RH = KW * B;
-    __shared__ float xe[2][2][KW][LANES];   // [step parity][first, last row of a band]: its Ez
+    __shared__ float xe[2][HZ ? 3 : 2][KW][LANES];   // [step parity][first, last row of a band]: its Ez (HZ: Ex;
+                                                     // and its last row's Ey)
     __shared__ float amps[32];              // the signal's K <= 31 samples of this launch
-    __shared__ float wsrc[KW][B][LANES];    // source weights of the cells of the waves that meet the box
+    __shared__ float wsrc[KW][B + HZ][LANES];   // source weights of the cells of the waves that meet the box (HZ:
+                                                // row B is the row above the band)
     __shared__ SnapBox snq;
     extern __shared__ float smp_all[];      // with monitor points: samples [KW][B][LANES], entries [KW][ELIST][2]
     const int npts = G.npts;
@@ -745,9 +766,9 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
     if (!bottom) klive = min(klive, RH - 1 - w * B);
     if (jb >= ny || jb + B <= 0) klive = 0;
     // uniform over the wave: do the source box, and the snapshot box, meet its rows and this region's columns
-    const bool src_band = S.src_sx > 0 && jb < S.src_y0 + S.src_sy && jb + B > S.src_y0 &&
+    const bool src_band = S.src_sx > 0 && jb - HZ < S.src_y0 + S.src_sy && jb + B > S.src_y0 &&
                           rx0 < S.src_x0 + S.src_sx && rx0 + LANES > S.src_x0;
-    const bool snap_band = S.snap && jb < S.snap_y0 + S.snap_sy && jb + B > S.snap_y0 &&
+    const bool snap_band = !HZ && S.snap && jb < S.snap_y0 + S.snap_sy && jb + B > S.snap_y0 &&
                            rx0 + cx0 < S.snap_x0 + S.snap_sx && rx0 + cx1 > S.snap_x0;
     // edge rules: 0 every row and column of the wave is interior to the grid (the usual case), 1 some column is
     // not, 2 the general form: some row is not, the cells are not square (only this form has the r products), or
@@ -787,7 +808,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
         });
     if (src_band || nmine > 0) edge = 2;    // the general form of the step samples and adds the source
 
-    // the fields, Hy of the row above the band (hyg), and gc = cb * rdy of cells without conductivity
+    // the fields, Hy (HZ: Hz) of the row above the band (hyg), and gc = cb * rdy of cells without conductivity
     float ez[B], hx[B], hy[B], gc[B], hyg = 0.0f;
     const float gb0 = S.kbh * rdy;                  // gb = fb * rdy of such a cell
     bool lossy = true;
@@ -813,7 +834,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
             hx[r] = at(ghx, off(jb + r));
             hy[r] = at(ghy, off(jb + r));
         }
-        hyg = at(ghy, off(jb - 1));
+        hyg = at(HZ ? gez : ghy, off(jb - 1));
         if (one) {
 #pragma unroll
             for (int r = 0; r < B; ++r) {
@@ -878,18 +899,21 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
         };
         if (E == 2 && src_band) {
 #pragma unroll
-            for (int r = 0; r < B; ++r) {
-                const long o = src_cell(r);
+            for (int r = 0; r < B + HZ; ++r) {
+                const long o = src_cell(r < B ? r : -1);
                 wsrc[w][r][l] = o >= 0 ? gload(S.src_add, o) : 0.0f;
             }
         }
         for (int k = 0; k < K; ++k) {
-            float(*x)[KW][LANES] = xe[k & 1];
-            x[0][w][l] = ez[0];
-            x[1][w][l] = ez[B - 1];
+            auto x = xe[k & 1];
+            x[0][w][l] = HZ ? hx[0] : ez[0];
+            x[1][w][l] = HZ ? hx[B - 1] : ez[B - 1];
+            if (HZ) x[2][w][l] = hy[B - 1];
             __syncthreads();
             if (k < klive) {
                 const float ezb = x[0][wd][l], ezg = x[1][wu][l];
+                float eyg = 0.0f;
+                if (HZ) eyg = x[2][wu][l];
                 // what the source adds at the end of this step: with few rows per wave (the small grids' shapes, where
                 // a step's latency counts) read and multiplied here, off the step's chain
                 float add[B], amp = 0.0f;
@@ -906,20 +930,38 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
                 };
                 if (E == 2 && src_band) amp = amps[k];
                 if (plain_src && B <= 4) src_adds(0);
-                // H: the row above the band (its Hy only), then the band
-                hyg = L ? upd_hy(fag, gbg, E == 2 ? rxy : 1.0f, hyg, ez[0], ezg) : fmaf(gb0, ez[0] - ezg, hyg);
+                // H: the row above the band (its Hy, or Hz, only), then the band
+                if (HZ) {
+                    const float r1 = E == 2 ? rxy : 1.0f;
+                    const float hg = computed(L ? upd_hz(fag, gbg, r1, hyg, from_right(eyg), eyg, hx[0], ezg)
+                                                : fmaf(-gb0, (from_right(eyg) - eyg) - (hx[0] - ezg), hyg));
+                    hyg = E == 0 || (hxok && (E < 2 || (jb >= 1 && jb <= ny - 1))) ? hg : hyg;
 #pragma unroll
-                for (int r = 0; r < B; ++r) {
-                    const float ezR = from_right(ez[r]);
-                    const float ed = r < B - 1 ? ez[r + 1] : ezb;
-                    if (!L) {
-                        hx[r] = fmaf(-gb0, ezR - ez[r], hx[r]);
-                        hy[r] = fmaf(gb0, ed - ez[r], hy[r]);
-                    } else {
-                        const float hn = computed(upd_hx(fa[r], gb[r], hx[r], ezR, ez[r]));
-                        hx[r] = E == 0 || hxok ? hn : hx[r];
-                        if (E < 2 || jb + r < ny - 1)
-                            hy[r] = upd_hy(fa[r], gb[r], E == 2 ? rxy : 1.0f, hy[r], ed, ez[r]);
+                    for (int r = 0; r < B; ++r) {
+                        const float eyR = from_right(hy[r]);
+                        const float exN = r < B - 1 ? hx[r + 1] : ezb;
+                        if (!L) {
+                            ez[r] = fmaf(-gb0, (eyR - hy[r]) - (exN - hx[r]), ez[r]);
+                        } else {
+                            const float hn = computed(upd_hz(fa[r], gb[r], r1, ez[r], eyR, hy[r], exN, hx[r]));
+                            ez[r] = E == 0 || (hxok && (E < 2 || jb + r < ny - 1)) ? hn : ez[r];
+                        }
+                    }
+                } else {
+                    hyg = L ? upd_hy(fag, gbg, E == 2 ? rxy : 1.0f, hyg, ez[0], ezg) : fmaf(gb0, ez[0] - ezg, hyg);
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        const float ezR = from_right(ez[r]);
+                        const float ed = r < B - 1 ? ez[r + 1] : ezb;
+                        if (!L) {
+                            hx[r] = fmaf(-gb0, ezR - ez[r], hx[r]);
+                            hy[r] = fmaf(gb0, ed - ez[r], hy[r]);
+                        } else {
+                            const float hn = computed(upd_hx(fa[r], gb[r], hx[r], ezR, ez[r]));
+                            hx[r] = E == 0 || hxok ? hn : hx[r];
+                            if (E < 2 || jb + r < ny - 1)
+                                hy[r] = upd_hy(fa[r], gb[r], E == 2 ? rxy : 1.0f, hy[r], ed, ez[r]);
+                        }
                     }
                 }
                 // snapshot of call-relative step q*K+k at the stored cells: the Ez this step reads, the Hx, Hy it
@@ -945,16 +987,34 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
                         }
                 }
                 // E
+                if (HZ) {
+                    const float r1 = E == 2 ? rxy : 1.0f;
 #pragma unroll
-                for (int r = 0; r < B; ++r) {
-                    const float hxl = from_left(hx[r]);
-                    const float hu = r > 0 ? hy[r - 1] : hyg;
-                    if (!L) {
-                        ez[r] = fmaf(gc[r], (hy[r] - hu) - (hx[r] - hxl), ez[r]);
-                    } else if (E < 2 || (jb + r >= 1 && jb + r <= ny - 2)) {
-                        const float en =
-                            computed(upd_ez(ca[r], gcl[r], E == 2 ? rxy : 1.0f, ez[r], hx[r], hxl, hy[r], hu));
-                        ez[r] = E == 0 || xin ? en : ez[r];
+                    for (int r = 0; r < B; ++r) {
+                        const float hzL = from_left(ez[r]);
+                        const float hzU = r > 0 ? ez[r - 1] : hyg;
+                        if (!L) {
+                            hx[r] = fmaf(gc[r], ez[r] - hzU, hx[r]);
+                            hy[r] = fmaf(-gc[r], ez[r] - hzL, hy[r]);
+                        } else {
+                            const float xn = computed(upd_ex(ca[r], gcl[r], hx[r], ez[r], hzU));
+                            const float yn = computed(upd_ey(ca[r], gcl[r], r1, hy[r], ez[r], hzL));
+                            hx[r] = E == 0 || (hxok && (E < 2 || (jb + r >= 1 && jb + r <= ny - 2))) ? xn : hx[r];
+                            hy[r] = E == 0 || (xin && (E < 2 || jb + r <= ny - 2)) ? yn : hy[r];
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        const float hxl = from_left(hx[r]);
+                        const float hu = r > 0 ? hy[r - 1] : hyg;
+                        if (!L) {
+                            ez[r] = fmaf(gc[r], (hy[r] - hu) - (hx[r] - hxl), ez[r]);
+                        } else if (E < 2 || (jb + r >= 1 && jb + r <= ny - 2)) {
+                            const float en =
+                                computed(upd_ez(ca[r], gcl[r], E == 2 ? rxy : 1.0f, ez[r], hx[r], hxl, hy[r], hu));
+                            ez[r] = E == 0 || xin ? en : ez[r];
+                        }
                     }
                 }
                 // the source box, after E (it touches only the Ez of its own cells)
@@ -964,13 +1024,18 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
                         if (B > 4 && r % 4 == 0) src_adds(r);
                         ez[r] += add[r];
                     }
+                    if (HZ) {
+                        const float v = wsrc[w][B][l], a = computed(v * amp);
+                        hyg += v != 0.0f ? a : 0.0f;
+                    }
                 } else if (E == 2 && src_band) {
 #pragma unroll
-                    for (int r = 0; r < B; ++r) {
-                        const long o = src_cell(r);
+                    for (int r = 0; r < B + HZ; ++r) {
+                        const long o = src_cell(r < B ? r : -1);
+                        float& f = r < B ? ez[r < B ? r : 0] : hyg;
                         if (o >= 0)
-                            ez[r] = (S.src_mul ? gload(S.src_mul, o) : 1.0f) * ez[r] +
-                                    wsrc[w][r][l] * (SEL ? box_amp(S, o, n0 + k, amp) : amp);
+                            f = (S.src_mul ? gload(S.src_mul, o) : 1.0f) * f +
+                                wsrc[w][r][l] * (SEL ? box_amp(S, o, n0 + k, amp) : amp);
                     }
                 }
             }
@@ -1038,7 +1103,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? 6 : 1)) void k_ye
     }
 }
 
-template <int B, int KW>
+template <int B, int KW, bool HZ>
 int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int K, int* step, int rd0, int nlaunch,
          const int* ent_start, const int* ents, float* stage, const Gather2D& G, bool sel, hipStream_t st) {
     const dim3 b(LANES, KW);
@@ -1050,10 +1115,10 @@ int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int K, int* step, i
     for (int q = 0; q < nlaunch; ++q) {
         const dim3 g(ntiles + (q > 0 && G.npts > 0 ? gather_blocks : 0));
         if (sel)
-            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, true>), g, b, lds, st, sims, tiles, ntiles, K, step, q, (rd0 + q) & 1,
+            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, true, HZ>), g, b, lds, st, sims, tiles, ntiles, K, step, q, (rd0 + q) & 1,
                                ent_start, ents, stage, G);
         else
-            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, false>), g, b, lds, st, sims, tiles, ntiles, K, step, q,
+            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, false, HZ>), g, b, lds, st, sims, tiles, ntiles, K, step, q,
                                (rd0 + q) & 1, ent_start, ents, stage, G);
         BZ_CHECK_LAUNCH("bz_yee2d_runk(steps)");
     }
@@ -1173,24 +1238,24 @@ extern "C" int bz_yee2d_run2(const bz_sim2d* sims, int nsims, const int* tiles, 
     return BZ_OK;
 }
 
-extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
-                             int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
-                             float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
-                             float* series, int nfreq, const double* phasor, double* dft, int src_sel,
-                             void* stream) {
+template <bool HZ>
+static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows,
+                     int waves, int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
+                     float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow, float* series,
+                     int nfreq, const double* phasor, double* dft, int src_sel, void* stream) {
     BZ_REQUIRE(sims && nsims > 0 && tiles && ntiles > 0 && step && nlaunch >= 0 && (rd0 == 0 || rd0 == 1),
-               "bz_yee2d_runk: bad arguments");
+               name + ": bad arguments");
     const int shape = rows * 100 + waves;
     BZ_REQUIRE(shape == 804 || shape == 808 || shape == 816 || shape == 408 || shape == 416 || shape == 1604,
-               "bz_yee2d_runk: (rows, waves) must be (8, 4), (8, 8), (8, 16), (4, 8), (4, 16) or (16, 4)");
+               name + ": (rows, waves) must be (8, 4), (8, 8), (8, 16), (4, 8), (4, 16) or (16, 4)");
     BZ_REQUIRE(ksteps >= 1 && 2 * ksteps < LANES && 2 * ksteps < waves * rows,
-               "bz_yee2d_runk: ksteps must leave inner cells (2 * ksteps < 64 and < rows * waves)");
+               name + ": ksteps must leave inner cells (2 * ksteps < 64 and < rows * waves)");
     BZ_REQUIRE(npts >= 0 && (npts == 0 || (ent_start && ents && stage && slot)),
-               "bz_yee2d_runk: monitor points without tables");
-    BZ_REQUIRE(nfreq >= 0 && (nfreq == 0 || (phasor && dft)), "bz_yee2d_runk: DFT requested without buffers");
-    BZ_REQUIRE(!grp || (nslot > 0 && nrow > 0), "bz_yee2d_runk: point groups need nslot > 0 and nrow > 0");
+               name + ": monitor points without tables");
+    BZ_REQUIRE(nfreq >= 0 && (nfreq == 0 || (phasor && dft)), name + ": DFT requested without buffers");
+    BZ_REQUIRE(!grp || (nslot > 0 && nrow > 0), name + ": point groups need nslot > 0 and nrow > 0");
     BZ_REQUIRE((long)npts * (nfreq > 0 ? nfreq : 1) / 256 < (1L << 31) - 1,
-               "bz_yee2d_runk: too many monitor points x frequencies");
+               name + ": too many monitor points x frequencies");
     if (nlaunch == 0) return BZ_OK;
     Gather2D G;
     G.pts = nullptr;
@@ -1206,7 +1271,7 @@ extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, 
     const hipStream_t st = (hipStream_t)stream;
     if (npts == 0) ent_start = ents = nullptr;
 #define BZ_RUNK(R, W) \
-    runk<R, W>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, ent_start, ents, stage, G, src_sel != 0, st)
+    runk<R, W, HZ>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, ent_start, ents, stage, G, src_sel != 0, st)
     switch (shape) {
         case 804: return BZ_RUNK(8, 4);
         case 808: return BZ_RUNK(8, 8);
@@ -1216,6 +1281,24 @@ extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, 
         default: return BZ_RUNK(16, 4);
     }
 #undef BZ_RUNK
+}
+
+extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
+                             int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
+                             float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
+                             float* series, int nfreq, const double* phasor, double* dft, int src_sel,
+                             void* stream) {
+    return runk_call<false>("bz_yee2d_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, ent_start, ents,
+                            stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel, stream);
+}
+
+extern "C" int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
+                             int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
+                             float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
+                             float* series, int nfreq, const double* phasor, double* dft, int src_sel,
+                             void* stream) {
+    return runk_call<true>("bz_yee2d_hz_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, ent_start, ents,
+                            stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel, stream);
 }
 
 extern "C" int bz_yee2d_coef(const bz_sim2d* sims, int nsims, int max_cells, void* stream) {

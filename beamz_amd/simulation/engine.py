@@ -139,14 +139,15 @@ class Grid:
                 return (f"bz_yee3d_step2 (two steps per pass, {self.waves2} waves x {self.rows2} rows, "
                         f"{self.kseg2_eff()}-plane segments)")
             return f"bz_yee3d_step (fused z-march, {self.rows} rows/wave)" if self.kernel == "fused" else "bz_update_3d (two-pass)"
-        if self.pol == "Hz":
+        hz = "hz_" if self.pol == "Hz" else ""
+        f = self._f2d
+        if f and f.kstep and (hz or self.kernel == "fused"):
+            k, r = f.kstep, f.krows * f.kwaves
+            return f"bz_yee2d_{hz}runk ({k} steps per pass, 64x{r} regions, {64 - 2 * k}x{r - 2 * k} inner)"
+        if hz:
             return "bz_yee2d_hz_run ((Hz, Ex, Ey), fused, batched)"
         if self.kernel != "fused":
             return "bz_update_h_2d + bz_update_e_2d"
-        f = self._f2d
-        if f and f.kstep:
-            k, r = f.kstep, f.krows * f.kwaves
-            return f"bz_yee2d_runk ({k} steps per pass, 64x{r} regions, {64 - 2 * k}x{r - 2 * k} inner)"
         return "bz_yee2d_run (fused, batched)"
 
     def start_timing(self):
@@ -790,10 +791,10 @@ class Fused2D:
         self.use_graph = bool(graph)
         self.graphs = {}
         if self.pol == "Hz":
-            # the (Hz, Ex, Ey) family has the one-step kernel only
+            # the (Hz, Ex, Ey) family has the one-step and the K-step kernels
             if any(sn is not None for sn in self.snapshots):
                 raise ValueError("snapshot boxes need the (Ez, Hx, Hy) polarisation")
-            pairs, kstep = False, 0
+            pairs = False
         if pairs is None:
             # small batches are launch-latency bound, and a pair's serial row march is slower there
             # (800 x 400: 13.4 us/step in pairs against 10.2 with one step per launch)
@@ -1152,7 +1153,7 @@ class Fused2D:
 
     def _launch_k(self, nl, rd0):
         ptr = lambda t: t.data_ptr() if t is not None else None
-        N.call("bz_yee2d_runk", self.desc_dev.data_ptr(), len(self.grids), self.tilesk.data_ptr(), self.ntilesk,
+        N.call("bz_yee2d_hz_runk" if self.pol == "Hz" else "bz_yee2d_runk", self.desc_dev.data_ptr(), len(self.grids), self.tilesk.data_ptr(), self.ntilesk,
                self.krows, self.kwaves, self.kstep, self.step.data_ptr(), rd0, nl, ptr(self.ent_start),
                ptr(self.ents), ptr(self.stagek), self.npts, ptr(self.slot), ptr(self.grp), self.nslot, self.nrow,
                ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft), int(self.multi_src),
