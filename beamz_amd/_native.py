@@ -58,6 +58,12 @@ class Adj2D(C.Structure):
 
 TILE_ANCHORED = 0x40000000     # BZ_TILE_ANCHORED
 
+
+class GatherTable(C.Structure):
+    _fields_ = [("comp", vp), ("stage_off", vp), ("off", vp), ("n", i32), ("row", vp), ("series", vp), ("nfreq", i32),
+                ("phasor", vp), ("dft", vp)]
+
+
 # name -> argtypes (restype is int unless listed in _RESTYPE)
 SIGNATURES = {
     "bz_last_error": [],
@@ -70,6 +76,8 @@ SIGNATURES = {
                       i32, i32, vp],
     "bz_yee3d_step2": [P6, P6, vp, vp, i32, i32, i32, i32, f64, f64, f64, f64, f64, f64, C.POINTER(BoxSource),
                        C.POINTER(f32), i32, vp, C.POINTER(i32), i32, i32, i32, vp],
+    "bz_yee3d_run2": [P6, P6, vp, vp, i32, i32, i32, i32, f64, f64, f64, f64, f64, f64, C.POINTER(BoxSource), vp, i32,
+                      i32, vp, C.POINTER(i32), C.POINTER(GatherTable), i32, i32, i32, i32, vp],
     "bz_yee3d_step3": [P6, P6, vp, vp, i32, i32, i32, i32, f64, f64, f64, f64, f64, f64, C.POINTER(BoxSource),
                        C.POINTER(f32), C.POINTER(f32), i32, vp, vp, C.POINTER(i32), i32, i32, i32, vp],
     "bz_yee3d_step2_noalloc": [P6, P6, vp, vp, i32, i32, i32, i32, f64, f64, f64, f64, f64, f64,

@@ -25,8 +25,16 @@
 // (clamped in-grid reads) only feed values that are not stored.
 // HBM traffic per two cell-updates: 8 reads + 6 writes of FP32 (56 B) plus
 // the halo columns, rows and planes.
+// What bounds it: on a large grid the issue of about 260 vector operations per halo-inclusive cell pair (20% of the
+// rows and 6% of the columns are halo), at two workgroups of 512 per CU (95 VGPRs); on a small one the serial march
+// of a segment of kseg + 3 planes. Sources and staging box sit in LDS, with the planes on which a wave can meet them
+// worked out once: as kernel arguments tested on every plane they cost 130 spilled scalar registers and 120 VGPRs.
+// us per pair before / after: 480x240x160 295 / 286, 300x200x100 112 / 97, 200x120x64 46 / 37, 120x72x40 24 / 20.
+// Tried and slower: 80 VGPRs for three workgroups per CU (20 spills: 609 at 480x240x160, 31 at 120x72x40), loads one
+// plane ahead (378 at 480x240x160), three rows per wave (322), 16 waves (22 at 120x72x40).
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -39,6 +47,7 @@ namespace {
 constexpr int LANES = 64;
 constexpr int OXT = LANES - 4;   // stored columns per wave
 constexpr int NXCD = 8;
+#define BZ_GLOBAL __attribute__((address_space(1)))
 
 struct Fields6 {
     float* p[6];
@@ -46,6 +55,7 @@ struct Fields6 {
 
 struct Boxes2 {
     int n;
+    int x0, y0, z0, x1, y1, z1;    // the cells the boxes cover lie in [x0, x1) x [y0, y1) x [z0, z1)
     bz_box_source b[BZ_MAX_BOX];   // b[q].amp: amplitude of step n
     float amp1[BZ_MAX_BOX];        // amplitude of step n + 1
 };
@@ -53,6 +63,21 @@ struct Boxes2 {
 struct Stage {
     float* p;   // [6][sz][sy][sx] (Ex, Ey, Ez, Hx, Hy, Hz of step n+1), or NULL
     int x0, y0, z0, sx, sy, sz;
+};
+
+// Monitor samples of the previous pair, taken by extra workgroups of a launch (n 0: none): 4 us a pair as a launch
+// of its own at 120x72x40, hidden beside the tiles here.
+struct Gather3D {
+    const float* base0[6];       // the staging slot that holds its first step
+    const int* comp;
+    const int64_t* off0;
+    const int64_t* off1;         // offsets into the field buffer this launch only reads (its second step)
+    int n, act0, act1, nfreq;
+    float* series0;
+    float* series1;
+    const double* phasor0;
+    const double* phasor1;
+    double* dft;
 };
 
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -81,15 +106,15 @@ __device__ __forceinline__ void ecoef(float sig, float eps, const Coef& c, float
 
 __device__ __forceinline__ void add_sources(float& ex, float& ey, float& ez, int i, int j, int k, const Boxes2& src,
                                             bool second) {
-#pragma unroll
-    for (int q = 0; q < BZ_MAX_BOX; ++q) {
-        if (q >= src.n) break;
+#pragma unroll 1
+    for (int q = 0; q < src.n; ++q) {
         const bz_box_source& b = src.b[q];
         const int a = i - b.x0, bb = j - b.y0, cc = k - b.z0;
         if (a >= 0 && a < b.sx && bb >= 0 && bb < b.sy && cc >= 0 && cc < b.sz) {
             const long rr = ((long)cc * b.sy + bb) * b.sx + a;
-            const float m = b.mul ? b.mul[rr] : 1.0f;
-            const float v = b.add[rr] * (second ? src.amp1[q] : b.amp);
+            // (global, not flat, accesses: the pointers come from LDS)
+            const float m = b.mul ? ((const BZ_GLOBAL float*)b.mul)[rr] : 1.0f;
+            const float v = ((const BZ_GLOBAL float*)b.add)[rr] * (second ? src.amp1[q] : b.amp);
             // selects, not a component-indexed write (which would place ex, ey, ez in scratch memory)
             ex = b.comp == 0 ? m * ex + v : ex;
             ey = b.comp == 1 ? m * ey + v : ey;
@@ -111,15 +136,63 @@ struct Carry2 {
     float ca2[R], cb2[R];              // E coefficients at plane k-2
 };
 
+// Terms of the previous pair's two steps for (point, frequency) g, in step order: k_gather2's operations (there
+// the compiler contracts each multiply and add; this file switches contraction off).
+__device__ __forceinline__ void gather_prev(const Gather3D& G, const Fields6& S, long g) {
+    const int p = (int)(g % G.n), k = (int)(g / G.n);
+    if (k >= max(G.nfreq, 1)) return;
+    const int c = G.comp[p];
+    float v0 = 0.0f, v1 = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+        if (q == c) {
+            if (G.act0) v0 = G.base0[q][G.off0[p]];
+            if (G.act1) v1 = S.p[q][G.off1[p]];
+        }
+    if (k == 0) {
+        if (G.act0 && G.series0) G.series0[p] = v0;
+        if (G.act1 && G.series1) G.series1[p] = v1;
+    }
+    if (k >= G.nfreq) return;
+    double* a = G.dft + 2 * ((long)k * G.n + p);
+    double re = a[0], im = a[1];
+    if (G.act0) {
+        const double dv = (double)v0;
+        re = fma(dv, G.phasor0[2 * k], re);
+        im = fma(dv, G.phasor0[2 * k + 1], im);
+    }
+    if (G.act1) {
+        const double dv = (double)v1;
+        re = fma(dv, G.phasor1[2 * k], re);
+        im = fma(dv, G.phasor1[2 * k + 1], im);
+    }
+    a[0] = re;
+    a[1] = im;
+}
+
 template <int R, int W>
 __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, const float* __restrict__ eps,
                                                        const float* __restrict__ sig, int nx, int ny, int nz, int ld,
                                                        int kseg, int gx, int gy, int gz, int per_xcd, Coef c,
-                                                       float rdx, float rdy, float rdz, Boxes2 src, Stage stg) {
+                                                       float rdx, float rdy, float rdz, Boxes2 src_arg,
+                                                       Stage stg_arg, Gather3D G) {
     constexpr int T = W * R;
+    if ((int)blockIdx.x >= per_xcd * NXCD) {
+        gather_prev(G, S, (long)((int)blockIdx.x - per_xcd * NXCD) * (LANES * W) + threadIdx.y * LANES + threadIdx.x);
+        return;
+    }
     __shared__ float xa[W][4][LANES];   // first row of each wave: Ez(n), Ex(n) at k; Ez(n+1), Ex(n+1) at k-1
     __shared__ float xh[W][2][LANES];   // last row: Hz(n+2), Hx(n+2) at k-2
     __shared__ float xb[W][2][LANES];   // last row: Hz(n+1), Hx(n+1) at k
+
+    // the source boxes and the staging box, written before the first barrier and read after it by the few waves
+    // and planes that meet them: as kernel arguments their 80 values sat in spilled scalar registers in every wave
+    __shared__ Boxes2 src;
+    __shared__ Stage stg;
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        src = src_arg;
+        stg = stg_arg;
+    }
 
     const int h = blockIdx.x;
     const int tile = (h % NXCD) * per_xcd + h / NXCD;
@@ -145,6 +218,14 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
     const bool xe = i <= nx - 2;
     const bool lane_out = l >= 2 && l <= LANES - 3 && i >= 0 && i < nx;
     const int wd = min(w + 1, W - 1), wu = max(w - 1, 0);   // neighbour waves (edge waves read their own slot)
+
+    // planes on which this wave's rows and columns can meet a source, or the staging box (empty: never)
+    const int wr = __builtin_amdgcn_readfirstlane(jb), wx = tx * OXT - 2;
+    const bool src_xy = src_arg.n > 0 && wr < src_arg.y1 && wr + R > src_arg.y0 && wx < src_arg.x1 && wx + LANES > src_arg.x0;
+    const int sz0 = src_xy ? src_arg.z0 : 0, sz1 = src_xy ? src_arg.z1 : 0;
+    const bool stg_xy = stg_arg.p && wr < stg_arg.y0 + stg_arg.sy && wr + R > stg_arg.y0 &&
+                        wx < stg_arg.x0 + stg_arg.sx && wx + LANES > stg_arg.x0;
+    const int gz0 = stg_xy ? max(k0, stg_arg.z0) : 0, gz1 = stg_xy ? min(k1, stg_arg.z0 + stg_arg.sz) : 0;
 
     Carry2<R> C;
 #pragma unroll
@@ -248,14 +329,14 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
                                ? ca * C.ey0[r] + cb * ((h1x[r] - C.h1x[r]) * rdz - (h1z[r] - hzL) * rdx)
                                : C.ey0[r];
                 float ezz = (kz && yin && xin) ? ca * ez[r] + cb * ((h1y[r] - hyL) * rdx - (h1x[r] - hxU) * rdy) : ez[r];
-                if (src.n) add_sources(ex, ey, ezz, i, j, k, src, false);
+                if (k >= sz0 && k < sz1) add_sources(ex, ey, ezz, i, j, k, src, false);
                 e1x[r] = ex;
                 e1y[r] = ey;
                 e1z[r] = ezz;
             }
         }
         // ---- monitor samples of step n+1 (owned cells inside the staging box) ----
-        if (stg.p && k >= k0 && k < k1 && lane_out) {
+        if (k >= gz0 && k < gz1 && lane_out) {
             const long plane = (long)stg.sz * stg.sy * stg.sx;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
@@ -263,7 +344,7 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
                 const int a = i - stg.x0, b = j - stg.y0, cc = k - stg.z0;
                 if (j >= J0 + 2 && j < J0 + T - 2 && j < ny && a >= 0 && a < stg.sx && b >= 0 && b < stg.sy &&
                     cc >= 0 && cc < stg.sz) {
-                    float* q = stg.p + ((long)cc * stg.sy + b) * stg.sx + a;
+                    BZ_GLOBAL float* q = (BZ_GLOBAL float*)stg.p + ((long)cc * stg.sy + b) * stg.sx + a;
                     q[0] = e1x[r];
                     q[plane] = e1y[r];
                     q[2 * plane] = e1z[r];
@@ -321,7 +402,7 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
                 float ezz = (kz && yin && xin) ? ca * C.f1z[r] + cb * ((C.h2y[r] - hyL) * rdx - (C.h2x[r] - hxU) * rdy)
                                                : C.f1z[r];
                 if (kst && lane_out && j >= J0 + 2 && j < J0 + T - 2 && j < ny) {
-                    if (src.n) add_sources(ex, ey, ezz, i, j, m2, src, true);
+                    if (m2 >= sz0 && m2 < sz1) add_sources(ex, ey, ezz, i, j, m2, src, true);
                     const uint32_t o = mp + ro[r];
                     put(D.p[0], o, ex);
                     put(D.p[1], o, ey);
@@ -366,17 +447,84 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
 template <int R, int W>
 int launch(const Fields6& S, const Fields6& D, const float* eps, const float* sig, int nx, int ny, int nz, int ld,
            int kseg, const Coef& c, float rdx, float rdy, float rdz, const Boxes2& bs, const Stage& stg,
-           hipStream_t st) {
+           const Gather3D& G, hipStream_t st) {
     constexpr int T = W * R;
     const int gx = (nx + OXT - 1) / OXT;
     const int gy = (ny + (T - 4) - 1) / (T - 4);
     const int gz = (nz + kseg - 1) / kseg;
     const int n = gx * gy * gz;
     const int per_xcd = (n + NXCD - 1) / NXCD;
-    auto kern = k_yee3d_tb2<R, W>;
-    hipLaunchKernelGGL(kern, dim3(per_xcd * NXCD), dim3(LANES, W), 0, st, S, D, eps, sig, nx, ny, nz, ld, kseg, gx,
-                       gy, gz, per_xcd, c, rdx, rdy, rdz, bs, stg);
+    const long gt = (long)G.n * (G.nfreq > 0 ? G.nfreq : 1);
+    const dim3 grid(per_xcd * NXCD + (unsigned)((gt + LANES * W - 1) / (LANES * W)));
+    hipLaunchKernelGGL((k_yee3d_tb2<R, W>), grid, dim3(LANES, W), 0, st, S, D, eps, sig, nx, ny, nz, ld, kseg, gx, gy,
+                       gz, per_xcd, c, rdx, rdy, rdz, bs, stg, G);
     BZ_CHECK_LAUNCH("bz_yee3d_step2");
+    return BZ_OK;
+}
+
+// One pair of checked arguments.
+int launch_pair(const Fields6& S, const Fields6& D, const float* eps, const float* sig, int nx, int ny, int nz, int ld,
+                int kseg, int rows, int waves, const Coef& c, float rx, float ry, float rz, const Boxes2& bs,
+                const Stage& stg, const Gather3D& G, hipStream_t st) {
+    if (waves == 16) return launch<2, 16>(S, D, eps, sig, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, G, st);
+    switch (rows) {
+        case 2: return launch<2, 8>(S, D, eps, sig, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, G, st);
+        case 3: return launch<3, 8>(S, D, eps, sig, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, G, st);
+        default: return launch<4, 8>(S, D, eps, sig, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, G, st);
+    }
+}
+
+// The checks and the launch structs that bz_yee3d_step2 and bz_yee3d_run2 share.
+int check_pair(const std::string& name, float* const src[6], float* const dst[6], const float* eps_r,
+               const float* sigma, int nx, int ny, int nz, int ld, const bz_box_source* boxes, const float* amps,
+               int nbox, const float* stage, const int* stage_box, int& kseg, int rows, int waves, Boxes2& bs,
+               Stage& stg, Fields6& S, Fields6& D) {
+    BZ_REQUIRE(src && dst && eps_r && sigma, name + ": null pointer");
+    for (int q = 0; q < 6; ++q)
+        BZ_REQUIRE(src[q] && dst[q] && src[q] != dst[q], name + ": bad field buffers");
+    BZ_REQUIRE(nx >= 2 && ny >= 2 && nz >= 2 && ld >= nx, name + ": bad shape");
+    BZ_REQUIRE(4.0 * nz * ny * ld < 4294967295.0, name + ": a field array exceeds 4 GiB (32-bit offsets)");
+    BZ_REQUIRE(nbox >= 0 && nbox <= BZ_MAX_BOX && (nbox == 0 || (boxes && amps)), name + ": bad source list");
+    bs = Boxes2{};
+    bs.n = nbox;
+    for (int q = 0; q < nbox; ++q) {
+        const bz_box_source& b = boxes[q];
+        BZ_REQUIRE(b.comp >= 0 && b.comp <= 2 && b.add && b.sx > 0 && b.sy > 0 && b.sz > 0 && b.x0 >= 0 &&
+                       b.y0 >= 0 && b.z0 >= 0 && b.x0 + b.sx <= nx && b.y0 + b.sy <= ny && b.z0 + b.sz <= nz,
+                   name + ": source box outside the grid");
+        bs.b[q] = b;
+        bs.x0 = q ? std::min(bs.x0, b.x0) : b.x0;
+        bs.y0 = q ? std::min(bs.y0, b.y0) : b.y0;
+        bs.z0 = q ? std::min(bs.z0, b.z0) : b.z0;
+        bs.x1 = q ? std::max(bs.x1, b.x0 + b.sx) : b.x0 + b.sx;
+        bs.y1 = q ? std::max(bs.y1, b.y0 + b.sy) : b.y0 + b.sy;
+        bs.z1 = q ? std::max(bs.z1, b.z0 + b.sz) : b.z0 + b.sz;
+    }
+    stg.p = const_cast<float*>(stage);
+    stg.x0 = stg.y0 = stg.z0 = stg.sx = stg.sy = stg.sz = 0;
+    if (stage) {
+        BZ_REQUIRE(stage_box, name + ": staging buffer without its box");
+        stg.x0 = stage_box[0];
+        stg.y0 = stage_box[1];
+        stg.z0 = stage_box[2];
+        stg.sx = stage_box[3];
+        stg.sy = stage_box[4];
+        stg.sz = stage_box[5];
+        BZ_REQUIRE(stg.sx > 0 && stg.sy > 0 && stg.sz > 0 && stg.x0 >= 0 && stg.y0 >= 0 && stg.z0 >= 0 &&
+                       stg.x0 + stg.sx <= nx && stg.y0 + stg.sy <= ny && stg.z0 + stg.sz <= nz,
+                   name + ": staging box outside the grid");
+    }
+    if (kseg <= 0) kseg = 32;
+    BZ_REQUIRE(kseg >= 2, name + ": kseg must be at least 2");
+    BZ_REQUIRE(waves == 8 || (waves == 16 && rows == 2), name + ": waves must be 8 (rows 2, 3, 4) or 16 (rows 2)");
+    if (rows < 2 || rows > 4) {
+        bz::set_error(name + ": rows must be 2, 3 or 4");
+        return BZ_EINVAL;
+    }
+    for (int q = 0; q < 6; ++q) {
+        S.p[q] = src[q];
+        D.p[q] = dst[q];
+    }
     return BZ_OK;
 }
 
@@ -386,55 +534,94 @@ extern "C" int bz_yee3d_step2(float* const src[6], float* const dst[6], const fl
                               int nx, int ny, int nz, int ld, double dx, double dy, double dz, double dt, double mu0,
                               double eps0, const bz_box_source* boxes, const float* amp1, int nbox, float* stage,
                               const int* stage_box, int kseg, int rows, int waves, void* stream) {
-    BZ_REQUIRE(src && dst && eps_r && sigma, "bz_yee3d_step2: null pointer");
-    for (int q = 0; q < 6; ++q)
-        BZ_REQUIRE(src[q] && dst[q] && src[q] != dst[q], "bz_yee3d_step2: bad field buffers");
-    BZ_REQUIRE(nx >= 2 && ny >= 2 && nz >= 2 && ld >= nx, "bz_yee3d_step2: bad shape");
-    BZ_REQUIRE(4.0 * nz * ny * ld < 4294967295.0, "bz_yee3d_step2: a field array exceeds 4 GiB (32-bit offsets)");
-    BZ_REQUIRE(nbox >= 0 && nbox <= BZ_MAX_BOX && (nbox == 0 || (boxes && amp1)), "bz_yee3d_step2: bad source list");
     Boxes2 bs;
-    bs.n = nbox;
-    for (int q = 0; q < nbox; ++q) {
-        const bz_box_source& b = boxes[q];
-        BZ_REQUIRE(b.comp >= 0 && b.comp <= 2 && b.add && b.sx > 0 && b.sy > 0 && b.sz > 0 && b.x0 >= 0 &&
-                       b.y0 >= 0 && b.z0 >= 0 && b.x0 + b.sx <= nx && b.y0 + b.sy <= ny && b.z0 + b.sz <= nz,
-                   "bz_yee3d_step2: source box outside the grid");
-        bs.b[q] = b;
-        bs.amp1[q] = amp1[q];
-    }
     Stage stg;
-    stg.p = stage;
-    stg.x0 = stg.y0 = stg.z0 = stg.sx = stg.sy = stg.sz = 0;
-    if (stage) {
-        BZ_REQUIRE(stage_box, "bz_yee3d_step2: staging buffer without its box");
-        stg.x0 = stage_box[0];
-        stg.y0 = stage_box[1];
-        stg.z0 = stage_box[2];
-        stg.sx = stage_box[3];
-        stg.sy = stage_box[4];
-        stg.sz = stage_box[5];
-        BZ_REQUIRE(stg.sx > 0 && stg.sy > 0 && stg.sz > 0 && stg.x0 >= 0 && stg.y0 >= 0 && stg.z0 >= 0 &&
-                       stg.x0 + stg.sx <= nx && stg.y0 + stg.sy <= ny && stg.z0 + stg.sz <= nz,
-                   "bz_yee3d_step2: staging box outside the grid");
-    }
-    if (kseg <= 0) kseg = 32;
-    BZ_REQUIRE(kseg >= 2, "bz_yee3d_step2: kseg must be at least 2");
     Fields6 S, D;
-    for (int q = 0; q < 6; ++q) {
-        S.p[q] = src[q];
-        D.p[q] = dst[q];
+    const int rc = check_pair("bz_yee3d_step2", src, dst, eps_r, sigma, nx, ny, nz, ld, boxes, amp1, nbox, stage,
+                              stage_box, kseg, rows, waves, bs, stg, S, D);
+    if (rc != BZ_OK) return rc;
+    for (int q = 0; q < nbox; ++q) bs.amp1[q] = amp1[q];
+    return launch_pair(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, rows, waves, make_coef(dt, mu0, eps0),
+                       (float)(1.0 / dx), (float)(1.0 / dy), (float)(1.0 / dz), bs, stg, Gather3D{},
+                       (hipStream_t)stream);
+}
+
+extern "C" int bz_yee3d_run2(float* const src[6], float* const dst[6], const float* eps_r, const float* sigma, int nx,
+                             int ny, int nz, int ld, double dx, double dy, double dz, double dt, double mu0,
+                             double eps0, const bz_box_source* boxes, const float* amps, int nbox, int npairs,
+                             float* stage, const int* stage_box, const bz_gather_table* tables, int ntables, int kseg,
+                             int rows, int waves, void* stream) {
+    BZ_REQUIRE(npairs >= 0 && ntables >= 0 && (ntables == 0 || (tables && stage && stage_box)),
+               "bz_yee3d_run2: bad arguments");
+    for (int t = 0; t < ntables; ++t) {
+        const bz_gather_table& g = tables[t];
+        BZ_REQUIRE(g.n > 0 && g.comp && g.stage_off && g.off && g.row && g.nfreq >= 0 &&
+                       (g.nfreq == 0 || (g.phasor && g.dft)),
+                   "bz_yee3d_run2: incomplete monitor table");
+        BZ_REQUIRE((long)g.n * (g.nfreq > 0 ? g.nfreq : 1) / 256 < (1L << 31) - 1,
+                   "bz_yee3d_run2: too many points x frequencies");
     }
+    Boxes2 bs;
+    Stage stg;
+    Fields6 F[2];
+    const int rc = check_pair("bz_yee3d_run2", src, dst, eps_r, sigma, nx, ny, nz, ld, boxes, amps, nbox, stage,
+                              stage_box, kseg, rows, waves, bs, stg, F[0], F[1]);
+    if (rc != BZ_OK || npairs == 0) return rc;
     const Coef c = make_coef(dt, mu0, eps0);
     const float rx = (float)(1.0 / dx), ry = (float)(1.0 / dy), rz = (float)(1.0 / dz);
     const hipStream_t st = (hipStream_t)stream;
-    if (waves == 16 && rows == 2) return launch<2, 16>(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, st);
-    BZ_REQUIRE(waves == 8, "bz_yee3d_step2: waves must be 8 (rows 2, 3, 4) or 16 (rows 2)");
-    switch (rows) {
-        case 2: return launch<2, 8>(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, st);
-        case 3: return launch<3, 8>(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, st);
-        case 4: return launch<4, 8>(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, c, rx, ry, rz, bs, stg, st);
-        default: bz::set_error("bz_yee3d_step2: rows must be 2, 3 or 4"); return BZ_EINVAL;
+    const long cells = (long)stg.sx * stg.sy * stg.sz;
+    // table t's arguments for pair q: its first step's samples in staging slot q & 1
+    auto of_pair = [&](int t, int q) {
+        const bz_gather_table& g = tables[t];
+        Gather3D G{};
+        const int r0 = g.row[2 * q], r1 = g.row[2 * q + 1];
+        if (r0 < 0 && r1 < 0) return G;
+        for (int k = 0; k < 6; ++k) G.base0[k] = stage + (6 * (q & 1) + k) * cells;
+        G.comp = g.comp;
+        G.off0 = g.stage_off;
+        G.off1 = g.off;
+        G.n = g.n;
+        G.act0 = r0 >= 0;
+        G.act1 = r1 >= 0;
+        G.nfreq = g.nfreq;
+        if (r0 >= 0 && g.series) G.series0 = g.series + (long)r0 * g.n;
+        if (r1 >= 0 && g.series) G.series1 = g.series + (long)r1 * g.n;
+        if (r0 >= 0 && g.nfreq) G.phasor0 = g.phasor + 2L * r0 * g.nfreq;
+        if (r1 >= 0 && g.nfreq) G.phasor1 = g.phasor + 2L * r1 * g.nfreq;
+        G.dft = g.dft;
+        return G;
+    };
+    auto gather = [&](const Gather3D& G, const Fields6& after) {
+        if (G.n == 0) return (int)BZ_OK;
+        const float* base1[6];
+        for (int k = 0; k < 6; ++k) base1[k] = after.p[k];
+        return bz_gather2(G.base0, G.off0, base1, G.comp, G.off1, G.n, G.act0, G.act1, G.series0, G.series1, G.nfreq,
+                          G.phasor0, G.phasor1, G.dft, stream);
+    };
+    // One call, since a pair on a small grid is shorter than its two Python calls were (33 us at 120x72x40; now 20 per
+    // pair with the samples). With one table, pair q - 1's samples are taken by extra workgroups of pair q's launch: its first step sits in
+    // the staging slot that launch does not write, its second step in the buffer that launch only reads
+    const bool fused = ntables == 1;
+    for (int q = 0; q < npairs; ++q) {
+        for (int k = 0; k < nbox; ++k) {
+            bs.b[k].amp = amps[(long)2 * q * nbox + k];
+            bs.amp1[k] = amps[(long)(2 * q + 1) * nbox + k];
+        }
+        bool need = false;
+        for (int t = 0; t < ntables; ++t) need = need || tables[t].row[2 * q] >= 0;
+        Stage sq = stg;
+        sq.p = need ? stage + 6 * (q & 1) * cells : nullptr;
+        const Fields6 &S = F[q & 1], &D = F[(q & 1) ^ 1];
+        const int e = launch_pair(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, rows, waves, c, rx, ry, rz, bs, sq,
+                                  fused && q > 0 ? of_pair(0, q - 1) : Gather3D{}, st);
+        if (e != BZ_OK) return e;
+        for (int t = 0; t < ntables && (!fused || q == npairs - 1); ++t) {
+            const int g = gather(of_pair(t, q), D);
+            if (g != BZ_OK) return g;
+        }
     }
+    return BZ_OK;
 }
 
 // ---------------- allocation-free variant: staging box in a library-owned device array ----------------

@@ -411,8 +411,13 @@ class Grid:
                 self._fused3d_triple(n)
                 n += 3
             elif end - n >= 2 and self.tb2 and self._pair_ok():
-                self._fused3d_pair(n)
-                n += 2
+                if self.timing or self.tb3:       # launches timed (or mixed with three-step ones) one by one
+                    self._fused3d_pair(n)
+                    n += 2
+                else:
+                    npairs = (end - n) // 2
+                    self._fused3d_pairs(n, npairs)
+                    n += 2 * npairs
             else:
                 self.step(n)
                 n += 1
@@ -495,7 +500,7 @@ class Grid:
         cells = sx * sy * sz
         if cells > max_cells:
             return False
-        buf = T.zeros(6 * cells, dtype=T.float32, device=self.dev)
+        buf = T.zeros(12 * cells, dtype=T.float32, device=self.dev)     # two slots (bz_yee3d_run2)
         for p in plans:
             o = p.off.cpu().numpy()
             pk, pr = o // plane, o % plane
@@ -503,6 +508,34 @@ class Grid:
             p.stage_off = T.from_numpy(((pk - z0) * sy + (pj - y0)) * sx + (pi - x0)).to(self.dev)
         return {"plans": plans, "buf": buf, "box": (C.c_int * 6)(x0, y0, z0, sx, sy, sz),
                 "base": N.ptrs6([buf.data_ptr() + 4 * q * cells for q in range(6)])}
+
+    def _fused3d_pairs(self, n, npairs):
+        """Steps n .. n + 2 npairs - 1 as pairs, every launch and its monitor samples from one call."""
+        steps, nb = 2 * npairs, len(self.sources)
+        arr = (N.BoxSource * N.MAX_BOX)(*[s.box[0] for s in self.sources])
+        amps = np.ascontiguousarray(np.stack([np.real(s.signal[n:n + steps]) for s in self.sources], axis=1)
+                                    if nb else np.zeros((steps, 0)), dtype=np.float32)
+        if len(amps) < steps:
+            raise IndexError(f"steps {n}..{n + steps - 1} run past a source signal")
+        stg = self._stage
+        tables, rows = [], []
+        for t in stg["plans"]:
+            row = np.full(steps, -1, np.int32)
+            rec = np.nonzero((t.record_steps >= n) & (t.record_steps < n + steps))[0]
+            if not len(rec):
+                continue
+            row[t.record_steps[rec] - n] = rec
+            rows.append(row)
+            ptr = lambda x: x.data_ptr() if x is not None else None
+            tables.append(N.GatherTable(t.comp.data_ptr(), t.stage_off.data_ptr(), t.off.data_ptr(), t.n,
+                                        row.ctypes.data, ptr(t.series), t.nfreq, ptr(t.phasor), ptr(t.dft)))
+        src, dst = self._fb[self._cur], self._fb[1 - self._cur]
+        N.call("bz_yee3d_run2", N.ptrs6([src[k].data_ptr() for k in COMP3]), N.ptrs6([dst[k].data_ptr() for k in COMP3]),
+               self.eps.data_ptr(), self.sig.data_ptr(), self.nx, self.ny, self.nz, self.ld, self.dx, self.dy, self.dz,
+               self.dt, MU_0, EPS_0, arr, amps.ctypes.data, nb, npairs, stg["buf"].data_ptr() if tables else None,
+               stg["box"] if tables else None, (N.GatherTable * max(1, len(tables)))(*tables), len(tables),
+               self.kseg2_eff(), self.rows2, self.waves2, self.stream)
+        self._cur = (self._cur + npairs) % 2
 
     def _fused3d_pair(self, n):
         """Steps n and n+1 in one launch of the two-step kernel, then the monitor samples of both."""
@@ -555,8 +588,8 @@ class Grid:
             amp2[q] = float(np.real(s.signal[n + 2]))
         stg = self._stage
         if stg["plans"] and "buf2" not in stg:
-            stg["buf2"] = self.torch.zeros_like(stg["buf"])
-            cells = stg["buf"].numel() // 6
+            cells = stg["buf"].numel() // 12
+            stg["buf2"] = stg["buf"][6 * cells:]
             stg["base2"] = N.ptrs6([stg["buf2"].data_ptr() + 4 * q * cells for q in range(6)])
         need1 = any(p.slot.get(n) is not None for p in stg["plans"])
         need2 = any(p.slot.get(n + 1) is not None for p in stg["plans"])

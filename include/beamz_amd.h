@@ -39,6 +39,7 @@
  *                           fdtd.py:200-310 restricted to d/dz = 0 (its 2D path numpy_backend.py:34-88 has
  *                           only the (Ez, Hx, Hy) family)
  *   bz_yee3d_step2 ........ two consecutive bz_yee3d_step steps in one pass (same bits)
+ *   bz_yee3d_run2 ......... many bz_yee3d_step2 passes and their monitor samples from one call
  *   bz_yee3d_step3 ........ three consecutive bz_yee3d_step steps in one pass (same bits)
  *   bz_yee2d_run2 ......... two consecutive bz_yee2d_run steps per pass (same bits, no grid power)
  *   bz_yee2d_runk ......... K consecutive bz_yee2d_run steps per pass (same bits, no grid power), with
@@ -114,6 +115,31 @@ int bz_yee3d_step2(float* const src[6], float* const dst[6], const float* eps_r,
                    int nx, int ny, int nz, int ld, double dx, double dy, double dz, double dt,
                    double mu0, double eps0, const bz_box_source* boxes, const float* amp1, int nbox,
                    float* stage, const int* stage_box, int kseg, int rows, int waves, void* stream);
+
+/* Monitor points of a bz_yee3d_run2 call: sample p reads component comp[p] (0..5) at stage_off[p] of the staging box
+ * (steps 2q) or off[p] of the fields (steps 2q + 1); row (host array, 2 * npairs entries) is each step's row of
+ * series and phasor, or -1 where the step is not recorded. */
+typedef struct bz_gather_table {
+    const int* comp;
+    const int64_t* stage_off;
+    const int64_t* off;
+    int n;
+    const int* row;
+    float* series;              /* [rows][n], or NULL */
+    int nfreq;
+    const double* phasor;       /* [rows][nfreq] complex */
+    double* dft;                /* [nfreq][n] complex accumulators */
+} bz_gather_table;
+
+/* npairs bz_yee3d_step2 passes with their monitor samples (bz_gather2), the same bits, from one call: pair q reads src
+ * and writes dst for even q and the other way round for odd q. amps (host): [2 * npairs][nbox] source amplitudes of
+ * the steps (boxes[q].amp is not read). stage: 2 slots of 6 * sx * sy * sz floats (pair q writes slot q & 1). With
+ * one table, a pair's samples are taken by extra workgroups of the next pair's launch. */
+int bz_yee3d_run2(float* const src[6], float* const dst[6], const float* eps_r, const float* sigma, int nx, int ny,
+                  int nz, int ld, double dx, double dy, double dz, double dt, double mu0, double eps0,
+                  const bz_box_source* boxes, const float* amps, int nbox, int npairs, float* stage,
+                  const int* stage_box, const bz_gather_table* tables, int ntables, int kseg, int rows, int waves,
+                  void* stream);
 
 /* ---------------- three-step 3D kernel ----------------
  * Steps n, n+1 and n+2 of bz_yee3d_step (fdtd.py:200-310 with the soft sources of helper.py:62-118, the

@@ -26,6 +26,14 @@ def test_3d_step_checks():
            match="bz_yee3d_step2: bad shape")                                  # row pitch below nx
     einval("bz_yee3d_step2", a, b, FAKE, FAKE, 10, 10, 10, 64, *geo, None, None, 1, None, None, 0, 2, 8, None,
            match="bz_yee3d_step2: bad source list")                            # a box count without boxes
+    run2 = lambda s, d, ntab, kseg, rows: einval(
+        "bz_yee3d_run2", s, d, FAKE, FAKE, 10, 10, 10, 64, *geo, None, None, 0, 4, FAKE if ntab else None,
+        (N.C.c_int * 6)(0, 0, 0, 1, 1, 1) if ntab else None, (N.GatherTable * 1)() if ntab else None, ntab, kseg, rows,
+        8, None, match="bz_yee3d_run2: " + {0: "rows must be", 1: "incomplete monitor table"}[ntab]
+        if kseg != 1 else "bz_yee3d_run2: kseg must be")
+    run2(a, b, 1, 0, 2)
+    run2(a, b, 0, 0, 5)
+    run2(a, b, 0, 1, 2)
 
 
 def test_2d_and_adjoint_checks():
