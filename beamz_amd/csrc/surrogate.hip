@@ -8,12 +8,12 @@
 // convolution weights [Co][3][3][Ci] (K = tap*Ci + ci contiguous), FP32 master
 // weights, gradients and biases.
 //
-// GEMM tiling: a workgroup of 4 waves computes a 64 x 64 tile of C = A * B^T
-// with A [M][K] and B [N][K] both staged K-contiguous in LDS, each wave one
-// 32 x 32 block: 64-wide K slices (4 MFMAs per wave and slice) for forward and
-// backward-data, 128-pixel slices (8 MFMAs) for the weight gradient; the next
-// slice's global loads are in flight during the current slice's MFMAs. The
-// operand / result lane layout of the 32x32x16 bf16 MFMA is: lane l supplies
+// GEMM tiling: a workgroup computes a tile of C = A * B^T with A [M][K] and
+// B [N][K] both staged K-contiguous in LDS, each wave blocks of 32 x 32:
+// 64-wide K slices for forward and backward-data (tiles of 64 x 64 up to
+// 128 x 128), 128-pixel slices for the weight gradient; the next slice's
+// global loads are in flight during the current slice's MFMAs. The operand /
+// result lane layout of the 32x32x16 bf16 MFMA is: lane l supplies
 // A[l%32][8*(l/32)+t] and B[8*(l/32)+t][l%32], t = 0..7, and holds
 // C[8*(r/4) + 4*(l/32) + r%4][l%32] in accumulator r = 0..15.
 //   forward: M = pixels, N = Co, K = 9*Ci, A = im2col(x) built on the fly;
@@ -62,11 +62,9 @@ __device__ __forceinline__ void pixel(int p, const Geo& g, int& b, int& y, int& 
 // Tile rows are padded to FK + 8 elements, so the consecutive lanes of an MFMA operand read (rows r .. r + 15,
 // one chunk each) fall on distinct banks; with FK = 64 the eight lanes storing a row write its 128 contiguous
 // bytes (four lanes per row, two chunks each, put two rows on the same banks).
-// TAP (Cs % FK == 0): a slice lies within one tap, so the tap and its pixel shift are computed once per slice
-// (uniform) and each lane adds offsets to its pixels' precomputed bases, instead of two integer divisions per
-// chunk and lane (the per-lane index arithmetic outweighed the MFMAs several times over).
-template <int FK, bool TAP>
-__global__ __launch_bounds__(256, TAP ? 8 : 1) void k_conv_gemm(const uint16_t* __restrict__ src, const uint16_t* __restrict__ wk,
+// The general form: k_conv_tile takes channel counts in multiples of 64 and aligned tensors.
+template <int FK>
+__global__ __launch_bounds__(256) void k_conv_gemm(const uint16_t* __restrict__ src, const uint16_t* __restrict__ wk,
                                                    const float* __restrict__ bias, uint16_t* __restrict__ out,
                                                    const uint16_t* __restrict__ mask, Geo g, int Cs, int N, int sign,
                                                    int relu) {
@@ -79,43 +77,11 @@ __global__ __launch_bounds__(256, TAP ? 8 : 1) void k_conv_gemm(const uint16_t* 
     const int t = threadIdx.x;
     const int pr = t / CPR, cq = t % CPR, kq = cq * 8;
     const int K = 9 * Cs;
-    // per staged row h: the pixel (TAP: its element offset, P * Cs < 2^31, checked by the entry points, and in
-    // bits 16 h + tap of tapok whether the tap's source pixel is inside the image; else its b, y, x)
-    int py[NH], px[NH], pofs[NH], wofs[NH];
-    unsigned tapok = 0;
+    int py[NH], px[NH], pb[NH];      // the pixel of each staged row
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-        wofs[h] = min(n0 + pr + h * RSTEP, N - 1) * K + kq;   // N * K < 2^31 (checked by the entry points)
-        int pb;
-        pixel(min(m0 + pr + h * RSTEP, P - 1), g, pb, py[h], px[h]);
-        pofs[h] = TAP ? ((pb * g.H + py[h]) * g.W + px[h]) * Cs + kq : pb;
-        if (TAP && m0 + pr + h * RSTEP < P) {
-#pragma unroll
-            for (int tap = 0; tap < 9; ++tap) {
-                const int yy = py[h] + sign * (tap / 3 - 1), xx = px[h] + sign * (tap % 3 - 1);
-                if (yy >= 0 && yy < g.H && xx >= 0 && xx < g.W) tapok |= 1u << (16 * h + tap);
-            }
-        }
-    }
+    for (int h = 0; h < NH; ++h) pixel(min(m0 + pr + h * RSTEP, P - 1), g, pb[h], py[h], px[h]);
     uint4 a[NH], bw[NH];
     auto load = [&](int k0) {
-        if (TAP) {
-            const int tap = k0 / Cs;
-            const int ky = tap / 3, kx = tap - 3 * ky;
-            const int dy = sign * (ky - 1), dx = sign * (kx - 1);
-            const int cs = k0 - tap * Cs;
-            const int shift = (dy * g.W + dx) * Cs;
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                const bool ok = (tapok >> (16 * h + tap)) & 1u;
-                // every lane loads from a valid address (its own pixel where the tap falls outside) and selects 0
-                const uint4 v = *reinterpret_cast<const uint4*>(src + pofs[h] + cs + (ok ? shift : 0));
-                const uint4 w = *reinterpret_cast<const uint4*>(wk + wofs[h] + k0);
-                a[h] = ok ? v : make_uint4(0, 0, 0, 0);
-                bw[h] = n0 + pr + h * RSTEP < N ? w : make_uint4(0, 0, 0, 0);
-            }
-            return;
-        }
         const int k = k0 + kq;
         const int tap = k / Cs, c = k - tap * Cs;
         const int ky = tap / 3, kx = tap - 3 * (tap / 3);
@@ -126,7 +92,7 @@ __global__ __launch_bounds__(256, TAP ? 8 : 1) void k_conv_gemm(const uint16_t* 
             if (k < K) {
                 const int yy = py[h] + sign * (ky - 1), xx = px[h] + sign * (kx - 1);
                 if (m0 + pr + h * RSTEP < P && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
-                    a[h] = *reinterpret_cast<const uint4*>(src + (((long)pofs[h] * g.H + yy) * g.W + xx) * Cs + c);
+                    a[h] = *reinterpret_cast<const uint4*>(src + (((long)pb[h] * g.H + yy) * g.W + xx) * Cs + c);
                 const int nrow = n0 + pr + h * RSTEP;
                 if (nrow < N) bw[h] = *reinterpret_cast<const uint4*>(wk + (long)nrow * K + k);
             }
@@ -168,6 +134,178 @@ __global__ __launch_bounds__(256, TAP ? 8 : 1) void k_conv_gemm(const uint16_t* 
             if (relu) v = fmaxf(v, 0.0f);
             const long o = (long)m * N + n;
             out[o] = (mask && !(b2f(mask[o]) > 0.0f)) ? (uint16_t)0 : f2b(v);
+        }
+    }
+}
+
+// The halves of v where those of y are positive, else 0 (the ReLU derivative).
+__device__ __forceinline__ uint4 keep_positive(uint4 v, const uint4& y) {
+    uint16_t* vh = reinterpret_cast<uint16_t*>(&v);
+    const uint16_t* yh = reinterpret_cast<const uint16_t*>(&y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        if (!(b2f(yh[e]) > 0.0f)) vh[e] = 0;
+    return v;
+}
+
+// Forward (sign = +1) or backward-data (sign = -1) 3x3 convolution as an implicit GEMM (Cs % 64 == 0, N % TN == 0).
+// A workgroup of WM x WN waves computes TM = 32 MI WM pixels x TN = 32 NI WN channels, each wave MI x NI blocks of
+// 32 x 32, in slices of 64 input channels of one tap. Both operands of a slice go from memory into LDS without
+// registers (16 bytes per lane, 8 rows of 128 bytes per wave and instruction), the next slice's while the current
+// one's MFMAs run; a tap outside the image, or a pixel past the last, is an offset past the end of the buffer, which
+// the hardware reads as zeros. Rows are not padded (such a load writes 1 KB in a row): chunk c of row r sits in
+// place c ^ ((r >> 1) & 7), which puts the 16 rows of an operand read on distinct banks.
+// The MFMA takes the weights as its first operand: a lane holds one pixel and 4 consecutive channels in 4
+// accumulators; after an exchange with lane +-32 it stores 8 channels, 16 bytes, at once.
+// Bound by the matrix units' issue with 2 to 4 waves per SIMD (850 to 910 TFLOP/s on 16- and 32-pixel rows at 256 and
+// 128 channels, where a library's 8192^3 product reaches 1118); with 64 channels, whose 9 slices are soon over, by
+// filling and draining the pipeline. Batch 128, us, against 64 x 64 tiles staged through registers (the same bits):
+// 16 x 16, 256 -> 256 78 -> 43, 128 -> 256 38 -> 23; 32 x 32, 128 -> 128 69 -> 46, 64 -> 128 39 -> 28; 64 x 64,
+// 64 -> 64 73 -> 60 (row march). 8 waves of 64 x 32 per 128 x 128 tile rather than 4 of 64 x 64 (46 on the first).
+constexpr uint32_t OUTSIDE = 0xFFFFFFF0u;      // past every buffer: their sizes are multiples of 128 bytes
+
+__device__ __forceinline__ uint32_t f2b2(float lo, float hi) { return (uint32_t)f2b(lo) | ((uint32_t)f2b(hi) << 16); }
+
+__device__ __forceinline__ void to_lds(__amdgpu_buffer_rsrc_t r, uint16_t* lds, uint32_t off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
+}
+
+template <int WM, int WN, int MI, int NI>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* __restrict__ src,
+                                                            const uint16_t* __restrict__ wk,
+                                                            const float* __restrict__ bias, uint16_t* __restrict__ out,
+                                                            const uint16_t* __restrict__ mask, Geo g, int Cs, int N,
+                                                            int sign, int relu, int mtiles, int per_xcd) {
+    constexpr int WV = WM * WN, BM = 32 * MI * WM, BN = 32 * NI * WN;
+    constexpr int NA = BM / 8 / WV, NB = BN / 8 / WV;      // loads of a wave per slice
+    static_assert(NA >= 1 && NB >= 1 && NA * 8 * WV == BM && NB * 8 * WV == BN, "whole loads per wave");
+    // (separate arrays, each used by one half of the loop: the compiler then knows that a slice's operand reads do
+    // not touch what the loads in flight write)
+    __shared__ __attribute__((aligned(16))) uint16_t A0[BM * 64], A1[BM * 64], B0[BN * 64], B1[BN * 64];
+    // consecutive pixel tiles, which share input rows, on one XCD
+    const int tile = ((int)blockIdx.x % 8) * per_xcd + (int)blockIdx.x / 8;
+    if (tile >= mtiles) return;
+    const int P = g.B * g.H * g.W, K = 9 * Cs;
+    const int m0 = tile * BM, n0 = blockIdx.y * BN;
+    const int t = threadIdx.x, l = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(src), 0, (int)((uint32_t)P * (uint32_t)Cs * 2u),
+                                                      0x00020000);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wk), 0, N * K * 2, 0x00020000);
+    uint32_t pofs[NA], wofs[NB];
+    uint32_t tapok[NA];
+#pragma unroll
+    for (int h = 0; h < NA; ++h) {
+        const int row = (wave * NA + h) * 8 + (l >> 3), m = m0 + row;
+        const int cq = (l & 7) ^ ((row >> 1) & 7);
+        int pb, py, px;
+        pixel(min(m, P - 1), g, pb, py, px);
+        pofs[h] = 2u * ((uint32_t)min(m, P - 1) * (uint32_t)Cs + 8u * cq);
+        // (columns a tap may have | the rows it may have) per kernel row and column of the tap
+        const uint32_t left = sign > 0 ? px > 0 : px + 1 < g.W, right = sign > 0 ? px + 1 < g.W : px > 0;
+        const uint32_t up = sign > 0 ? py > 0 : py + 1 < g.H, down = sign > 0 ? py + 1 < g.H : py > 0;
+        const uint32_t cols = left | 2u | right << 2;
+        tapok[h] = m < P ? (up ? cols : 0u) | cols << 3 | (down ? cols << 6 : 0u) : 0u;
+    }
+#pragma unroll
+    for (int h = 0; h < NB; ++h) {
+        const int row = (wave * NB + h) * 8 + (l >> 3);
+        wofs[h] = 2u * ((uint32_t)(n0 + row) * (uint32_t)K + 8u * ((l & 7) ^ ((row >> 1) & 7)));
+    }
+    const int per_tap = Cs / 64, slices = 9 * per_tap;
+    auto load = [&](uint16_t* a, uint16_t* b, int s) {
+        const int tap = s / per_tap, cs = 64 * (s - tap * per_tap);
+        const int ky = tap / 3, kx = tap - 3 * ky;
+        const uint32_t shift = 2u * (uint32_t)((sign * ((ky - 1) * g.W + kx - 1)) * Cs + cs);
+#pragma unroll
+        for (int h = 0; h < NA; ++h)
+            to_lds(rs, a + (wave * NA + h) * 512, (tapok[h] >> tap) & 1u ? pofs[h] + shift : OUTSIDE);
+#pragma unroll
+        for (int h = 0; h < NB; ++h) to_lds(rw, b + (wave * NB + h) * 512, wofs[h] + 128u * (uint32_t)s);
+    };
+    f32x16 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    const int wm = wave % WM, wn = wave / WM;
+    const int row = l & 31, g2 = l >> 5, sw = (row >> 1) & 7;
+    auto compute = [&](const uint16_t* a, const uint16_t* b) {
+        const uint16_t* ar = a + (wm * 32 * MI + row) * 64;
+        const uint16_t* br = b + (wn * 32 * NI + row) * 64;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const int c = 8 * ((2 * kk + g2) ^ sw);
+            bf16x8 av[MI], bv[NI];
+#pragma unroll
+            for (int i = 0; i < MI; ++i) av[i] = *reinterpret_cast<const bf16x8*>(ar + i * 2048 + c);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) bv[j] = *reinterpret_cast<const bf16x8*>(br + j * 2048 + c);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv[j], av[i], acc[i][j], 0, 0, 0);
+        }
+    };
+    // every load of this wave is in LDS, then every wave's; nobody still reads what the next loads overwrite
+    auto sync = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    load(A0, B0, 0);
+    sync();
+    int s = 0;
+    for (; s + 2 < slices; s += 2) {
+        load(A1, B1, s + 1);
+        compute(A0, B0);
+        sync();
+        load(A0, B0, s + 2);
+        compute(A1, B1);
+        sync();
+    }
+    if (s + 1 < slices) load(A1, B1, s + 1);
+    compute(A0, B0);
+    if (s + 1 < slices) {
+        sync();
+        compute(A1, B1);
+    }
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+        const int nb = n0 + (wn * NI + j) * 32;
+        float bb[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) bb[q][k] = bias ? bias[nb + 8 * q + 4 * g2 + k] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int m = m0 + (wm * MI + i) * 32 + row;
+            const long o = (long)m * N + nb + 8 * g2;
+#pragma unroll
+            for (int q = 0; q < 4; q += 2) {
+                uint32_t d[2][2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    float v[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        v[k] = acc[i][j][4 * (q + e) + k] + bb[q + e][k];
+                        v[k] = (relu != 0) & !(v[k] > 0.0f) ? 0.0f : v[k];
+                    }
+                    d[e][0] = f2b2(v[0], v[1]);
+                    d[e][1] = f2b2(v[2], v[3]);
+                }
+                // lower lanes: channels 8q .. 8q + 7; upper lanes: 8q + 8 .. 8q + 15
+                const auto s0 = __builtin_amdgcn_permlane32_swap(d[0][0], d[1][0], false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(d[0][1], d[1][1], false, false);
+                uint4 v = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+                if (m < P) {
+                    if (mask) v = keep_positive(v, *reinterpret_cast<const uint4*>(mask + o + 8 * q));
+                    *reinterpret_cast<uint4*>(out + o + 8 * q) = v;
+                }
+            }
         }
     }
 }
@@ -299,7 +437,7 @@ __global__ __launch_bounds__(64 * (W / 32) * (CB / 32)) void k_conv_march(const 
 // MFMAs run. Needs H*W % 64 == 0 and W % 64 == 0 or 64 % W == 0, Cs % CC == 0.
 // Used for 32-channel inputs (level-0 layers: 172 -> 139 us for batch 128 at 128 x 128). With 64 or more
 // channels the direct weight reads (1 KB per MFMA and wave from L2) cost more than the tap re-reads they
-// replace (92 -> 125 us), so those layers keep k_conv_gemm; staging the weights in LDS is the next step.
+// replace (92 -> 125 us), so those layers take k_conv_tile.
 template <int CC>
 __global__ __launch_bounds__(256) void k_conv_halo(const uint16_t* __restrict__ src, const uint16_t* __restrict__ wk,
                                                    const float* __restrict__ bias, uint16_t* __restrict__ out, const uint16_t* __restrict__ mask, Geo g,
@@ -1369,7 +1507,8 @@ inline dim3 rows_grid(long per_row, long rows) {
 
 // Row-march convolution for rows of 64 or 128 pixels: input channels 32 (or 64 for 64-pixel rows), output
 // channels in blocks of 32 (64 where 32 input channels meet 64-pixel rows); bands of at least 16 rows, about
-// 1024 workgroups. Returns false where no shape applies (the caller takes the tiled GEMM).
+// 1024 workgroups, or, where those are fewer than two per CU, of at least 4 rows, 512 workgroups (128 x 128, 32 -> 32,
+// batch 16: 23.6 -> 12.6 us, batch 2: 21.0 -> 7.8). Returns false where no shape applies (the caller takes a GEMM).
 static bool conv_march(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out, const uint16_t* mask,
                        int B, int H, int W, int Cin, int Cout, int sign, int relu, hipStream_t st) {
     int cb;
@@ -1379,7 +1518,7 @@ static bool conv_march(const uint16_t* src, const uint16_t* wk, const float* bia
     else return false;
     const long rows = (long)B * H;
     const long nblk = Cout / cb;
-    long nz = std::max(1L, std::min(rows / 16, 1024 / nblk));
+    long nz = std::max(1L, std::max(std::min(rows / 16, 1024 / nblk), std::min(rows / 4, 512 / nblk)));
     const int band = (int)((rows + nz - 1) / nz);
     nz = (rows + band - 1) / band;
     const dim3 grid(1, (unsigned)nblk, (unsigned)nz);
@@ -1414,6 +1553,39 @@ static bool conv_march(const uint16_t* src, const uint16_t* wk, const float* bia
     return true;
 }
 
+template <int WM, int WN, int MI, int NI>
+static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out,
+                        const uint16_t* mask, const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
+    const long P = (long)g.B * g.H * g.W;
+    const int mt = (int)((P + 32 * MI * WM - 1) / (32 * MI * WM)), per_xcd = (mt + 7) / 8;
+    hipLaunchKernelGGL((k_conv_tile<WM, WN, MI, NI>), dim3(per_xcd * 8, Cout / (32 * NI * WN)), dim3(64 * WM * WN), 0,
+                       st, src, wk, bias, out, mask, g, Cin, Cout, sign, relu, mt, per_xcd);
+}
+
+// The tiled convolution (k_conv_tile): 64-channel slices, tensors aligned to its 16-byte accesses, weights of 32-bit
+// offsets. Tiles of 128 x 128 while they give every CU one (16 x 16 x 256 -> 256: batch 128 43 us, 64-wide ones 55;
+// at batch 16, 64 tiles, 21 against 15), then 128 x 64 on the same terms (64 x 64 x 64 -> 64, batch 128: 60 us,
+// 64 x 64 tiles 67), then 64 x 64 (16 x 16 x 256 -> 256, batch 16: 14 us, 128 x 64 tiles 15). 32-channel remainders
+// take 128 x 32, except 64-pixel rows in numbers that fill the row march (64 -> 32 channels: batch 128 36 us against
+// 42 here, batch 16 30 against 9).
+static bool conv_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out, const uint16_t* mask,
+                      const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
+    const uintptr_t all = (uintptr_t)src | (uintptr_t)wk | (uintptr_t)out | (uintptr_t)mask;
+    if (Cin % 64 || (all & 15) || 18L * Cin * Cout >= (1L << 31)) return false;
+    const long P = (long)g.B * g.H * g.W, mt = (P + 127) / 128;
+    if (Cout % 64) {
+        if (g.W == 64 && Cin == 64 && (long)g.B * g.H / 16 * (Cout / 32) >= 512) return false;
+        launch_tile<4, 1, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+    } else if (Cout % 128 == 0 && mt * (Cout / 128) >= 256) {
+        launch_tile<2, 4, 2, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+    } else if (mt * (Cout / 64) >= 256) {
+        launch_tile<4, 2, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+    } else {
+        launch_tile<2, 2, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+    }
+    return true;
+}
+
 extern "C" int bz_nn_conv3x3(const uint16_t* x, const uint16_t* w16, const float* bias, uint16_t* y, int B, int H,
                              int W, int Ci, int Co, int relu, void* stream) {
     BZ_REQUIRE(x && w16 && y && B > 0 && H > 0 && W > 0, "bz_nn_conv3x3: bad arguments");
@@ -1421,14 +1593,15 @@ extern "C" int bz_nn_conv3x3(const uint16_t* x, const uint16_t* w16, const float
     const long P = (long)B * H * W;
     BZ_REQUIRE(P * (long)(Ci > Co ? Ci : Co) < (1L << 31), "bz_nn_conv3x3: tensor too large");
     Geo g{B, H, W};
-    if (conv_march(x, w16, bias, y, nullptr, B, H, W, Ci, Co, 1, relu, (hipStream_t)stream))
+    if (conv_tile(x, w16, bias, y, nullptr, g, Ci, Co, 1, relu, (hipStream_t)stream))
+        ;
+    else if (conv_march(x, w16, bias, y, nullptr, B, H, W, Ci, Co, 1, relu, (hipStream_t)stream))
         ;
     else if (halo_ok(g) && Ci == 32)
         hipLaunchKernelGGL(k_conv_halo<32>, dim3((unsigned)(P / 64), (Co + TN - 1) / TN), dim3(256), 0,
                            (hipStream_t)stream, x, w16, bias, y, (const uint16_t*)nullptr, g, Ci, Co, 1, relu);
     else
-        hipLaunchKernelGGL((Ci % 64 == 0 ? k_conv_gemm<64, true>
-                                         : ((9 * Ci) % 64 == 0 ? k_conv_gemm<64, false> : k_conv_gemm<32, false>)),
+        hipLaunchKernelGGL(((9 * Ci) % 64 == 0 ? k_conv_gemm<64> : k_conv_gemm<32>),
                            dim3((unsigned)((P + TM - 1) / TM), (Co + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream,
                            x, w16, bias, y, (const uint16_t*)nullptr, g, Ci, Co, 1, relu);
     BZ_CHECK_LAUNCH("bz_nn_conv3x3");
@@ -1451,14 +1624,15 @@ static int conv_dgrad(const uint16_t* gz, const uint16_t* wt16, const uint16_t* 
         return BZ_EINVAL;
     }
     Geo g{B, H, W};
-    if (conv_march(gz, wt16, nullptr, gx, mask, B, H, W, Co, Ci, -1, 0, (hipStream_t)stream))
+    if (conv_tile(gz, wt16, nullptr, gx, mask, g, Co, Ci, -1, 0, (hipStream_t)stream))
+        ;
+    else if (conv_march(gz, wt16, nullptr, gx, mask, B, H, W, Co, Ci, -1, 0, (hipStream_t)stream))
         ;
     else if (halo_ok(g) && Co == 32)
         hipLaunchKernelGGL(k_conv_halo<32>, dim3((unsigned)(P / 64), (Ci + TN - 1) / TN), dim3(256), 0,
                            (hipStream_t)stream, gz, wt16, (const float*)nullptr, gx, mask, g, Co, Ci, -1, 0);
     else
-        hipLaunchKernelGGL((Co % 64 == 0 ? k_conv_gemm<64, true>
-                                         : ((9 * Co) % 64 == 0 ? k_conv_gemm<64, false> : k_conv_gemm<32, false>)),
+        hipLaunchKernelGGL(((9 * Co) % 64 == 0 ? k_conv_gemm<64> : k_conv_gemm<32>),
                            dim3((unsigned)((P + TM - 1) / TM), (Ci + TN - 1) / TN), dim3(256), 0, (hipStream_t)stream,
                            gz, wt16, (const float*)nullptr, gx, mask, g, Co, Ci, -1, 0);
     BZ_CHECK_LAUNCH(name);
