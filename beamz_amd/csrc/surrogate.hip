@@ -1719,8 +1719,14 @@ static void tree_sum2(const SumSeg& a, const SumSeg& b, float* scratch, hipStrea
 // R = max(1, 64 / W) rows per step: 32-wide channel blocks on 128-pixel rows, 64-wide where the counts allow
 // otherwise (16- and 32-pixel rows need 64-wide output blocks, 16-pixel rows 64-wide input blocks too; on
 // the deep levels they measured faster than 32-wide blocks with fewer bands). The rows are cut into nz bands
-// (multiples of R rows) for about 2048 workgroups, at least 16 rows per band, at most 8 M (64- and 128-pixel
-// rows) or 16 M partial floats (the ordered sums read them all).
+// (multiples of R rows). Four and more channel blocks: one workgroup per place on the chip (a CU holds one of 6 or 12
+// waves at these kernels' 166 to 174 registers, two of 3 waves), at least 16 rows per band: more bands only add partial
+// sums to write and read back (about 2048 workgroups, at most 8 M (64- and 128-pixel rows) or 16 M partial floats,
+// measured at batch 128, us with the sums, before / after: 16 x 16 256 -> 256 97 / 80, 128 -> 256 63 / 49, 32 x 32
+// 128 -> 128 83 / 68). Fewer blocks keep that older count, whose partial rows the tests of the ordered sums are
+// written for, raised to one workgroup per place with bands of 4 rows for rows of 64 and more pixels (64 x 64
+// 64 -> 64, batch 16: 30 us with 16-row bands, 25 with 4). Halving some bands so that every place gets the same
+// number of rows measured slower than equal ones (56 -> 59 us at 32 x 32 64 -> 128).
 struct MarchPlan {
     bool ok;
     int nco, nci, rows_per_step, nz, band;
@@ -1736,9 +1742,15 @@ inline MarchPlan march_plan(int B, int H, int W, int Ci, int Co) {
     const long rows = (long)B * H;
     const long nblk = (long)(Co / (32 * nco)) * (Ci / (32 * nci));
     const long nw = (long)Co * 9 * Ci;
-    long nz = std::max(1L, 2048 / nblk);
-    nz = std::min(nz, std::max(1L, rows / 16));
-    nz = std::min(nz, std::max(1L, (W >= 64 ? 8L << 20 : 16L << 20) / nw));
+    const long places = 256 * (nco + nci >= 3 ? 1 : 2) / nblk;
+    long nz;
+    if (nblk >= 4) {
+        nz = std::max(1L, std::min(places, rows / 16));
+    } else {
+        nz = std::min(2048 / nblk, std::max(1L, rows / 16));
+        nz = std::min(nz, std::max(1L, (W >= 64 ? 8L << 20 : 16L << 20) / nw));
+        if (W >= 64) nz = std::max(nz, std::min(places, rows / 4));
+    }
     long band = (rows + nz - 1) / nz;
     band = (band + R - 1) / R * R;
     m.ok = true;
