@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 namespace {
 
@@ -151,8 +152,8 @@ __device__ __forceinline__ uint4 keep_positive(uint4 v, const uint4& y) {
 // Forward (sign = +1) or backward-data (sign = -1) 3x3 convolution as an implicit GEMM (Cs % 64 == 0, N % TN == 0).
 // A workgroup of WM x WN waves computes TM = 32 MI WM pixels x TN = 32 NI WN channels, each wave MI x NI blocks of
 // 32 x 32, in slices of 64 input channels of one tap. Both operands of a slice go from memory into LDS without
-// registers (16 bytes per lane, 8 rows of 128 bytes per wave and instruction), the next slice's while the current
-// one's MFMAs run; a tap outside the image, or a pixel past the last, is an offset past the end of the buffer, which
+// registers (16 bytes per lane, 8 rows of 128 bytes per wave and instruction), those of the next ST - 1 slices in
+// flight while the current one's MFMAs run (ST 2 or 4 slots); a tap outside the image, or a pixel past the last, is an offset past the end of the buffer, which
 // the hardware reads as zeros. Rows are not padded (such a load writes 1 KB in a row): chunk c of row r sits in
 // place c ^ ((r >> 1) & 7), which puts the 16 rows of an operand read on distinct banks.
 // The MFMA takes the weights as its first operand: a lane holds one pixel and 4 consecutive channels in 4
@@ -170,7 +171,7 @@ __device__ __forceinline__ void to_lds(__amdgpu_buffer_rsrc_t r, uint16_t* lds, 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
 }
 
-template <int WM, int WN, int MI, int NI>
+template <int WM, int WN, int MI, int NI, int ST>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* __restrict__ src,
                                                             const uint16_t* __restrict__ wk,
                                                             const float* __restrict__ bias, uint16_t* __restrict__ out,
@@ -182,6 +183,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
     // (separate arrays, each used by one half of the loop: the compiler then knows that a slice's operand reads do
     // not touch what the loads in flight write)
     __shared__ __attribute__((aligned(16))) uint16_t A0[BM * 64], A1[BM * 64], B0[BN * 64], B1[BN * 64];
+    __shared__ __attribute__((aligned(16))) uint16_t A2[ST == 4 ? BM * 64 : 8], A3[ST == 4 ? BM * 64 : 8],
+        B2[ST == 4 ? BN * 64 : 8], B3[ST == 4 ? BN * 64 : 8];
     // consecutive pixel tiles, which share input rows, on one XCD
     const int tile = ((int)blockIdx.x % 8) * per_xcd + (int)blockIdx.x / 8;
     if (tile >= mtiles) return;
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
         for (int h = 0; h < NA; ++h)
             to_lds(rs, a + (wave * NA + h) * 512, (tapok[h] >> tap) & 1u ? pofs[h] + shift : OUTSIDE);
 #pragma unroll
-        for (int h = 0; h < NB; ++h) to_lds(rw, b + (wave * NB + h) * 512, wofs[h] + 128u * (uint32_t)s);
+        for (int h = 0; h < NB; ++h) to_lds(rw, b + (wave * NB + h) * 512, s < slices ? wofs[h] + 128u * (uint32_t)s : OUTSIDE);
     };
     f32x16 acc[MI][NI];
 #pragma unroll
@@ -249,27 +252,67 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv[j], av[i], acc[i][j], 0, 0, 0);
         }
     };
-    // every load of this wave is in LDS, then every wave's; nobody still reads what the next loads overwrite
-    auto sync = [&]() {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+    // the slice about to be read is in LDS (this wave's loads, then every wave's), and nobody still reads what the
+    // next loads overwrite; `ahead` later slices may stay in flight (a __syncthreads would wait for them too)
+    auto sync = [&](auto ahead) {
+        constexpr int V = (NA + NB) * decltype(ahead)::value;
+        static_assert(V < 64, "vmcnt");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(V) : "memory");
     };
-    load(A0, B0, 0);
-    sync();
-    int s = 0;
-    for (; s + 2 < slices; s += 2) {
-        load(A1, B1, s + 1);
+    typedef std::integral_constant<int, 0> I0;
+    typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 2> I2;
+    if constexpr (ST == 2) {
+        load(A0, B0, 0);
+        sync(I0());
+        int s = 0;
+        for (; s + 2 < slices; s += 2) {
+            load(A1, B1, s + 1);
+            compute(A0, B0);
+            sync(I0());
+            load(A0, B0, s + 2);
+            compute(A1, B1);
+            sync(I0());
+        }
+        if (s + 1 < slices) load(A1, B1, s + 1);
         compute(A0, B0);
-        sync();
-        load(A0, B0, s + 2);
-        compute(A1, B1);
-        sync();
-    }
-    if (s + 1 < slices) load(A1, B1, s + 1);
-    compute(A0, B0);
-    if (s + 1 < slices) {
-        sync();
-        compute(A1, B1);
+        if (s + 1 < slices) {
+            sync(I0());
+            compute(A1, B1);
+        }
+    } else {
+        // slices >= 9: three in flight; the last rounds load past the end (weights and taps outside: zeros)
+        load(A0, B0, 0);
+        load(A1, B1, 1);
+        load(A2, B2, 2);
+        int s = 0;
+        for (; s + 4 <= slices; s += 4) {
+            sync(I2());
+            load(A3, B3, s + 3);
+            compute(A0, B0);
+            sync(I2());
+            load(A0, B0, s + 4);
+            compute(A1, B1);
+            sync(I2());
+            load(A1, B1, s + 5);
+            compute(A2, B2);
+            sync(I2());
+            load(A2, B2, s + 6);
+            compute(A3, B3);
+        }
+        if (s < slices) {
+            sync(I2());
+            compute(A0, B0);
+        }
+        if (s + 1 < slices) {
+            sync(I1());
+            compute(A1, B1);
+        }
+        if (s + 2 < slices) {
+            sync(I0());
+            compute(A2, B2);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing lands in LDS after this workgroup
     }
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
@@ -292,7 +335,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         v[k] = acc[i][j][4 * (q + e) + k] + bb[q + e][k];
-                        v[k] = (relu != 0) & !(v[k] > 0.0f) ? 0.0f : v[k];
+                        v[k] = ((relu != 0) & !(v[k] > 0.0f)) ? 0.0f : v[k];
                     }
                     d[e][0] = f2b2(v[0], v[1]);
                     d[e][1] = f2b2(v[2], v[3]);
@@ -1048,14 +1091,16 @@ __global__ __launch_bounds__(256) void k_conv_first_rows(const uint16_t* __restr
         const int yy = y0 + ry - 1, xx = rx - 1;
         xs[q] = (yy >= 0 && yy < g.H && xx >= 0 && xx < W) ? b2f(x[((long)bi * g.H + yy) * W + xx]) : 0.0f;
     }
+    float* wl = xs + (RB + 2) * WP;           // the weights once through LDS: a thread's 72 lie 9 apart in memory
+    for (int q = t; q < 9 * Co; q += 256) wl[q] = b2f(f2b(w[q]));
     float wv[8][9], bv[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap) wv[e][tap] = b2f(f2b(w[(c + e) * 9 + tap]));
-        bv[e] = b[c + e];
-    }
+    for (int e = 0; e < 8; ++e) bv[e] = b[c + e];
     __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) wv[e][tap] = wl[(c + e) * 9 + tap];
     uint16_t* __restrict__ yc = y + (long)row0 * W * Co + c;
     int ly = r / W, lx = r - (r / W) * W;
     for (int q = r; q < RB * W; q += R) {
@@ -1374,14 +1419,16 @@ __global__ void k_head(const uint16_t* __restrict__ a, const float* __restrict__
     }
 }
 
-// The head with 8 channels per thread: a workgroup of 256 threads per sample splits its pixels into S = 256 / (C / 8)
+// The head with 8 channels per thread: a workgroup of 1024 threads per sample splits its pixels into S = 1024 / (C / 8)
 // interleaved slices (thread t: channels 8 (t % (C / 8)) .. +7 by 16-byte loads, pixels t / (C / 8) + S k); the
-// slices' sums are added in slice order in LDS (deterministic). C % 8 == 0 and 256 % (C / 8) == 0.
-__global__ __launch_bounds__(256) void k_head8(const uint16_t* __restrict__ a, const float* __restrict__ fw,
-                                               const float* __restrict__ fb, float* __restrict__ gap,
-                                               float* __restrict__ out, int HW, int C, int nout) {
+// slices' sums are added in slice order in LDS, and 32 lanes share an output (deterministic). C % 8 == 0 and
+// 256 % (C / 8) == 0. Bound by the latency of its dependent passes, at any batch: 256 threads with one lane per output
+// took 17 us at 256 pixels x 256 channels, this 7.5.
+__global__ __launch_bounds__(1024) void k_head8(const uint16_t* __restrict__ a, const float* __restrict__ fw,
+                                                const float* __restrict__ fb, float* __restrict__ gap,
+                                                float* __restrict__ out, int HW, int C, int nout) {
     extern __shared__ float sh[];
-    const int G = C / 8, S = 256 / G;
+    const int G = C / 8, S = 1024 / G;
     float* red = sh;             // [S][C]
     float* sg = sh + S * C;      // [C]
     const int b = blockIdx.x, t = threadIdx.x, cg = t % G, sl = t / G;
@@ -1399,17 +1446,20 @@ __global__ __launch_bounds__(256) void k_head8(const uint16_t* __restrict__ a, c
 #pragma unroll
     for (int e = 0; e < 8; ++e) red[sl * C + 8 * cg + e] = acc[e];
     __syncthreads();
-    for (int c = t; c < C; c += 256) {
+    for (int c = t; c < C; c += 1024) {
         float v = 0.0f;
+#pragma unroll 8
         for (int q = 0; q < S; ++q) v += red[q * C + c];
         sg[c] = v / (float)HW;
         gap[(long)b * C + c] = sg[c];
     }
     __syncthreads();
-    for (int j = t; j < nout; j += 256) {
-        float v = fb[j];
-        for (int c = 0; c < C; ++c) v += fw[j * C + c] * sg[c];
-        out[(long)b * nout + j] = v;
+    for (int j = t / 32; j < nout; j += 32) {
+        float v = 0.0f;
+#pragma unroll 8
+        for (int c = t % 32; c < C; c += 32) v += fw[j * C + c] * sg[c];
+        for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off);
+        if (t % 32 == 0) out[(long)b * nout + j] = fb[j] + v;
     }
 }
 
@@ -1553,12 +1603,12 @@ static bool conv_march(const uint16_t* src, const uint16_t* wk, const float* bia
     return true;
 }
 
-template <int WM, int WN, int MI, int NI>
+template <int WM, int WN, int MI, int NI, int ST>
 static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out,
                         const uint16_t* mask, const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
     const long P = (long)g.B * g.H * g.W;
     const int mt = (int)((P + 32 * MI * WM - 1) / (32 * MI * WM)), per_xcd = (mt + 7) / 8;
-    hipLaunchKernelGGL((k_conv_tile<WM, WN, MI, NI>), dim3(per_xcd * 8, Cout / (32 * NI * WN)), dim3(64 * WM * WN), 0,
+    hipLaunchKernelGGL((k_conv_tile<WM, WN, MI, NI, ST>), dim3(per_xcd * 8, Cout / (32 * NI * WN)), dim3(64 * WM * WN), 0,
                        st, src, wk, bias, out, mask, g, Cin, Cout, sign, relu, mt, per_xcd);
 }
 
@@ -1567,7 +1617,9 @@ static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bi
 // at batch 16, 64 tiles, 21 against 15), then 128 x 64 on the same terms (64 x 64 x 64 -> 64, batch 128: 60 us,
 // 64 x 64 tiles 67), then 64 x 64 (16 x 16 x 256 -> 256, batch 16: 14 us, 128 x 64 tiles 15). 32-channel remainders
 // take 128 x 32, except 64-pixel rows in numbers that fill the row march (64 -> 32 channels: batch 128 36 us against
-// 42 here, batch 16 30 against 9).
+// 42 here, batch 16 30 against 9). Where a CU gets one tile at most, nothing runs beside its barriers: three slices
+// in flight there (16 x 16 256 -> 256, batch 16: 15 -> 11 us, 256 -> 128, batch 128: 30 -> 23), one where two or more
+// tiles share a CU and the LDS (64 x 64 64 -> 64, batch 128: 63 us, 93 with three).
 static bool conv_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out, const uint16_t* mask,
                       const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
     const uintptr_t all = (uintptr_t)src | (uintptr_t)wk | (uintptr_t)out | (uintptr_t)mask;
@@ -1575,13 +1627,15 @@ static bool conv_tile(const uint16_t* src, const uint16_t* wk, const float* bias
     const long P = (long)g.B * g.H * g.W, mt = (P + 127) / 128;
     if (Cout % 64) {
         if (g.W == 64 && Cin == 64 && (long)g.B * g.H / 16 * (Cout / 32) >= 512) return false;
-        launch_tile<4, 1, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+        launch_tile<4, 1, 1, 1, 2>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     } else if (Cout % 128 == 0 && mt * (Cout / 128) >= 256) {
-        launch_tile<2, 4, 2, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+        (mt * (Cout / 128) > 256 ? launch_tile<2, 4, 2, 1, 2> : launch_tile<2, 4, 2, 1, 4>)(
+            src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     } else if (mt * (Cout / 64) >= 256) {
-        launch_tile<4, 2, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+        (mt * (Cout / 64) > 256 ? launch_tile<4, 2, 1, 1, 2> : launch_tile<4, 2, 1, 1, 4>)(
+            src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     } else {
-        launch_tile<2, 2, 1, 1>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+        launch_tile<2, 2, 1, 1, 4>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     }
     return true;
 }
@@ -1835,11 +1889,14 @@ extern "C" int bz_nn_conv_first(const uint16_t* x, const float* w, const float* 
                                 int Co, void* stream) {
     BZ_REQUIRE(x && w && b && y && B > 0 && H > 0 && W > 0 && Co > 0, "bz_nn_conv_first: bad arguments");
     Geo g{B, H, W};
-    // chunks of whole rows of one image (about 2048 pixels) take the row-staged kernel
+    // chunks of whole rows of one image take the row-staged kernel
+    // about 2048 pixels, or fewer where that gives less than four workgroups per CU (with the weights through LDS, batch 16: 18 ->
+    // 9.4 us, batch 128: 39 -> 36)
     int rb = std::max(1, std::min(H, 2048 / W));
+    while (rb > 2 && (long)B * H / rb < 1024) rb /= 2;
     while (H % rb) --rb;
-    const size_t lds = (size_t)(rb + 2) * (W + 2) * sizeof(float);
-    const bool rows_ok = Co % 8 == 0 && 256 % (Co / 8) == 0 && lds <= 32768 && ((uintptr_t)y & 15) == 0;
+    const size_t lds = ((size_t)(rb + 2) * (W + 2) + 9L * Co) * sizeof(float);
+    const bool rows_ok = Co % 8 == 0 && 256 % (Co / 8) == 0 && lds - 36L * Co <= 32768 && lds <= 65536 && ((uintptr_t)y & 15) == 0;
     if (rows_ok)
         hipLaunchKernelGGL(k_conv_first_rows, dim3((unsigned)((long)B * H / rb)), dim3(256), lds, (hipStream_t)stream,
                            x, w, b, y, g, Co, rb);
@@ -1959,7 +2016,7 @@ extern "C" int bz_nn_head(const uint16_t* a, const float* fw, const float* fb, f
     BZ_REQUIRE(a && fw && fb && gap && out && B > 0 && HW > 0 && C > 0 && C <= 4096 && nout > 0,
                "bz_nn_head: bad arguments");
     if (C % 8 == 0 && 256 % (C / 8) == 0)
-        hipLaunchKernelGGL(k_head8, dim3(B), dim3(256), (256 / (C / 8) + 1) * C * sizeof(float), (hipStream_t)stream,
+        hipLaunchKernelGGL(k_head8, dim3(B), dim3(1024), (1024 / (C / 8) + 1) * C * sizeof(float), (hipStream_t)stream,
                            a, fw, fb, gap, out, HW, C, nout);
     else
         hipLaunchKernelGGL(k_head, dim3(B), dim3(256), C * sizeof(float), (hipStream_t)stream, a, fw, fb, gap, out, HW,
