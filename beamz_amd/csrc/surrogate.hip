@@ -1248,6 +1248,64 @@ __global__ __launch_bounds__(256) void k_conv_first_dgrad8(const uint16_t* __res
     gx[p] = s;
 }
 
+// The input gradient of the first convolution for Co = 32: gx[p] = sum_tap (gz . w[tap])[p - tap]. A workgroup owns RB
+// whole rows of one image. Its waves form the products T[q][tap] = sum_co gz[q][co] w[co][tap] of 16 pixels at a time
+// for the rows y0 - 1 .. y0 + RB with one 16x16x32 MFMA (A: pixels, its 8 channels per lane straight from memory; B:
+// the 9 taps in 16 columns) and leave them in LDS, [tap][RB + 2][W + 2] with zero edges; then each pixel adds its nine
+// taps in tap order. Reads gz once (and two rows per band again).
+// Bound by the read of gz; 256 x 128 x 128: 190 us with the products on the vector units, here 78.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void k_conv_first_dgrad32(const uint16_t* __restrict__ gz, const float* __restrict__ w,
+                                                            float* __restrict__ gx, Geo g, int RB) {
+    extern __shared__ float T[];
+    const int W = g.W, WP = W + 2, plane = (RB + 2) * WP | 1;      // odd: a wave's taps fall on different banks
+    const int row0 = blockIdx.x * RB, b = row0 / g.H, y0 = row0 - b * g.H;
+    const int t = threadIdx.x, l = t & 63, wave = t >> 6;
+    for (int q = t; q < 9 * plane; q += 256) T[q] = 0.0f;
+    // lane l: row (A) or column (B) l % 16, channels 8 (l / 16) .. + 7
+    const int col = l & 15, kg = 8 * (l >> 4);
+    uint16_t wb[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) wb[e] = col < 9 ? f2b(w[(kg + e) * 9 + col]) : (uint16_t)0;
+    const bf16x8 bw = __builtin_bit_cast(bf16x8, make_uint4(pack2(wb[0], wb[1]), pack2(wb[2], wb[3]), pack2(wb[4], wb[5]), pack2(wb[6], wb[7])));
+    __syncthreads();
+    const int ya = max(y0 - 1, 0), yb = min(y0 + RB, g.H - 1);       // the band's rows and those beside it
+    const int n = (yb - ya + 1) * W;
+    const uint16_t* src = gz + ((long)b * g.H + ya) * W * 32;
+    for (int p4 = wave * 64; p4 < n; p4 += 256) {                    // four loads in flight
+        bf16x8 a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            a[u] = __builtin_bit_cast(
+                bf16x8, *reinterpret_cast<const uint4*>(src + (long)min(p4 + 16 * u + col, n - 1) * 32 + kg));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bw, acc, 0, 0, 0);
+            // lane l holds pixels 4 (l / 16) + r of tap l % 16
+            const int q = p4 + 16 * u + 4 * (l >> 4);
+            int y = q / W, x = q - y * W;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (col < 9 && q + r < n) T[col * plane + (ya + y - y0 + 1) * WP + x + 1] = acc[r];
+                if (++x == W) {
+                    x = 0;
+                    ++y;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int q = t; q < RB * W; q += 256) {
+        const int y = q / W, x = q - y * W;
+        const float* c = T + (y + 1) * WP + x + 1;
+        float s = 0.0f;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) s += c[tap * plane - (tap / 3 - 1) * WP - (tap % 3 - 1)];
+        gx[((long)row0 + y) * W + x] = s;
+    }
+}
+
 // Column sums (bias gradient): gb[c] += sum_p g[p][c] over the workgroup's `chunk` pixel rows. Thread t
 // reads channels 8*(t % G) .. +7 (G = ceil(C/8) groups, 16-byte loads when C % 8 == 0) of every R-th row
 // (R = 256 / G), the R partial sums of each channel are added in LDS, and one atomic per channel and
@@ -1953,7 +2011,15 @@ extern "C" int bz_nn_conv_first_bwd(const uint16_t* x, const uint16_t* gz, const
     }
     BZ_CHECK_LAUNCH("bz_nn_conv_first_bwd(w)");
     if (gx) {
-        if (Co % 8 == 0 && Co <= 64 && ((uintptr_t)gz & 15) == 0)
+        // 32 channels, bands of up to 8 rows whose products leave room for three workgroups per CU (one row: up to 604
+        // pixels)
+        int rb = 8;
+        while (rb > 1 && (H % rb || 36L * (rb + 2) * (W + 2) > 49152)) --rb;
+        const size_t lds = 36L * ((long)(rb + 2) * (W + 2) | 1);
+        if (Co == 32 && lds <= 65536 && ((uintptr_t)gz & 15) == 0)
+            hipLaunchKernelGGL(k_conv_first_dgrad32, dim3((unsigned)((long)B * H / rb)), dim3(256), lds, st, gz, w, gx,
+                               g, rb);
+        else if (Co % 8 == 0 && Co <= 64 && ((uintptr_t)gz & 15) == 0)
             hipLaunchKernelGGL(k_conv_first_dgrad8, grid1(P), dim3(256), 0, st, gz, w, gx, g, Co);
         else
             hipLaunchKernelGGL(k_conv_first_dgrad, grid1(P), dim3(256), 0, st, gz, w, gx, g, Co);
