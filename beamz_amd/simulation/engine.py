@@ -200,7 +200,8 @@ class Grid:
     def add_point_source(self, comp, idx, w, mul, signal):
         """idx: (m, ndim) integer cell indices; w, mul: (m,) FP64 host arrays."""
         T = self.torch
-        off = np.array([self.offset(*(r if self.is_3d else (0, *r))) for r in idx], dtype=np.int64)
+        cells = np.asarray(idx, dtype=np.int64).reshape(-1, 3 if self.is_3d else 2).T
+        off = np.ascontiguousarray(self.offset(*(cells if self.is_3d else (0, *cells))))
         if len(np.unique(off)) != len(off):
             raise ValueError("point source offsets must be unique")
         src = _PointSource(comp, T.from_numpy(off).to(self.dev), T.from_numpy(np.asarray(w, np.float32)).to(self.dev),
@@ -246,12 +247,12 @@ class Grid:
         p.comp = T.from_numpy(np.asarray(comps, dtype=np.int32)).to(self.dev)
         p.off = T.from_numpy(np.asarray(offs, dtype=np.int64)).to(self.dev)
         p.record_steps = np.asarray(record_steps, dtype=np.int64)
-        p.slot = {int(s): q for q, s in enumerate(p.record_steps)}
+        p.slot = dict(zip(p.record_steps.tolist(), range(len(p.record_steps))))
         nrec = len(p.record_steps)
         p.series = T.zeros((max(nrec, 1), p.n), dtype=T.float32, device=self.dev) if keep_series else None
         p.nfreq = 0 if dft_omegas is None else len(dft_omegas)
         if p.nfreq:
-            ts = np.asarray([t_all[s] for s in p.record_steps], dtype=np.float64)
+            ts = np.asarray(t_all, dtype=np.float64)[p.record_steps]
             ph = np.exp(-1j * np.outer(ts, np.asarray(dft_omegas, dtype=np.float64)))   # (nrec, nfreq)
             p.phasor = T.from_numpy(np.ascontiguousarray(ph).view(np.float64)).to(self.dev)
             p.dft = T.zeros((p.nfreq, p.n, 2), dtype=T.float64, device=self.dev)
@@ -679,8 +680,15 @@ def kstep_owner_tables(tiles, pts, dims, K, rh):
     gy = np.maximum(1, -(-(nys - 2 * K) // iy))
     tx = np.where(anc, np.clip((i - K) // ix, 0, gx - 1), i // ix)
     ty = np.where(anc, np.clip((j - K) // iy, 0, gy - 1), j // iy)
-    index = {(int(a), int(b), int(c)): q for q, (a, (_, b, c)) in enumerate(zip(of, tiles)) if a >= 0}
-    t = np.array([index.get((int(a), int(b), int(c)), -1) for a, b, c in zip(sim, tx, ty)], np.int64)
+    have = np.nonzero(of >= 0)[0]
+    key = lambda a, b, c: (a * (1 << 20) + b) * (1 << 20) + c          # (a grid has fewer regions per axis)
+    keys = key(of[have], tiles[have, 1], tiles[have, 2])
+    srt = np.argsort(keys)
+    want = key(sim, tx, ty)
+    t = np.full(len(pts), -1, np.int64)
+    if len(have):
+        at = np.minimum(np.searchsorted(keys[srt], want), len(have) - 1)
+        t = np.where(keys[srt][at] == want, have[srt][at], -1)
     low = np.where(anc, 0, K)
     code = ((j - (ty * iy - low)) << 10) | ((i - (tx * ix - low)) << 2) | comp
     own = np.nonzero(t >= 0)[0]

@@ -271,12 +271,9 @@ class FDTD:
 
     # ---------------- setup ----------------
     def _time_table(self):
-        t = np.empty(self.num_steps + 1)
-        acc = 0
-        for n in range(self.num_steps + 1):
-            t[n] = acc
-            acc += self.dt
-        return t
+        t = np.full(self.num_steps + 1, self.dt, dtype=np.float64)     # added one by one, as the steps do
+        t[0] = 0.0
+        return np.add.accumulate(t)
 
     def _plan_sources(self):
         """Point sources of every design source on the real grid and, with complex fields, on the imaginary
@@ -332,17 +329,14 @@ class FDTD:
             pts = mon.get_grid_points_2d(self.dx, self.dy)
             # the second component (Hx, or Ex) is never written at column nx-1: a zero to read
             sentinel = (1, g.offset(0, 0, self.nx - 1))
+            x, y = np.asarray(pts, dtype=np.int64).reshape(-1, 2).T
             comps, offs = [], []
             for ci, name in enumerate(g.names):
                 sy, sx = shp[name]
-                for x, y in pts:
-                    if 0 <= y < sy and 0 <= x < sx:
-                        comps.append(ci)
-                        offs.append(g.offset(0, int(y), int(x)))
-                    else:
-                        comps.append(sentinel[0])
-                        offs.append(sentinel[1])
-            return comps, offs, ("line", len(pts))
+                ok = (0 <= y) & (y < sy) & (0 <= x) & (x < sx)
+                comps.append(np.where(ok, ci, sentinel[0]))
+                offs.append(np.where(ok, g.offset(0, y, x), sentinel[1]))
+            return np.concatenate(comps), np.concatenate(offs), ("line", len(pts))
         sl = mon.get_grid_slice_3d(self.dx, self.dy, self.dz)
         normal = mon.plane_normal
         regions = {}
@@ -381,9 +375,9 @@ class FDTD:
                 o = (a * self.ny + fixed) * g.ld + b
             else:
                 o = (a * self.ny + b) * g.ld + fixed
-            comps += [ci] * o.size
-            offs += o.ravel().tolist()
-        return comps, offs, ("plane", (m0, m1))
+            comps.append(np.full(o.size, ci))
+            offs.append(o.ravel())
+        return np.concatenate(comps), np.concatenate(offs), ("plane", (m0, m1))
 
     def _plan_monitors(self, t_all):
         g = self.grid
@@ -396,12 +390,15 @@ class FDTD:
                 mon._fields = {k: [] for k in g.names}
                 mon._fields["t"] = []
             comps, offs, layout = self._monitor_samples(mon)
-            last = mon.last_record_step
-            steps = []
-            for n in range(self.num_steps):
-                if n - last >= mon.record_interval:
-                    steps.append(n)
-                    last = n
+            last, every = mon.last_record_step, mon.record_interval
+            if isinstance(every, (int, np.integer)):
+                steps = np.arange(max(0, last + every), self.num_steps, max(1, every))
+            else:
+                steps = []
+                for n in range(self.num_steps):
+                    if n - last >= every:
+                        steps.append(n)
+                        last = n
             omegas = None if mon.dft_frequencies is None else 2 * np.pi * mon.dft_frequencies
             keep = bool(mon.should_record_fields or mon.accumulate_power)
             plan = g.add_gather(comps, offs, steps, t_all, omegas, keep_series=keep)
@@ -421,7 +418,7 @@ class FDTD:
     def _materialize(self, plan):
         """Copy a monitor's device samples into the reference's host structures."""
         mon = plan.monitor
-        done = [s for s in plan.record_steps if s < self.current_step]
+        done = plan.record_steps[plan.record_steps < self.current_step]
         nrec = len(done)
         new = slice(plan.fetched, nrec)
         names = self.grid.names
@@ -487,6 +484,14 @@ class FDTD:
         if self.current_step < self.num_steps:
             mon._pull = self._make_pull(plan)
 
+    def _eps_max(self):
+        """np.max(self.epsilon_r), by all host threads for a large real array."""
+        e = self.epsilon_r
+        if (isinstance(e, np.ndarray) and e.size >= 1 << 20 and e.dtype in (np.float32, np.float64) and
+                e.flags.c_contiguous and e.flags.writeable and e.dtype.isnative):
+            return self.backend.torch.from_numpy(e).max().numpy()
+        return np.max(e)
+
     def initialize_simulation(self, save=True, live=True, axis_scale=[-1, 1], save_animation=False,
                               animation_filename="fdtd_animation.mp4", clean_visualization=True, save_fields=None,
                               decimate_save=1, accumulate_power=False, save_memory_mode=False,
@@ -508,7 +513,7 @@ class FDTD:
             self.results[k] = []
         self.save_memory_mode = save_memory_mode
         self.accumulate_power = accumulate_power
-        n_max = np.sqrt(np.max(self.epsilon_r))
+        n_max = np.sqrt(self._eps_max())
         ok, courant, lim = check_fdtd_stability(dt=self.dt, dx=self.dx, dy=self.dy, n_max=n_max, safety_factor=1.0)
         if not ok:
             display_status(f"Simulation may be unstable! Courant number = {courant:.3f} > {lim:.3f}", "warning")
@@ -584,7 +589,7 @@ class FDTD:
         end = min(self.num_steps, self.current_step + count)
         while self.current_step < end:
             n = self.current_step
-            stop = n + 1
+            stop = n + 1 if self._save_results else end
             if not self._needs_host(n):
                 while stop < end and not self._needs_host(stop):
                     stop += 1
