@@ -103,18 +103,19 @@ __device__ __forceinline__ float box_amp(const bz_sim2d& S, long rr, int n, floa
 //   Hx' = fa Hx - gb (Ez[i+1] - Ez)            (= fa Hx - fb dEz/dy)
 //   Hy' = fa Hy + gb r (Ez[j+1] - Ez)          (= fa Hy + fb dEz/dx)
 //   Ez' = ca Ez + gc (r (Hy - Hy[j-1]) - (Hx - Hx[i-1]))
-// The curl term is the multiply of the last fused multiply-add and the field's own product is rounded before
-// it: where fa = ca = 1 (no conductivity) that product is the field itself, so the K-step kernel leaves it out
-// there (8 vector operations per cell and step instead of 11) and still gives these bits.
+// The field's own term is the multiply of the last fused multiply-add: where fa = ca = 1 (no conductivity) that is an
+// addition, so the K-step kernel needs one coefficient per cell there and still gives these bits. Fusing the curl term
+// instead (8 vector operations per cell and step there, not 11) moves a spectrum's error against 64 bits either way
+// by its own size, and is not used.
 __device__ __forceinline__ float upd_hx(float fa, float gb, float hx, float ezR, float ez) {
-    return fmaf(-gb, ezR - ez, fa * hx);
+    return fmaf(fa, hx, -(gb * (ezR - ez)));
 }
 __device__ __forceinline__ float upd_hy(float fa, float gb, float r, float hy, float ed, float ez) {
-    return fmaf(gb, r * (ed - ez), fa * hy);
+    return fmaf(fa, hy, gb * (r * (ed - ez)));
 }
 __device__ __forceinline__ float upd_ez(float ca, float gc, float r, float ez, float hx, float hxl, float hy,
                                         float hu) {
-    return fmaf(gc, fmaf(r, hy - hu, -(hx - hxl)), ca * ez);
+    return fmaf(ca, ez, gc * fmaf(r, hy - hu, -(hx - hxl)));
 }
 
 // The (Hz, Ex, Ey) updates, likewise one arithmetic for its two kernels:
@@ -948,14 +949,14 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                         }
                     }
                 } else {
-                    hyg = L ? upd_hy(fag, gbg, E == 2 ? rxy : 1.0f, hyg, ez[0], ezg) : fmaf(gb0, ez[0] - ezg, hyg);
+                    hyg = L ? upd_hy(fag, gbg, E == 2 ? rxy : 1.0f, hyg, ez[0], ezg) : hyg + gb0 * (ez[0] - ezg);
 #pragma unroll
                     for (int r = 0; r < B; ++r) {
                         const float ezR = from_right(ez[r]);
                         const float ed = r < B - 1 ? ez[r + 1] : ezb;
                         if (!L) {
-                            hx[r] = fmaf(-gb0, ezR - ez[r], hx[r]);
-                            hy[r] = fmaf(gb0, ed - ez[r], hy[r]);
+                            hx[r] -= gb0 * (ezR - ez[r]);
+                            hy[r] += gb0 * (ed - ez[r]);
                         } else {
                             const float hn = computed(upd_hx(fa[r], gb[r], hx[r], ezR, ez[r]));
                             hx[r] = E == 0 || hxok ? hn : hx[r];
@@ -1009,7 +1010,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                         const float hxl = from_left(hx[r]);
                         const float hu = r > 0 ? hy[r - 1] : hyg;
                         if (!L) {
-                            ez[r] = fmaf(gc[r], (hy[r] - hu) - (hx[r] - hxl), ez[r]);
+                            ez[r] += gc[r] * ((hy[r] - hu) - (hx[r] - hxl));
                         } else if (E < 2 || (jb + r >= 1 && jb + r <= ny - 2)) {
                             const float en =
                                 computed(upd_ez(ca[r], gcl[r], E == 2 ? rxy : 1.0f, ez[r], hx[r], hxl, hy[r], hu));
