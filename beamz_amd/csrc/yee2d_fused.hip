@@ -118,18 +118,18 @@ __device__ __forceinline__ float upd_ez(float ca, float gc, float r, float ez, f
     return fmaf(ca, ez, gc * fmaf(r, hy - hu, -(hx - hxl)));
 }
 
-// The (Hz, Ex, Ey) updates, likewise one arithmetic for its two kernels:
-//   Hz' = fa Hz - gb (r (Ey[i+1] - Ey) - (Ex[j+1] - Ex)),  Ex' = ca Ex + gc (Hz - Hz[j-1]),
-//   Ey' = ca Ey - gc r (Hz - Hz[i-1])
-__device__ __forceinline__ float upd_hz(float fa, float gb, float r, float hz, float eyR, float ey, float exN,
-                                        float ex) {
-    return fmaf(-gb, fmaf(r, eyR - ey, -(exN - ex)), fa * hz);
+// The (Hz, Ex, Ey) updates, likewise one arithmetic for its two kernels (no term folded or fused: the rounding its
+// one-step kernel always had):
+//   Hz' = fa Hz - fb (dEy/dx - dEx/dy),  Ex' = ca Ex + cb dHz/dy,  Ey' = ca Ey - cb dHz/dx
+__device__ __forceinline__ float upd_hz(float fa, float fb, float rdx, float rdy, float hz, float eyR, float ey,
+                                        float exN, float ex) {
+    return fa * hz - fb * ((eyR - ey) * rdx - (exN - ex) * rdy);
 }
-__device__ __forceinline__ float upd_ex(float ca, float gc, float ex, float hz, float hzU) {
-    return fmaf(gc, hz - hzU, ca * ex);
+__device__ __forceinline__ float upd_ex(float ca, float cb, float rdy, float ex, float hz, float hzU) {
+    return ca * ex + cb * ((hz - hzU) * rdy);
 }
-__device__ __forceinline__ float upd_ey(float ca, float gc, float r, float ey, float hz, float hzL) {
-    return fmaf(-gc, r * (hz - hzL), ca * ey);
+__device__ __forceinline__ float upd_ey(float ca, float cb, float rdx, float ey, float hz, float hzL) {
+    return ca * ey - cb * ((hz - hzL) * rdx);
 }
 
 // Monitor sample p of step n, read from the buffer step n wrote.
@@ -304,7 +304,6 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
     c.ke = S.ke;
     c.kbe = S.kbe;
     const float rdx = S.rdx, rdy = S.rdy;
-    const float rxy = rdx / rdy;   // 1 on square cells
     const uint32_t ic = (uint32_t)min(max(i, 0), nx - 1);
     // register row r = row j0-1+r, clamped into the grid
     uint32_t ro[SEG + 2];
@@ -333,7 +332,7 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
         float fa, fb;
         h_coef(sg[r], c, fa, fb);
         const float eyR = __shfl_down(ey[r], 1, LANES);
-        hzn[r] = (hzx && j < ny - 1) ? upd_hz(fa, fb * rdy, rxy, hz[r], eyR, ey[r], ex[r + 1], ex[r]) : hz[r];
+        hzn[r] = (hzx && j < ny - 1) ? upd_hz(fa, fb, rdx, rdy, hz[r], eyR, ey[r], ex[r + 1], ex[r]) : hz[r];
         hzl[r] = __shfl_up(hzn[r], 1, LANES);
     }
     // Ex, Ey of rows j0 .. j0+SEG-1, the source on Hz, stores
@@ -348,9 +347,8 @@ __global__ __launch_bounds__(LANES* WPG) void k_yee2d_hz(const bz_sim2d* __restr
         if (out && j < ny) {
             float ca, cb;
             e_coef(sg[r], ee[r], c, ca, cb);
-            const float gc = cb * rdy;
-            const float exn = (j >= 1 && j <= ny - 2 && hzx) ? upd_ex(ca, gc, ex[r], hzn[r], hzn[r - 1]) : ex[r];
-            const float eyn = (j <= ny - 2 && i >= 1 && i <= nx - 2) ? upd_ey(ca, gc, rxy, ey[r], hzn[r], hzl[r]) : ey[r];
+            const float exn = (j >= 1 && j <= ny - 2 && hzx) ? upd_ex(ca, cb, rdy, ex[r], hzn[r], hzn[r - 1]) : ex[r];
+            const float eyn = (j <= ny - 2 && i >= 1 && i <= nx - 2) ? upd_ey(ca, cb, rdx, ey[r], hzn[r], hzl[r]) : ey[r];
             float hzo = hzn[r];
             const int a = i - S.src_x0, b = j - S.src_y0;
             if (a >= 0 && a < S.src_sx && b >= 0 && b < S.src_sy) {
@@ -706,10 +704,10 @@ constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further 
 // source lookup is compiled out.
 // What bounds it: on many grids the load phase of a region beside vector issue (8 waves x 8 rows in 80 registers
 // let three workgroups of a CU overlap those; with 128 registers it was two), on one small grid the chain of a
-// step (LDS round trip, barrier, six dependent operations) and the launch itself. Measured, with 4-value
-// coefficients, two barriers per step, unanchored regions and 128 registers before: 64 grids of 256 x 256 cells
-// 7.3 -> 4.95 us/step, 16 grids of 600 x 600 cells 8.6 -> 5.8, twelve of 256..1024 a side 6.3 -> 4.5, one grid of
-// 800 x 400 cells with a 16-frequency line 1.33 (K = 12) -> 1.09 (K = 16).
+// step (LDS round trip, barrier, eight dependent operations) and the launch itself. Measured, whole calls, with
+// 4-value coefficients, two barriers per step, unanchored regions and 128 registers before: 64 grids of 256 x 256
+// cells 15.6 -> 10.7 ms, twelve of 256..1024 a side 4.6 -> 3.2 ms; one grid of 800 x 400 cells with a 16-frequency
+// line 1.33 (K = 12) -> 1.1 us/step (K = 16). HZ, 701 x 403 cells, 1500 steps: 10.0 ms at one step per launch, 3.1.
 // HZ: the (Hz, Ex, Ey) polarisation in the slots of (Ez, Hx, Hy). Its H update reads Ex of the next row and Ey of
 // the next column, its E update Hz of the previous row and column: the bands exchange Ex of the first row and Ex,
 // Ey of the last, and each keeps the Hz of the row above (with its source, which this family adds to Hz).
@@ -756,7 +754,8 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
     const int n0 = *step + K * q;
     const float rdy = S.rdy;
     // 1 on square cells; uniform, so kept in a scalar register
-    const float rxy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(S.rdx / rdy)));
+    const float rdx = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(S.rdx)));
+    const float rxy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(rdx / rdy)));
     const bool hxok = i < nx - 1;
     const bool xin = i >= 1 && i <= nx - 2;
     const bool lane_out = l >= cx0 && l < cx1 && i < nx;
@@ -811,7 +810,8 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
 
     // the fields, Hy (HZ: Hz) of the row above the band (hyg), and gc = cb * rdy of cells without conductivity
     float ez[B], hx[B], hy[B], gc[B], hyg = 0.0f;
-    const float gb0 = S.kbh * rdy;                  // gb = fb * rdy of such a cell
+    const float ry = HZ ? 1.0f : rdy;               // what the coefficients carry (HZ: fb and cb themselves)
+    const float gb0 = S.kbh * ry;                   // gb = fb * rdy of such a cell
     bool lossy = true;
 #pragma unroll
     for (int r = 0; r < B; ++r) ez[r] = hx[r] = hy[r] = gc[r] = 0.0f;
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
 #pragma unroll
             for (int r = 0; r < B; ++r) {
                 m = fminf(m, gc[r]);
-                gc[r] *= rdy;
+                gc[r] *= ry;
             }
             lossy = __ballot(m < 0.0f) != 0;
         }
@@ -858,14 +858,14 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                 // precomputed by k_coef2d (the same roundings), one 16-byte (fa, fb, ca, cb) per cell
                 const float4 g4 = at4(cf, 4u * off(jb - 1));
                 fag = g4.x;
-                gbg = g4.y * rdy;
+                gbg = g4.y * ry;
 #pragma unroll
                 for (int r = 0; r < B; ++r) {
                     const float4 v = at4(cf, 4u * off(jb + r));
                     fa[r] = v.x;
-                    gb[r] = v.y * rdy;
+                    gb[r] = v.y * ry;
                     ca[r] = v.z;
-                    gcl[r] = v.w * rdy;
+                    gcl[r] = v.w * ry;
                 }
             } else {
                 Coef c;
@@ -882,12 +882,12 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                     e_coef(sg, at(S.eps, off(jb + r)), c, d, e);
                     if (r < 0) {
                         fag = a;
-                        gbg = b * rdy;
+                        gbg = b * ry;
                     } else {
                         fa[r] = a;
-                        gb[r] = b * rdy;
+                        gb[r] = b * ry;
                         ca[r] = d;
-                        gcl[r] = e * rdy;
+                        gcl[r] = e * ry;
                     }
                 }
             }
@@ -933,18 +933,17 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                 if (plain_src && B <= 4) src_adds(0);
                 // H: the row above the band (its Hy, or Hz, only), then the band
                 if (HZ) {
-                    const float r1 = E == 2 ? rxy : 1.0f;
-                    const float hg = computed(L ? upd_hz(fag, gbg, r1, hyg, from_right(eyg), eyg, hx[0], ezg)
-                                                : fmaf(-gb0, (from_right(eyg) - eyg) - (hx[0] - ezg), hyg));
+                    const float hg = computed(upd_hz(L ? fag : 1.0f, L ? gbg : gb0, rdx, rdy, hyg, from_right(eyg), eyg,
+                                                     hx[0], ezg));
                     hyg = E == 0 || (hxok && (E < 2 || (jb >= 1 && jb <= ny - 1))) ? hg : hyg;
 #pragma unroll
                     for (int r = 0; r < B; ++r) {
                         const float eyR = from_right(hy[r]);
                         const float exN = r < B - 1 ? hx[r + 1] : ezb;
                         if (!L) {
-                            ez[r] = fmaf(-gb0, (eyR - hy[r]) - (exN - hx[r]), ez[r]);
+                            ez[r] = upd_hz(1.0f, gb0, rdx, rdy, ez[r], eyR, hy[r], exN, hx[r]);
                         } else {
-                            const float hn = computed(upd_hz(fa[r], gb[r], r1, ez[r], eyR, hy[r], exN, hx[r]));
+                            const float hn = computed(upd_hz(fa[r], gb[r], rdx, rdy, ez[r], eyR, hy[r], exN, hx[r]));
                             ez[r] = E == 0 || (hxok && (E < 2 || jb + r < ny - 1)) ? hn : ez[r];
                         }
                     }
@@ -989,17 +988,16 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                 }
                 // E
                 if (HZ) {
-                    const float r1 = E == 2 ? rxy : 1.0f;
 #pragma unroll
                     for (int r = 0; r < B; ++r) {
                         const float hzL = from_left(ez[r]);
                         const float hzU = r > 0 ? ez[r - 1] : hyg;
                         if (!L) {
-                            hx[r] = fmaf(gc[r], ez[r] - hzU, hx[r]);
-                            hy[r] = fmaf(-gc[r], ez[r] - hzL, hy[r]);
+                            hx[r] = upd_ex(1.0f, gc[r], rdy, hx[r], ez[r], hzU);
+                            hy[r] = upd_ey(1.0f, gc[r], rdx, hy[r], ez[r], hzL);
                         } else {
-                            const float xn = computed(upd_ex(ca[r], gcl[r], hx[r], ez[r], hzU));
-                            const float yn = computed(upd_ey(ca[r], gcl[r], r1, hy[r], ez[r], hzL));
+                            const float xn = computed(upd_ex(ca[r], gcl[r], rdy, hx[r], ez[r], hzU));
+                            const float yn = computed(upd_ey(ca[r], gcl[r], rdx, hy[r], ez[r], hzL));
                             hx[r] = E == 0 || (hxok && (E < 2 || (jb + r >= 1 && jb + r <= ny - 2))) ? xn : hx[r];
                             hy[r] = E == 0 || (xin && (E < 2 || jb + r <= ny - 2)) ? yn : hy[r];
                         }
