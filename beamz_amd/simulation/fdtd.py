@@ -131,6 +131,19 @@ def mode_source_cells(src, dx, dy, dz, nx, ny, nz, ez_nz, is_3d):
     return idx, mul, add
 
 
+def record_steps(last, every, num_steps):
+    """The steps a monitor records: each n with n - last >= every, which then is last."""
+    if isinstance(every, (int, np.integer)) and isinstance(last, (int, np.integer)):
+        last, every = int(last), int(every)          # (a NumPy integer's width would bound their sum)
+        return np.arange(max(0, last + every), num_steps, max(1, every))
+    steps = []
+    for n in range(num_steps):
+        if n - last >= every:
+            steps.append(n)
+            last = n
+    return steps
+
+
 class FDTD:
     def __init__(self, design, time, mesh: str = "regular", resolution: float = 0.02e-6, backend="hip",
                  backend_options=None, devices=None, *, polarization="Ez", complex_fields=None):
@@ -390,15 +403,7 @@ class FDTD:
                 mon._fields = {k: [] for k in g.names}
                 mon._fields["t"] = []
             comps, offs, layout = self._monitor_samples(mon)
-            last, every = mon.last_record_step, mon.record_interval
-            if isinstance(every, (int, np.integer)):
-                steps = np.arange(max(0, last + every), self.num_steps, max(1, every))
-            else:
-                steps = []
-                for n in range(self.num_steps):
-                    if n - last >= every:
-                        steps.append(n)
-                        last = n
+            steps = record_steps(mon.last_record_step, mon.record_interval, self.num_steps)
             omegas = None if mon.dft_frequencies is None else 2 * np.pi * mon.dft_frequencies
             keep = bool(mon.should_record_fields or mon.accumulate_power)
             plan = g.add_gather(comps, offs, steps, t_all, omegas, keep_series=keep)
