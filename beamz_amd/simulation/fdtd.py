@@ -144,6 +144,14 @@ def record_steps(last, every, num_steps):
     return steps
 
 
+def time_table(dt, num_steps):
+    """The times of steps 0 .. num_steps: dt added one by one in its own type, as the steps add it (so a time axis
+    in 32 bits gives the times it always gave)."""
+    t = np.full(num_steps + 1, dt)
+    t[0] = 0
+    return np.add.accumulate(t, dtype=t.dtype).astype(np.float64)
+
+
 class FDTD:
     def __init__(self, design, time, mesh: str = "regular", resolution: float = 0.02e-6, backend="hip",
                  backend_options=None, devices=None, *, polarization="Ez", complex_fields=None):
@@ -284,9 +292,7 @@ class FDTD:
 
     # ---------------- setup ----------------
     def _time_table(self):
-        t = np.full(self.num_steps + 1, self.dt, dtype=np.float64)     # added one by one, as the steps do
-        t[0] = 0.0
-        return np.add.accumulate(t)
+        return time_table(self.dt, self.num_steps)
 
     def _plan_sources(self):
         """Point sources of every design source on the real grid and, with complex fields, on the imaginary
