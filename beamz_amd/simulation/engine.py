@@ -412,11 +412,12 @@ class Grid:
                 self._fused3d_triple(n)
                 n += 3
             elif end - n >= 2 and self.tb2 and self._pair_ok():
-                if self.timing or self.tb3:       # launches timed (or mixed with three-step ones) one by one
+                # the pairs that every source has samples for (without one: _fused3d_pair raises at the sample)
+                npairs = (min([end] + [len(s.signal) for s in self.sources]) - n) // 2
+                if self.timing or self.tb3 or npairs < 1:     # (timed, or mixed with three-step launches)
                     self._fused3d_pair(n)
                     n += 2
                 else:
-                    npairs = (end - n) // 2
                     self._fused3d_pairs(n, npairs)
                     n += 2 * npairs
             else:
@@ -511,13 +512,12 @@ class Grid:
                 "base": N.ptrs6([buf.data_ptr() + 4 * q * cells for q in range(6)])}
 
     def _fused3d_pairs(self, n, npairs):
-        """Steps n .. n + 2 npairs - 1 as pairs, every launch and its monitor samples from one call."""
+        """Steps n .. n + 2 npairs - 1 (within every source's signal) as pairs, every launch and its monitor samples
+        from one call."""
         steps, nb = 2 * npairs, len(self.sources)
         arr = (N.BoxSource * N.MAX_BOX)(*[s.box[0] for s in self.sources])
         amps = np.ascontiguousarray(np.stack([np.real(s.signal[n:n + steps]) for s in self.sources], axis=1)
                                     if nb else np.zeros((steps, 0)), dtype=np.float32)
-        if len(amps) < steps:
-            raise IndexError(f"steps {n}..{n + steps - 1} run past a source signal")
         stg = self._stage
         tables, rows = [], []
         for t in stg["plans"]:
