@@ -39,3 +39,34 @@ def test_runs_within_the_signals_take_every_step(grid):
         grid.add_point_source("Ez", np.array([[2, 3, 2 + q]]), np.ones(1), None, np.arange(n, dtype=float))
     grid.run(0, 10)
     assert steps_done(grid) == 10 and [c[0] for c in grid.calls] == ["bz_yee3d_run2"]
+
+
+def test_one_pair_goes_without_the_tables_of_a_run(grid):
+    """A run of two steps is one launch and one gather per table, and not the set-up of a whole run's tables."""
+    grid.add_gather([0, 1], [11, 12], np.arange(400), np.arange(401.0), [1.0], keep_series=False)
+    grid.add_gather([2], [13], np.arange(1, 400, 2), np.arange(401.0), [1.0], keep_series=False)
+    grid.run(6, 2)
+    assert [c[0] for c in grid.calls] == ["bz_yee3d_step2", "bz_gather2", "bz_gather2"]
+
+
+@pytest.mark.parametrize("n,steps", [(0, 400), (0, 4), (6, 6), (390, 10), (100, 48)])
+def test_rows_of_a_run_are_the_recorded_steps(grid, n, steps):
+    """The rows handed to the native call, for runs that look steps up and runs that scan the records."""
+    records = [np.arange(400), np.arange(2, 400, 5), np.array([5])]
+    for rec in records:
+        grid.add_gather([0], [11], rec, np.arange(401.0), [1.0], keep_series=False)
+    rows = {}
+
+    def call(name, *a):
+        assert name == "bz_yee3d_run2"
+        for t in range(a[21]):
+            rows[a[20][t].comp] = np.ctypeslib.as_array((N.C.c_int * steps).from_address(a[20][t].row)).copy()
+    N.call = call
+    grid.run(n, steps)
+    want = {}
+    for p, rec in zip(grid.monitors, records):
+        at = {int(s): q for q, s in enumerate(rec)}
+        row = [at.get(s, -1) for s in range(n, n + steps)]
+        if max(row) >= 0:
+            want[p.comp.data_ptr()] = row
+    assert {k: list(v) for k, v in rows.items()} == want
