@@ -571,13 +571,15 @@ extern "C" int bz_yee3d_run2(float* const src[6], float* const dst[6], const flo
     const float rx = (float)(1.0 / dx), ry = (float)(1.0 / dy), rz = (float)(1.0 / dz);
     const hipStream_t st = (hipStream_t)stream;
     const long cells = (long)stg.sx * stg.sy * stg.sz;
-    // table t's arguments for pair q: its first step's samples in staging slot q & 1
+    const bool fused = ntables == 1;
+    auto slot = [&](int q) { return fused ? q & 1 : 0; };
+    // table t's arguments for pair q: its first step's samples in staging slot `slot(q)`
     auto of_pair = [&](int t, int q) {
         const bz_gather_table& g = tables[t];
         Gather3D G{};
         const int r0 = g.row[2 * q], r1 = g.row[2 * q + 1];
         if (r0 < 0 && r1 < 0) return G;
-        for (int k = 0; k < 6; ++k) G.base0[k] = stage + (6 * (q & 1) + k) * cells;
+        for (int k = 0; k < 6; ++k) G.base0[k] = stage + (6 * slot(q) + k) * cells;
         G.comp = g.comp;
         G.off0 = g.stage_off;
         G.off1 = g.off;
@@ -602,7 +604,6 @@ extern "C" int bz_yee3d_run2(float* const src[6], float* const dst[6], const flo
     // One call, since a pair on a small grid is shorter than its two Python calls were (33 us at 120x72x40; now 20 per
     // pair with the samples). With one table, pair q - 1's samples are taken by extra workgroups of pair q's launch: its first step sits in
     // the staging slot that launch does not write, its second step in the buffer that launch only reads
-    const bool fused = ntables == 1;
     for (int q = 0; q < npairs; ++q) {
         for (int k = 0; k < nbox; ++k) {
             bs.b[k].amp = amps[(long)2 * q * nbox + k];
@@ -611,7 +612,7 @@ extern "C" int bz_yee3d_run2(float* const src[6], float* const dst[6], const flo
         bool need = false;
         for (int t = 0; t < ntables; ++t) need = need || tables[t].row[2 * q] >= 0;
         Stage sq = stg;
-        sq.p = need ? stage + 6 * (q & 1) * cells : nullptr;
+        sq.p = need ? stage + 6 * slot(q) * cells : nullptr;
         const Fields6 &S = F[q & 1], &D = F[(q & 1) ^ 1];
         const int e = launch_pair(S, D, eps_r, sigma, nx, ny, nz, ld, kseg, rows, waves, c, rx, ry, rz, bs, sq,
                                   fused && q > 0 ? of_pair(0, q - 1) : Gather3D{}, st);

@@ -504,14 +504,24 @@ class Grid:
         cells = sx * sy * sz
         if cells > max_cells:
             return False
-        buf = T.zeros(12 * cells, dtype=T.float32, device=self.dev)     # two slots (bz_yee3d_run2)
         for p in plans:
             o = p.off.cpu().numpy()
             pk, pr = o // plane, o % plane
             pj, pi = pr // self.ld, pr % self.ld
             p.stage_off = T.from_numpy(((pk - z0) * sy + (pj - y0)) * sx + (pi - x0)).to(self.dev)
-        return {"plans": plans, "buf": buf, "box": (C.c_int * 6)(x0, y0, z0, sx, sy, sz),
-                "base": N.ptrs6([buf.data_ptr() + 4 * q * cells for q in range(6)])}
+        return {"plans": plans, "box": (C.c_int * 6)(x0, y0, z0, sx, sy, sz), "cells": cells, "slots": 0, "used": []}
+
+    def _stage_slots(self, slots):
+        """The staging box with at least `slots` slots, allocated when a call first needs them (up to 201 MB each):
+        two for three-step launches and for a run of pairs whose samples the next launch takes, else one."""
+        stg = self._stage
+        if stg["plans"] and stg["slots"] < slots:
+            cells = stg["cells"]
+            buf = self.torch.zeros(6 * slots * cells, dtype=self.torch.float32, device=self.dev)
+            stg["used"].append(buf)               # launches that are still queued may use a smaller one
+            base = [N.ptrs6([buf.data_ptr() + 4 * (6 * k + q) * cells for q in range(6)]) for k in range(slots)]
+            stg.update(slots=slots, buf=buf, base=base[0], base2=base[-1])
+        return stg
 
     def _fused3d_pairs(self, n, npairs):
         """Steps n .. n + 2 npairs - 1 (within every source's signal) as pairs, every launch and its monitor samples
@@ -520,9 +530,8 @@ class Grid:
         arr = (N.BoxSource * N.MAX_BOX)(*[s.box[0] for s in self.sources])
         amps = np.ascontiguousarray(np.stack([np.real(s.signal[n:n + steps]) for s in self.sources], axis=1)
                                     if nb else np.zeros((steps, 0)), dtype=np.float32)
-        stg = self._stage
         tables, rows = [], []
-        for t in stg["plans"]:
+        for t in self._stage["plans"]:
             row = np.full(steps, -1, np.int32)
             if 8 * steps < len(t.record_steps):      # a few steps of a long run: looked up, no pass over all records
                 row[:] = [t.slot.get(s, -1) for s in range(n, n + steps)]
@@ -535,6 +544,7 @@ class Grid:
             ptr = lambda x: x.data_ptr() if x is not None else None
             tables.append(N.GatherTable(t.comp.data_ptr(), t.stage_off.data_ptr(), t.off.data_ptr(), t.n,
                                         row.ctypes.data, ptr(t.series), t.nfreq, ptr(t.phasor), ptr(t.dft)))
+        stg = self._stage_slots(2 if len(tables) == 1 else 1) if tables else None
         src, dst = self._fb[self._cur], self._fb[1 - self._cur]
         N.call("bz_yee3d_run2", N.ptrs6([src[k].data_ptr() for k in COMP3]), N.ptrs6([dst[k].data_ptr() for k in COMP3]),
                self.eps.data_ptr(), self.sig.data_ptr(), self.nx, self.ny, self.nz, self.ld, self.dx, self.dy, self.dz,
@@ -552,7 +562,7 @@ class Grid:
             b.amp = float(np.real(s.signal[n]))
             arr[q] = b
             amp1[q] = float(np.real(s.signal[n + 1]))
-        stg = self._stage
+        stg = self._stage_slots(1)
         need = any(p.slot.get(n) is not None for p in stg["plans"])
         src, dst = self._fb[self._cur], self._fb[1 - self._cur]
         ps = N.ptrs6([src[k].data_ptr() for k in COMP3])
@@ -592,11 +602,7 @@ class Grid:
             arr[q] = b
             amp1[q] = float(np.real(s.signal[n + 1]))
             amp2[q] = float(np.real(s.signal[n + 2]))
-        stg = self._stage
-        if stg["plans"] and "buf2" not in stg:
-            cells = stg["buf"].numel() // 12
-            stg["buf2"] = stg["buf"][6 * cells:]
-            stg["base2"] = N.ptrs6([stg["buf2"].data_ptr() + 4 * q * cells for q in range(6)])
+        stg = self._stage_slots(2)
         need1 = any(p.slot.get(n) is not None for p in stg["plans"])
         need2 = any(p.slot.get(n + 1) is not None for p in stg["plans"])
         src, dst = self._fb[self._cur], self._fb[1 - self._cur]
@@ -608,7 +614,7 @@ class Grid:
             e0.record()
         N.call("bz_yee3d_step3", ps, pd, self.eps.data_ptr(), self.sig.data_ptr(), self.nx, self.ny, self.nz,
                self.ld, self.dx, self.dy, self.dz, self.dt, MU_0, EPS_0, arr, amp1, amp2, len(self.sources),
-               stg["buf"].data_ptr() if need1 else None, stg["buf2"].data_ptr() if need2 else None,
+               stg["buf"].data_ptr() if need1 else None, stg["base2"][0] if need2 else None,
                stg["box"] if (need1 or need2) else None, self.kseg3_eff(), self.rows3, self.waves3, st)
         if self.timing:
             e1.record()

@@ -133,8 +133,9 @@ typedef struct bz_gather_table {
 
 /* npairs bz_yee3d_step2 passes with their monitor samples (bz_gather2), the same bits, from one call: pair q reads src
  * and writes dst for even q and the other way round for odd q. amps (host): [2 * npairs][nbox] source amplitudes of
- * the steps (boxes[q].amp is not read). stage: 2 slots of 6 * sx * sy * sz floats (pair q writes slot q & 1). With
- * one table, a pair's samples are taken by extra workgroups of the next pair's launch. */
+ * the steps (boxes[q].amp is not read). With one table, a pair's samples are taken by extra workgroups of the next
+ * pair's launch, and stage holds 2 slots of 6 * sx * sy * sz floats (pair q writes slot q & 1); with several, each
+ * pair's are taken before the next pair, from one slot. */
 int bz_yee3d_run2(float* const src[6], float* const dst[6], const float* eps_r, const float* sigma, int nx, int ny,
                   int nz, int ld, double dx, double dy, double dz, double dt, double mu0, double eps0,
                   const bz_box_source* boxes, const float* amps, int nbox, int npairs, float* stage,

@@ -14,7 +14,7 @@ def grid(monkeypatch):
     import torch
     g = Grid(SimpleNamespace(torch=torch, dev="cpu", stream=None), np.ones((8, 9, 10)), np.zeros((8, 9, 10)), 1.0, 1.0, 0.1,
              1.0)
-    g.kseg2, g.calls = 8, []
+    g.kseg2, g.kseg3, g.calls = 8, 8, []
     monkeypatch.setattr(N, "call", lambda name, *a: g.calls.append((name, a)))
     return g
 
@@ -70,3 +70,25 @@ def test_rows_of_a_run_are_the_recorded_steps(grid, n, steps):
         if max(row) >= 0:
             want[p.comp.data_ptr()] = row
     assert {k: list(v) for k, v in rows.items()} == want
+
+
+def test_the_staging_box_has_a_second_slot_only_for_calls_that_use_it(grid):
+    """One slot for single pairs and for several tables (each pair's samples are taken before the next pair); the run
+    of pairs with one table, and three-step launches, add the second."""
+    grid.add_gather([0, 1], [11, 500], np.arange(40), np.arange(41.0), [1.0], keep_series=False)
+    grid.run(0, 2)
+    one = grid._stage["buf"].numel()
+    box = list(grid._stage["box"])
+    assert one == 6 * box[3] * box[4] * box[5]
+    grid.run(2, 8)
+    assert grid._stage["buf"].numel() == 2 * one
+    assert grid.calls[-1][1][18] == grid._stage["buf"].data_ptr() == grid._stage["base"][0]
+    grid.tb3 = True
+    grid.run(10, 3)
+    assert grid.calls[-2][0] == "bz_yee3d_step3" and grid._stage["buf"].numel() == 2 * one
+    assert grid.calls[-2][1][19] == grid._stage["buf"].data_ptr() + 4 * one == grid._stage["base2"][0]
+    grid.tb3 = False
+    grid.add_gather([1], [500], np.arange(0, 40, 2), np.arange(41.0), [1.0], keep_series=False)
+    grid.run(13, 8)
+    assert grid.calls[-1][0] == "bz_yee3d_run2" and grid.calls[-1][1][21] == 2
+    assert grid._stage["buf"].numel() == 6 * int(np.prod(list(grid._stage["box"])[3:]))
