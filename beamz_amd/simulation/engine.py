@@ -867,6 +867,8 @@ class Fused2D:
             krows, kwaves = krows or r, kwaves or w
         if kstep and not self.kstep_applies():
             kstep = 0           # grid power needs every step: pairs or single steps instead
+        if kstep and self.pol == "Hz" and (kstep < 1 or not self.kshape_ok(int(kstep), krows or 8, kwaves or 8)):
+            kstep = 0           # this family took any shape when it had the one-step kernel only
         if kstep:
             self.set_kstep(kstep, krows or 8, kwaves or 8)
 
@@ -1020,6 +1022,9 @@ class Fused2D:
         self.set_kstep(*best)
         return best, timings
 
+    def kshape_ok(self, K, rows, waves):
+        return (int(rows), int(waves)) in self.KSHAPES and 2 * K < min(64, rows * waves)
+
     def set_kstep(self, K, rows=8, waves=8):
         """Tile list, monitor-owner tables and sample staging of the K-steps-per-pass kernel (K 0: off).
 
@@ -1031,7 +1036,7 @@ class Fused2D:
             self.kstep = 0
             return
         rows, waves = int(rows), int(waves)
-        if (rows, waves) not in self.KSHAPES or not 2 * K < min(64, rows * waves):
+        if not self.kshape_ok(K, rows, waves):
             raise ValueError(f"K steps per pass need (rows, waves) in {self.KSHAPES} and 2K < min(64, rows*waves)")
         if any(g.power is not None for g in self.grids):
             raise ValueError("K steps per pass do not accumulate grid power")
