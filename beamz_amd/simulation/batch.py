@@ -120,9 +120,13 @@ class FDTDBatch:
     def autotune(self, steps=20, segs=None):
         """Pick the kernel shape with the lowest measured step time: (K, rows, waves) when the engine runs K
         steps per pass, else the tile height (the two-step kernel's tiles when it runs pairs, else the one-step
-        kernel's); leaves the batch re-initialised."""
+        kernel's); leaves the batch re-initialised. ``segs``: the candidates. Tile heights given for (Hz, Ex, Ey)
+        members time the one-step kernel and stay with it."""
         T = self.sims[0].backend.torch
         if self.engine is None:
+            self.initialize()
+        if self.engine.kstep and self.engine.pol == "Hz" and segs is not None and all(np.ndim(q) == 0 for q in segs):
+            self.kstep = 0
             self.initialize()
         if self.engine.kstep:
             best, timings = self.engine.tune_kstep(steps=steps, candidates=segs)

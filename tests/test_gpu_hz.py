@@ -126,3 +126,26 @@ def test_hz_mode_source_matches_oracle(hip):
         ref = R.RefSim(sim.epsilon_r, sim.sigma, dx, dx, dt, len(t), sources=[src], polarization="Hz").run()
         for k in ("Hz", "Ex", "Ey"):
             assert rel_l2(np.real(getattr(sim, k)), ref.F[k]) < 1e-4, (enforce, k)
+
+
+def test_hz_batch_autotune_by_tile_height(hip):
+    """Tile heights as candidates time and choose the one-step kernel's tiles; without candidates the (K, rows, waves)
+    of the K-step kernel are timed. Either way the run's bits are those of the untuned one."""
+    def batch():
+        d, dx = design(97, 131)
+        t = np.arange(120) * 0.99 * dx / (bz.LIGHT_SPEED * np.sqrt(2))
+        d += bz.GaussianSource(position=(25 * dx, d.height / 2), width=dx / 4, signal=pulse(t))
+        return FDTDBatch([bz.FDTD(d, time=t, resolution=dx, polarization="Hz")], seg=8)
+    ref = batch()
+    ref.run()
+    for segs in ((2, 4), [8], None):
+        b = batch()
+        best, timings = b.autotune(steps=20, segs=segs)
+        assert set(timings) == set(segs or b.engine.KCANDIDATES) and best in timings
+        if segs:
+            assert b.engine.kstep == 0 and b.engine.seg == best
+        else:
+            assert (b.engine.kstep, b.engine.krows, b.engine.kwaves) == best
+        b.advance(b.num_steps)
+        for k in ("Hz", "Ex", "Ey"):
+            assert np.array_equal(getattr(b.sims[0], k), getattr(ref.sims[0], k)), (segs, k)
