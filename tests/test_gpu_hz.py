@@ -1,4 +1,4 @@
-"""GPU parity of the (Hz, Ex, Ey) polarisation (bz_yee2d_hz_run) against the FP64 oracle
+"""GPU parity of the (Hz, Ex, Ey) polarisation (bz_yee2d_hz_run, bz_yee2d_hz_runk) against the FP64 oracle
 (oracle/fdtd_ref.py RefSim(polarization="Hz"), pinned in tests/test_oracle_hz.py).
 
 Tolerances (relative L2): fields, monitor series and DFT 1e-4; monitor and grid power 2e-4;
@@ -84,15 +84,17 @@ def test_hz_polarisation_matches_fp64_oracle(hip):
 
 
 def test_hz_tile_heights_graphs_and_batch_are_bit_identical(hip):
-    base, *_ = run_case(power=False, seg2d=2)
-    for opts in ({"seg2d": 8}, {"seg2d": 16}, {"seg2d": 4, "graph2d": True}):
+    base, *_ = run_case(power=False, seg2d=2, kstep2d=0)      # one step per launch
+    for opts in ({"seg2d": 8, "kstep2d": 0}, {"seg2d": 16, "kstep2d": 0}, {"seg2d": 4, "kstep2d": 0, "graph2d": True},
+                 {"seg2d": 8}, {"seg2d": 16}, {"seg2d": 4, "graph2d": True}):        # then K steps per pass
         other, *_ = run_case(power=False, **opts)
+        assert other.grid.kernel_name().startswith("bz_yee2d_hz_run" + (" " if "kstep2d" in opts else "k ")), opts
         for k in ("Hz", "Ex", "Ey"):
             assert np.array_equal(getattr(other, k), getattr(base, k)), (opts, k)
     # a batch of uneven members, each bit-identical to its single run
     sims, singles = [], []
     for (nx, ny) in ((150, 84), (97, 131), (203, 66)):
-        single, *_ = run_case(nx, ny, power=False)
+        single, *_ = run_case(nx, ny, power=False, kstep2d=0)
         singles.append(single)
         d, dx = design(nx, ny)
         dt = 0.99 * dx / (bz.LIGHT_SPEED * np.sqrt(2))
