@@ -266,7 +266,9 @@ class AdjointProblem2D:
             # the coefficient arrays of the engine that last ran these materials: the forward engine with the full
             # history, else the recompute engine (it refreshes them at the start of every segment)
             eng = self.fwd if self.full else self.rec
-            cf = eng.coefs[b] if eng.kstep and eng.coefs is not None else None
+            if eng.kstep:
+                eng.coefficients()
+            cf = eng.coefs[b] if eng.kstep else None
             d.coef = cf.data_ptr() if cf is not None else None
             d.gc = eng.gcs[b].data_ptr() if cf is not None else None
             descs.append(d)

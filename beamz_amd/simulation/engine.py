@@ -1052,20 +1052,6 @@ class Fused2D:
             tiles = xcd_order(tiles, per_wg=1)
         self.kstep, self.krows, self.kwaves = K, rows, waves
         self.graphs = {}                     # captured launches hold the tables' addresses
-        if self.coefs is None:
-            # per-cell update coefficients, computed at the start of every run (bz_yee2d_coef): the K-step kernel
-            # then loads four numbers per cell instead of evaluating three divisions. The kernels address them
-            # with 32-bit byte offsets; a grid too large for that keeps coef NULL and the kernels divide.
-            self.coefs = [T.empty((g.ny, g.ld, 4), dtype=T.float32, device=self.dev)
-                          if 16 * g.ny * g.ld < 2 ** 32 else None for g in self.grids]
-            # and the one coefficient that cells without conductivity need
-            self.gcs = [None if c is None else T.empty(c.shape[:2], dtype=T.float32, device=self.dev)
-                        for c in self.coefs]
-            for d, c, h in zip(self.descs, self.coefs, self.gcs):
-                d.coef = c.data_ptr() if c is not None else None
-                d.gc = h.data_ptr() if h is not None else None
-            self.shift = None
-            self._desc_cache = {}
         self.tilesk = T.from_numpy(tiles.ravel()).to(self.dev)
         self.ntilesk = len(tiles)
         self.ent_start = self.ents = self.stagek = None
@@ -1075,6 +1061,25 @@ class Fused2D:
             self.ents = T.from_numpy(ents.ravel()).to(self.dev)
             self.ent_start = T.from_numpy(start).to(self.dev)
             self.stagek = T.zeros(2 * K * self.npts, dtype=T.float32, device=self.dev)   # two slots: q & 1
+
+    def coefficients(self):
+        """Allocate the K-step kernel's per-cell update coefficients: at the first run with it, so that an engine that
+        only holds tile lists has none (20 bytes per cell)."""
+        if self.coefs is not None:
+            return
+        T = self.torch
+        # computed at the start of every run (bz_yee2d_coef): the K-step kernel then loads four numbers per cell
+        # instead of evaluating three divisions. The kernels address them with 32-bit byte offsets; a grid too large
+        # for that keeps coef NULL and the kernels divide.
+        self.coefs = [T.empty((g.ny, g.ld, 4), dtype=T.float32, device=self.dev)
+                      if 16 * g.ny * g.ld < 2 ** 32 else None for g in self.grids]
+        # and the one coefficient that cells without conductivity need
+        self.gcs = [None if c is None else T.empty(c.shape[:2], dtype=T.float32, device=self.dev) for c in self.coefs]
+        for d, c, h in zip(self.descs, self.coefs, self.gcs):
+            d.coef = c.data_ptr() if c is not None else None
+            d.gc = h.data_ptr() if h is not None else None
+        self.shift = None
+        self._desc_cache = {}
 
     def _describe(self, g, snap=None):
         T = self.torch
@@ -1242,6 +1247,8 @@ class Fused2D:
             # the materials may have changed: the next K-step launch recomputes the coefficients, also when
             # this run is too short for one and a later run of the same materials passes coef=False
             self._coef_done = False
+        if self.kstep and count >= self.kstep:
+            self.coefficients()
         self._sync_descs(n0)
         self.step.fill_(n0)
         g0 = self.grids[0]

@@ -403,3 +403,21 @@ def test_gradient_pass_equals_in_kernel_accumulation(hip):
                     ref = g
                 assert np.array_equal(g, ref), (mode, pairs, kstep, gp, tab)
     assert np.abs(ref).max() > 0
+
+
+def test_the_tile_list_engine_of_a_full_history_holds_no_coefficients(hip):
+    """With the design-box history of every step the recompute engine never runs: the reverse sweep reads the forward
+    engine's coefficients. With checkpoints it holds its own."""
+    torch = hip
+    eps, sig, _ = materials(seed=5)
+    x0, y0, sx, sy = BOX
+    e_box = torch.from_numpy(eps[y0:y0 + sy, x0:x0 + sx]).float().cuda()[None]
+    for mode in ("full", "checkpoint"):
+        sim, mon, src, t = build(eps, sig, 64)
+        npts = len(mon.get_grid_points_2d(DX, DX))
+        prob = AdjointProblem2D([sim], [mon], np.ones(npts), BOX, kstep=8, checkpoint_every=16, snapshots=mode)
+        prob.forward(e_box)
+        prob.gradient()
+        held = prob.fwd if mode == "full" else prob.rec
+        assert (prob.rec.coefs is None) == (mode == "full")
+        assert prob._rs["descs"][0].coef == held.coefs[0].data_ptr()

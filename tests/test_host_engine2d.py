@@ -1,0 +1,48 @@
+"""Host side of the 2D engine (no GPU: its tables on the CPU, native calls recorded, not made)."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from beamz_amd import _native as N
+from beamz_amd.simulation.engine import Fused2D, Grid
+
+
+def grid(pol="Hz", nx=70, ny=40):
+    import torch
+    return Grid(SimpleNamespace(torch=torch, dev="cpu", stream=None), np.ones((ny, nx)), np.zeros((ny, nx)), 1.0, 1.0,
+                0.1, pol=pol)
+
+
+@pytest.mark.parametrize("shape", [(8, 3, 8), (40, 8, 8), (16, 4, 8), (8, 0, 7)])
+def test_shapes_that_do_not_apply_leave_the_one_step_kernel(shape):
+    """(K, rows, waves) that no kernel has are refused with (Ez, Hx, Hy) and were never read with (Hz, Ex, Ey)."""
+    K, rows, waves = shape
+    e = Fused2D([grid()], kstep=K, krows=rows, kwaves=waves)
+    assert e.kstep == 0 and not e.pairs
+    with pytest.raises(ValueError):
+        Fused2D([grid("Ez")], kstep=K, krows=rows, kwaves=waves)
+    assert Fused2D([grid()], kstep=-1).kstep == 0 and Fused2D([grid()], kstep=8).kstep == 8
+    assert Fused2D([grid()]).kstep and not Fused2D([grid()], krows=3).kstep
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """(entry point, arguments) of every native call; descriptors are not uploaded."""
+    made = []
+    monkeypatch.setattr(N, "call", lambda name, *a: made.append((name, a)))
+    monkeypatch.setattr(Fused2D, "_sync_descs", lambda self, n0, slot0=0: None)
+    return made
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+def test_coefficients_are_held_by_engines_that_run_k_steps(calls, pol):
+    """An engine that only holds tile lists (the reverse sweep's), or only takes single steps, has no coefficient
+    arrays; the first K-step launch allocates and fills them."""
+    e = Fused2D([grid(pol)], kstep=8)
+    assert e.tilesk is not None and e.coefs is None and e.gcs is None
+    e.run(0, 7)
+    assert e.coefs is None and not e.descs[0].coef
+    e.run(7, 8)
+    assert e.descs[0].coef == e.coefs[0].data_ptr() and e.descs[0].gc == e.gcs[0].data_ptr()
+    assert [c[0] for c in calls].count("bz_yee2d_coef") == 1
