@@ -355,8 +355,12 @@ __global__ __launch_bounds__(LANES* WPG) void k_adj2d_tb2(const bz_adj2d* __rest
 // order. Reads buffer rb, writes rb ^ 1.
 // Measured: the gradient of 16 designs of 600 x 600 cells, 3000 steps (reverse sweep, gradient pass, tables)
 // 39.1 -> 25.3 ms with one barrier per step, 11 instead of 18 operations per cell without conductivity, anchored
-// regions and the injection values of a launch staged in LDS. 99 registers: the gradient terms added in the sweep
-// (without l2hist) would spill at the 80 of the forward kernel.
+// regions and the injection values of a launch staged in LDS. 119 registers at 8 rows, 69 at 4: the gradient terms added
+// in the sweep (without l2hist) would spill at the 80 of the forward kernel.
+// A region with more injection values a launch than LDS holds (a diagonal line's box) reads them from the table one step
+// ahead, in a form of its own. One 256 x 256 grid, a line over 60 x 120 cells, us per step against summing them where
+// they are needed: 4.50 -> 2.15 (8, 8, 8), 2.27 -> 1.33 (8, 4, 8), 2.60 -> 1.36 (16, 4, 16). That form comes first: last,
+// it cost the others up to 3 % at 4 rows per wave.
 __device__ __forceinline__ float from_right(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, false));
 }
@@ -364,7 +368,7 @@ __device__ __forceinline__ float from_left(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, false));
 }
 
-// The part of the injection box inside a region.
+// The part of the injection box inside a region (sx 0: its values are not in LDS).
 struct InjBox {
     int x0, y0, sx, sy;
 };
@@ -425,15 +429,18 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
                              (grad_band && !A.l2hist)
                          ? 2
                          : (xedge ? 1 : 0);
-    // the design box, and the part of the injection box inside the region with its K steps' table values (sx 0:
-    // without the table or with more than INJ_LDS values the general form sums the injection itself), all written
+    // the design box, and the part of the injection box inside the region with its K steps' table values, all written
     // before the first barrier and read after it: from LDS they add no registers and no memory latency to a step
+    // (from_table: more values than LDS holds)
+    bool from_table = inj_band && A.inj_tab && !(grad_band && !A.l2hist);
     {
         const int x0 = max(A.inj_x0, rx0), x1 = min(A.inj_x0 + A.inj_sx, rx0 + LANES);
         const int y0 = max(A.inj_y0, ry0), y1 = min(A.inj_y0 + A.inj_sy, ry0 + RH);
         const bool meets = A.inj_w && A.inj_tab && x0 < x1 && y0 < y1;
         const int sx = meets && (long)K * (x1 - x0) * (y1 - y0) <= INJ_LDS ? x1 - x0 : 0, sy = y1 - y0;
-        if (threadIdx.x == 0 && threadIdx.y == 0) ibox = InjBox{x0, y0, sx, sy};
+        from_table = from_table && sx == 0;
+        if (threadIdx.x == 0 && threadIdx.y == 0)
+            ibox = InjBox{x0, y0, sx, sy};
         for (int q = w * LANES + l; q < K * sx * sy; q += LANES * KW) {
             const int k = q / (sx * sy), c = q - k * (sx * sy), n = n_top - k;
             const long cell = (long)(y0 + c / sx - A.inj_y0) * A.inj_sx + (x0 + c % sx - A.inj_x0);
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
     auto steps = [&](auto lossy_c, auto edge_c) {
         constexpr bool L = decltype(lossy_c)::value;
         constexpr int E = decltype(edge_c)::value;
-        const float r1 = E == 2 ? rxy : 1.0f;
+        const float r1 = E >= 2 ? rxy : 1.0f;
         // the four coefficients of every cell, and fa, gb of the row above
         float fa[B], gb[B], ca[B], gcl[B], fag = 1.0f, gbg = 0.0f;
         if (L) {
@@ -530,13 +537,26 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
                 }
             }
         }
+        // E == 3, from_table: the next step's injection values (their latency hides behind a step)
+        float ahead[B];
+        auto fetch = [&](int n) {
+            const float* __restrict__ tab = A.inj_tab + (long)max(n, 0) * A.inj_sx * A.inj_sy;
+            const int a = i - A.inj_x0;
+#pragma unroll
+            for (int r = 0; r < B; ++r) {
+                const int bb = jb + r - A.inj_y0;
+                // (-0 changes no value)
+                ahead[r] = n >= 1 && a >= 0 && a < A.inj_sx && bb >= 0 && bb < A.inj_sy ? tab[bb * A.inj_sx + a] : -0.0f;
+            }
+        };
+        if (E == 3) fetch(n_top);
         for (int k = 0; k < K; ++k) {
             const int n = n_top - k;
             float(*x)[KW][LANES] = xw[k & 1];
             // lE'' = M lE (kept in le) and w = gc lE'' on the interior
             float wv[B];
             auto interior = [&](int r) { return E == 0 || (xin && (E < 2 || (jb + r >= 1 && jb + r <= ny - 2))); };
-            if (E == 2 && src_band) {
+            if (E >= 2 && src_band) {
 #pragma unroll
                 for (int r = 0; r < B; ++r) le[r] = src_mul_at(A, i, jb + r) * le[r];
             }
@@ -569,7 +589,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
             if (k >= klive) continue;
             const float wb = x[0][wd][l], wg = x[1][wu][l];
             // lambda of the design cells into the history (a uniform base and 32-bit offsets)
-            if (grad_band && (E < 2 || A.l2hist)) {
+            if (grad_band && (E != 2 || A.l2hist)) {
                 const HistBox h = hbox;
                 const int hx0 = __builtin_amdgcn_readfirstlane(h.x0), hsx = __builtin_amdgcn_readfirstlane(h.sx);
                 const int hy0 = __builtin_amdgcn_readfirstlane(h.y0), hsy = __builtin_amdgcn_readfirstlane(h.sy);
@@ -597,7 +617,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
                 float mx = lx[r] + (wR - wv[r]);
                 if (E > 0) mx = hxok ? mx : 0.0f;
                 float my = mu_y(r1, ly[r], wv[r], wdn);
-                if (E == 2) my = j >= 0 && j <= ny - 2 ? my : 0.0f;
+                if (E >= 2) my = j >= 0 && j <= ny - 2 ? my : 0.0f;
                 const float g = L ? gb[r] : gb0;
                 const float fmx = g * mx, fmy = g * my;
                 lx[r] = L ? fa[r] * mx : mx;
@@ -613,7 +633,11 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
                 le[r] = lam_e(r1, cl2, fmx, fmxl, fmyu, fmy);
                 fmyu = fmy;
             }
-            if (E == 2 && inj_band && n >= 1) {
+            if (E == 3) {
+#pragma unroll
+                for (int r = 0; r < B; ++r) le[r] += ahead[r];
+                if (k + 1 < klive) fetch(n - 1);
+            } else if (E == 2 && inj_band && n >= 1) {
                 const InjBox h = ibox;
 #pragma unroll
                 for (int r = 0; r < B; ++r) {
@@ -626,13 +650,14 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 7 : (B == 8 ? 4 : 1)) void k_ad
         }
     };
     // One form runs (tests of separate copies of its number, as in the forward kernel)
-    const int form = klive == 0 || (lossy && edge == 2) ? 3 : (lossy ? 1 + edge : 0);
+    const int form = klive > 0 && from_table ? 4 : (klive == 0 || (lossy && edge == 2) ? 3 : (lossy ? 1 + edge : 0));
     auto is = [&](int f) {
         int v = form;
         asm volatile("" : "+s"(v));
         return v == f;
     };
     using std::bool_constant;
+    if (is(4)) steps(bool_constant<true>{}, std::integral_constant<int, 3>{});
     if (is(0)) steps(bool_constant<false>{}, std::integral_constant<int, 0>{});
     if (is(1)) steps(bool_constant<true>{}, std::integral_constant<int, 0>{});
     if (is(2)) steps(bool_constant<true>{}, std::integral_constant<int, 1>{});

@@ -337,7 +337,9 @@ typedef struct bz_adj2d {
                                            * bz_adj2d_grad then adds the terms, in the same order */
     float* inj_tab;                       /* NULL, or [num_steps][inj_sy][inj_sx]: the objective's injection
                                            * value of each cell at step n >= 1, as bz_adj2d_injtab computes it;
-                                           * bz_adj2d_runk then reads it instead of summing inj_w * phasor */
+                                           * bz_adj2d_runk then reads it instead of summing inj_w * phasor (but
+                                           * where it adds gradient terms, without l2hist, beside a part of the
+                                           * box of more than 2048 values a launch) */
     const float* gc;                      /* NULL, or bz_sim2d.gc of the same materials (read with coef) */
 } bz_adj2d;
 

@@ -421,3 +421,37 @@ def test_the_tile_list_engine_of_a_full_history_holds_no_coefficients(hip):
         held = prob.fwd if mode == "full" else prob.rec
         assert (prob.rec.coefs is None) == (mode == "full")
         assert prob._rs["descs"][0].coef == held.coefs[0].data_ptr()
+
+
+# a column, a slanted line (4 cells wide) and a diagonal (its box: 41 x 41 cells), from and to these cells
+@pytest.mark.parametrize("line", [((58, 8), (58, 48)), ((56, 8), (59, 48)), ((20, 8), (60, 48))])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 4, 16)])
+def test_the_k_step_sweep_reads_the_injection_table(hip, monkeypatch, shape, line):
+    """With the table of injection values the K-step reverse kernel sums no weights times phasors, however many cells
+    of the box a region holds: the weights are cleared once the table and the terminal condition are made, and the
+    gradient's bits are those of single steps with their weights (128 steps: whole launches only)."""
+    from beamz_amd import _native as N
+    torch = hip
+    eps, sig, _ = materials(seed=5)
+    x0, y0, sx, sy = BOX
+    e_box = torch.from_numpy(eps[y0:y0 + sy, x0:x0 + sx]).float().cuda()[None]
+    out = []
+    call = N.call
+    for K, rows, waves in ((0, 8, 8), shape):
+        sim, mon, src, t = build(eps, sig, 128)
+        mon.start, mon.end = (tuple(q * DX for q in cell) for cell in line)
+        c = np.exp(1j * np.linspace(0, 2, len(mon.get_grid_points_2d(DX, DX))))
+        prob = AdjointProblem2D([sim], [mon], c, BOX, kstep=K, snapshots="full")
+        prob.forward(e_box)
+        if K:
+            prob.rec.set_kstep(K, rows, waves)
+
+            def clear_weights(name, *a):
+                if name == "bz_adj2d_runk":
+                    for inj in prob._rs["inj"]:
+                        inj[4].zero_()
+                return call(name, *a)
+            monkeypatch.setattr(N, "call", clear_weights)
+        out.append(prob.gradient().cpu().numpy())
+        assert prob._rs["tabled"]
+    assert np.abs(out[0]).max() > 0 and np.array_equal(out[0], out[1])
