@@ -698,6 +698,12 @@ __global__ void k_gather2d_k(Gather2D G, const float* __restrict__ stage, const 
     gather_k(G, stage, *step + K * q, K, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
+// What a cell of weight v (-0: no cell of the source) adds at amplitude amp.
+__device__ __forceinline__ float src_term(float v, float amp) {
+    const float a = computed(v * amp);
+    return __float_as_uint(v) == 0x80000000u ? v : a;
+}
+
 constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further ones are read again every step)
 
 // SEL: some simulation's source box holds several sources (bz_sim2d.src_sel); without it the per-cell
@@ -892,7 +898,8 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                 }
             }
         }
-        // the source's weights of this wave's cells (0 outside its box), loaded once, in LDS
+        // the source's weights of this wave's cells, loaded once, in LDS: -0, which as an addend changes no value,
+        // outside its box, and a weight of zero as +0 (its product is added, NaN at an infinite amplitude)
         const bool plain_src = E == 2 && src_band && !SEL && !S.src_mul;
         auto src_cell = [&](int r) {
             const int a = i - S.src_x0, b = jb + r - S.src_y0;
@@ -902,7 +909,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
 #pragma unroll
             for (int r = 0; r < B + HZ; ++r) {
                 const long o = src_cell(r < B ? r : -1);
-                wsrc[w][r][l] = o >= 0 ? gload(S.src_add, o) : 0.0f;
+                wsrc[w][r][l] = o >= 0 ? gload(S.src_add, o) + 0.0f : -0.0f;
             }
         }
         for (int k = 0; k < K; ++k) {
@@ -925,8 +932,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                     for (int r = 0; r < 4; ++r) v[r] = wsrc[w][r0 + r][l];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float a = computed(v[r] * amp);
-                        add[r0 + r] = v[r] != 0.0f ? a : 0.0f;
+                        add[r0 + r] = src_term(v[r], amp);
                     }
                 };
                 if (E == 2 && src_band) amp = amps[k];
@@ -1023,10 +1029,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                         if (B > 4 && r % 4 == 0) src_adds(r);
                         ez[r] += add[r];
                     }
-                    if (HZ) {
-                        const float v = wsrc[w][B][l], a = computed(v * amp);
-                        hyg += v != 0.0f ? a : 0.0f;
-                    }
+                    if (HZ) hyg += src_term(wsrc[w][B][l], amp);
                 } else if (E == 2 && src_band) {
 #pragma unroll
                     for (int r = 0; r < B + HZ; ++r) {

@@ -62,3 +62,30 @@ def test_kstep_forms_give_the_bits_of_single_steps(hip, shape, damped, pol):
         assert set(a) == set(b) and any(np.any(v) for v in b.values())
         for k in b:
             assert np.array_equal(a[k], b[k]), (size, k)
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 4, 16), (3, 16, 4)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 0.0])
+def test_zero_weights_inside_a_source_box(hip, value, shape, pol):
+    """A source box with cells of weight 0 (and cells of no source, weight 0 too): the K-step kernels give what one step
+    per launch gives also where the signal is not finite (0 times infinity is NaN) and where it is 0."""
+    steps, K = 16, shape[0]
+    sig = np.cos(0.3 * np.arange(steps))
+    sig[K - 1] = value
+    out = []
+    for k in (0, K):
+        s, mons = world(113, 64, steps, True, 3, pol)
+        s.initialize_simulation(save=False, live=False)
+        g = s.grid
+        g.kstep2d, g.krows2d, g.kwaves2d = k, shape[1], shape[2]
+        g.sources = []
+        idx = np.array([(j, i) for j in range(5, 21) for i in range(40, 70) if (i + j) % 3])
+        w = np.where(idx.sum(axis=1) % 3 == 1, 1.0 / (1 + idx[:, 0]), 0.0)
+        g.add_point_source(g.names[0], idx, w, None, sig)
+        g.run(0, K)
+        out.append({n: np.real(getattr(s, n)).copy() for n in g.names})
+        assert bool(g._f2d.kstep) == bool(k)
+    for n in out[0]:
+        assert np.any(out[0][n]) and np.array_equal(out[0][n], out[1][n], equal_nan=True), n
+    assert np.isfinite(value) or not np.all(np.isfinite(out[0][s.grid.names[0]]))
