@@ -630,6 +630,8 @@ int run(const bz_sim2d* sims, const int* tiles, int ntiles, int* step, int nstep
 // tile to staging slot q & 1 of launch q, stage[q & 1][k][point], and accumulated into the FP64 DFT in step
 // order by extra workgroups of the next launch (by k_gather2d_k after the last one).
 // Reads buffer rd, writes rd ^ 1.
+// The tile list is made for P steps per launch (its regions' pitch and stored windows, P = K above); the last launch of
+// a run may advance K < P of them, so that one launch takes the steps a run has beyond a multiple of P.
 // Update coefficients of every cell: blockIdx.y is the simulation, the x blocks stride over its cells.
 __global__ __launch_bounds__(256) void k_coef2d(const bz_sim2d* __restrict__ sims) {
     const bz_sim2d& S = sims[blockIdx.y];
@@ -694,8 +696,8 @@ __device__ __forceinline__ void gather_k(const Gather2D& G, const float* __restr
 }
 
 // The gather of the last launch of a call (the others run inside the next launch).
-__global__ void k_gather2d_k(Gather2D G, const float* __restrict__ stage, const int* __restrict__ step, int q, int K) {
-    gather_k(G, stage, *step + K * q, K, (long)blockIdx.x * blockDim.x + threadIdx.x);
+__global__ void k_gather2d_k(Gather2D G, const float* __restrict__ stage, const int* __restrict__ step, int n, int K) {
+    gather_k(G, stage, *step + n, K, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // What a cell of weight v (-0: no cell of the source) adds at amplitude amp.
@@ -719,7 +721,7 @@ constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further 
 // Ey of the last, and each keeps the Hz of the row above (with its source, which this family adds to Hz).
 template <int B, int KW, bool SEL, bool HZ>
 __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
-                                                        const int* __restrict__ tiles, int ntiles, int K,
+                                                        const int* __restrict__ tiles, int ntiles, int P, int K,
                                                         const int* __restrict__ step, int q, int rd,
                                                         const int* __restrict__ ent_start,
                                                         const int* __restrict__ ents, float* __restrict__ stage_all,
@@ -737,7 +739,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
     if (t >= ntiles) {
         // monitor samples of the previous launch (q > 0): staging slot (q - 1) & 1, which this launch does not
         // write
-        gather_k(G, stage_all + (long)((q - 1) & 1) * K * npts, *step + K * (q - 1), K,
+        gather_k(G, stage_all + (long)((q - 1) & 1) * P * npts, *step + P * (q - 1), P,
                  (long)(t - ntiles) * (LANES * KW) + threadIdx.y * LANES + threadIdx.x);
         return;
     }
@@ -750,14 +752,14 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
     const int l = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.y);
     // region origin, and its window of stored cells [cx0, cx1) x [cy0, cy1)
-    const int rx0 = tx * (LANES - 2 * K) - (anch ? 0 : K), ry0 = ty * (RH - 2 * K) - (anch ? 0 : K);
+    const int rx0 = tx * (LANES - 2 * P) - (anch ? 0 : P), ry0 = ty * (RH - 2 * P) - (anch ? 0 : P);
     const bool top = anch && ty == 0, bottom = anch && ry0 + RH >= ny;
-    const int cx0 = anch && tx == 0 ? 0 : K, cx1 = anch && rx0 + LANES >= nx ? LANES : LANES - K;
-    const int cy0 = top ? 0 : K, cy1 = bottom ? RH : RH - K;
+    const int cx0 = anch && tx == 0 ? 0 : P, cx1 = anch && rx0 + LANES >= nx ? LANES : LANES - P;
+    const int cy0 = top ? 0 : P, cy1 = bottom ? RH : RH - P;
     const int i = rx0 + l;
     const int jb = ry0 + w * B;                     // grid row of the wave's first register row
     const int wr = rd ^ 1;
-    const int n0 = *step + K * q;
+    const int n0 = *step + P * q;
     const float rdy = S.rdy;
     // 1 on square cells; uniform, so kept in a scalar register
     const float rdx = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(S.rdx)));
@@ -970,13 +972,13 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                         }
                     }
                 }
-                // snapshot of call-relative step q*K+k at the stored cells: the Ez this step reads, the Hx, Hy it
+                // snapshot of call-relative step q*P+k at the stored cells: the Ez this step reads, the Hx, Hy it
                 // wrote
                 if (snap_band) {        // a uniform base per plane and 32-bit offsets
                     const SnapBox sn = snq;
                     const int qx0 = __builtin_amdgcn_readfirstlane(sn.x0), qsx = __builtin_amdgcn_readfirstlane(sn.sx);
                     const int qy0 = __builtin_amdgcn_readfirstlane(sn.y0), qsy = __builtin_amdgcn_readfirstlane(sn.sy);
-                    float* p0 = S.snap + (long)(q * K + k) * 3 * qsx * qsy;
+                    float* p0 = S.snap + (long)(q * P + k) * 3 * qsx * qsy;
                     float* p1 = p0 + (long)qsx * qsy;
                     float* p2 = p1 + (long)qsx * qsy;
                     const int a = i - qx0;
@@ -1045,7 +1047,7 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
             // rows, and the lanes read their entries' cells back between them (no workgroup barrier and no wait in
             // between: a wave's LDS operations complete in order)
             if (E == 2 && nmine > 0) {
-                float* __restrict__ stage = stage_all + ((long)(q & 1) * K + k) * npts;
+                float* __restrict__ stage = stage_all + ((long)(q & 1) * P + k) * npts;
                 for (int eb = 0; eb < min(nmine, ELIST); eb += LANES) {
                     const int2 ent = list[min(eb + l, nmine - 1)];
                     float val = 0.0f;
@@ -1105,32 +1107,31 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
     }
 }
 
+// nlaunch launches of P steps, then one of `part` (0: none).
 template <int B, int KW, bool HZ>
-int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int K, int* step, int rd0, int nlaunch,
+int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int P, int* step, int rd0, int nlaunch, int part,
          const int* ent_start, const int* ents, float* stage, const Gather2D& G, bool sel, hipStream_t st) {
     const dim3 b(LANES, KW);
     // sample staging and entry lists in LDS, only when there are monitor points
     const size_t lds = G.npts > 0 ? (size_t)KW * (B * LANES * sizeof(float) + ELIST * sizeof(int2)) : 0;
     const long gather_threads = (long)G.npts * (G.nfreq > 0 ? G.nfreq : 1);
     const int gather_blocks = (int)((gather_threads + LANES * KW - 1) / (LANES * KW));
+    const int total = nlaunch + (part > 0);
     // the gather of launch q-1 runs as extra workgroups of launch q; the last launch's gets a launch of its own
-    for (int q = 0; q < nlaunch; ++q) {
+    for (int q = 0; q < total; ++q) {
         const dim3 g(ntiles + (q > 0 && G.npts > 0 ? gather_blocks : 0));
-        if (sel)
-            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, true, HZ>), g, b, lds, st, sims, tiles, ntiles, K, step, q, (rd0 + q) & 1,
-                               ent_start, ents, stage, G);
-        else
-            hipLaunchKernelGGL((k_yee2d_tbk<B, KW, false, HZ>), g, b, lds, st, sims, tiles, ntiles, K, step, q,
-                               (rd0 + q) & 1, ent_start, ents, stage, G);
+        const auto kern = sel ? k_yee2d_tbk<B, KW, true, HZ> : k_yee2d_tbk<B, KW, false, HZ>;
+        hipLaunchKernelGGL(kern, g, b, lds, st, sims, tiles, ntiles, P, q < nlaunch ? P : part, step, q, (rd0 + q) & 1,
+                           ent_start, ents, stage, G);
         BZ_CHECK_LAUNCH("bz_yee2d_runk(steps)");
     }
     if (G.npts > 0) {
-        const int q = nlaunch - 1;
+        const int q = total - 1;
         hipLaunchKernelGGL(k_gather2d_k, dim3((int)((gather_threads + 255) / 256)), dim3(256), 0, st, G,
-                           stage + (long)(q & 1) * K * G.npts, step, q, K);
+                           stage + (long)(q & 1) * P * G.npts, step, P * q, part ? part : P);
         BZ_CHECK_LAUNCH("bz_yee2d_runk(gather)");
     }
-    hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, st, step, K * nlaunch);
+    hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, st, step, P * nlaunch + part);
     BZ_CHECK_LAUNCH("bz_yee2d_runk(tick)");
     return BZ_OK;
 }
@@ -1240,11 +1241,12 @@ extern "C" int bz_yee2d_run2(const bz_sim2d* sims, int nsims, const int* tiles, 
     return BZ_OK;
 }
 
+// nlaunch launches of ksteps steps, then one of `part` (0: none).
 template <bool HZ>
 static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows,
-                     int waves, int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
-                     float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow, float* series,
-                     int nfreq, const double* phasor, double* dft, int src_sel, void* stream) {
+                     int waves, int ksteps, int* step, int rd0, int nlaunch, int part, const int* ent_start,
+                     const int* ents, float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
+                     float* series, int nfreq, const double* phasor, double* dft, int src_sel, void* stream) {
     BZ_REQUIRE(sims && nsims > 0 && tiles && ntiles > 0 && step && nlaunch >= 0 && (rd0 == 0 || rd0 == 1),
                name + ": bad arguments");
     const int shape = rows * 100 + waves;
@@ -1258,7 +1260,7 @@ static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, c
     BZ_REQUIRE(!grp || (nslot > 0 && nrow > 0), name + ": point groups need nslot > 0 and nrow > 0");
     BZ_REQUIRE((long)npts * (nfreq > 0 ? nfreq : 1) / 256 < (1L << 31) - 1,
                name + ": too many monitor points x frequencies");
-    if (nlaunch == 0) return BZ_OK;
+    if (nlaunch == 0 && part == 0) return BZ_OK;
     Gather2D G;
     G.pts = nullptr;
     G.npts = npts;
@@ -1273,7 +1275,7 @@ static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, c
     const hipStream_t st = (hipStream_t)stream;
     if (npts == 0) ent_start = ents = nullptr;
 #define BZ_RUNK(R, W) \
-    runk<R, W, HZ>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, ent_start, ents, stage, G, src_sel != 0, st)
+    runk<R, W, HZ>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, part, ent_start, ents, stage, G, src_sel != 0, st)
     switch (shape) {
         case 804: return BZ_RUNK(8, 4);
         case 808: return BZ_RUNK(8, 8);
@@ -1290,17 +1292,31 @@ extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, 
                              float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
                              float* series, int nfreq, const double* phasor, double* dft, int src_sel,
                              void* stream) {
-    return runk_call<false>("bz_yee2d_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, ent_start, ents,
-                            stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel, stream);
+    return runk_call<false>("bz_yee2d_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, 0,
+                            ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
+                            stream);
 }
 
 extern "C" int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
-                             int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
-                             float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
-                             float* series, int nfreq, const double* phasor, double* dft, int src_sel,
-                             void* stream) {
-    return runk_call<true>("bz_yee2d_hz_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, ent_start, ents,
-                            stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel, stream);
+                                int ksteps, int* step, int rd0, int nlaunch, const int* ent_start, const int* ents,
+                                float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
+                                float* series, int nfreq, const double* phasor, double* dft, int src_sel,
+                                void* stream) {
+    return runk_call<true>("bz_yee2d_hz_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, 0,
+                           ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
+                           stream);
+}
+
+extern "C" int bz_yee2d_runk_steps(int hz, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows,
+                                   int waves, int ksteps, int* step, int rd0, int nsteps, const int* ent_start,
+                                   const int* ents, float* stage, int npts, const int* slot, const int* grp, int nslot,
+                                   int nrow, float* series, int nfreq, const double* phasor, double* dft, int src_sel,
+                                   void* stream) {
+    BZ_REQUIRE(ksteps >= 1 && nsteps >= 0, "bz_yee2d_runk_steps: bad step counts");
+    return (hz ? runk_call<true> : runk_call<false>)(
+        "bz_yee2d_runk_steps", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nsteps / ksteps,
+        nsteps % ksteps, ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
+        stream);
 }
 
 extern "C" int bz_yee2d_coef(const bz_sim2d* sims, int nsims, int max_cells, void* stream) {

@@ -979,6 +979,10 @@ class Fused2D:
         self.tiles2 = T.from_numpy(tiles.ravel()).to(self.dev)
         self.ntiles2 = len(tiles)
 
+    # Steps short of a launch, one by one / in a launch of their own, us a call: after one launch 2 steps 70 / 55 at
+    # 800 x 400, 8 steps 84 / 58; alone (with the pass over the coefficients) 10 steps 50 / 36, at 1000 x 990 8 steps
+    # 67 / 68 ((Hz, Ex, Ey): 69 / 79), 10 steps 82 / 71 (85 / 84)
+    PART_MIN, PART_ALONE = 2, 10
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
     # (K, rows, waves) candidates of tune_kstep. Forward sweeps: 64 grids of 256 x 256 cells 4.95 / 5.05 us/step
     # for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 4.49 / 4.45; 16 grids of 600 x 600 cells
@@ -1213,13 +1217,14 @@ class Fused2D:
         self.desc_dev = cached
         self.shift = key
 
-    def _launch_k(self, nl, rd0):
+    def _launch_k(self, count, rd0):
+        """count steps in launches of K, the last one of what is left."""
         ptr = lambda t: t.data_ptr() if t is not None else None
-        N.call("bz_yee2d_hz_runk" if self.pol == "Hz" else "bz_yee2d_runk", self.desc_dev.data_ptr(), len(self.grids), self.tilesk.data_ptr(), self.ntilesk,
-               self.krows, self.kwaves, self.kstep, self.step.data_ptr(), rd0, nl, ptr(self.ent_start),
-               ptr(self.ents), ptr(self.stagek), self.npts, ptr(self.slot), ptr(self.grp), self.nslot, self.nrow,
-               ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft), int(self.multi_src),
-               self.grids[0].stream)
+        N.call("bz_yee2d_runk_steps", int(self.pol == "Hz"), self.desc_dev.data_ptr(), len(self.grids),
+               self.tilesk.data_ptr(), self.ntilesk, self.krows, self.kwaves, self.kstep, self.step.data_ptr(), rd0,
+               count, ptr(self.ent_start), ptr(self.ents), ptr(self.stagek), self.npts, ptr(self.slot), ptr(self.grp),
+               self.nslot, self.nrow, ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft),
+               int(self.multi_src), self.grids[0].stream)
 
     def _launch(self, count):
         ptr = lambda t: t.data_ptr() if t is not None else None
@@ -1227,6 +1232,15 @@ class Fused2D:
         N.call("bz_yee2d_hz_run" if self.pol == "Hz" else "bz_yee2d_run", self.desc_dev.data_ptr(), len(self.grids), self.tiles.data_ptr(), self.ntiles,
                self.seg, self.step.data_ptr(), count, ptr(self.pts), self.npts, ptr(self.slot), ptr(self.grp),
                self.nslot, self.nrow, ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft), g0.stream)
+
+    def _in_k_steps(self, count):
+        """How many of a run's count steps go in K-step launches: whole ones, and a last one of the steps left where it
+        beats them one by one (engines that run pairs take those): from PART_MIN steps on, alone from PART_ALONE."""
+        if not self.kstep:
+            return 0
+        left = count % self.kstep
+        own = not self.pairs and left >= (self.PART_MIN if count > left else self.PART_ALONE)
+        return count if own else count - left
 
     def run(self, n0, count, coef=True):
         """Advance every grid by ``count`` steps starting at step index n0. coef=False skips recomputing the
@@ -1247,7 +1261,8 @@ class Fused2D:
             # the materials may have changed: the next K-step launch recomputes the coefficients, also when
             # this run is too short for one and a later run of the same materials passes coef=False
             self._coef_done = False
-        if self.kstep and count >= self.kstep:
+        inK = self._in_k_steps(count)
+        if inK:
             self.coefficients()
         self._sync_descs(n0)
         self.step.fill_(n0)
@@ -1256,34 +1271,33 @@ class Fused2D:
             e0, e1 = T.cuda.Event(enable_timing=True), T.cuda.Event(enable_timing=True)
             e0.record()
         total = count
-        if self.kstep and count >= self.kstep:
-            # launches of K steps each; launch q reads the buffer holding step n0 + qK and writes the other one
-            K = self.kstep
-            nl = count // K
-            ptr = lambda t: t.data_ptr() if t is not None else None
+        if inK:
+            # launches of K steps each (the last one may take fewer); launch q reads the buffer holding step n0 + qK and
+            # writes the other one
+            nl = -(-inK // self.kstep)
             # coefficients of the current materials (a caller may have written eps or sig since the last run)
             if not self._coef_done:
                 N.call("bz_yee2d_coef", self.desc_dev.data_ptr(), len(self.grids),
                        max(g.ny * g.ld for g in self.grids), g0.stream)
                 self._coef_done = True
             if self.use_graph:
-                # one captured graph per (launch count, first buffer); the step base lives in device memory
-                key = ("k", nl, n0 & 1)
+                # one captured graph per (step count, first buffer); the step base lives in device memory
+                key = ("k", inK, n0 & 1)
                 gr = self.graphs.get(key)
                 if gr is None:
                     gr = T.cuda.CUDAGraph()
                     T.cuda.synchronize(self.dev)
                     with T.cuda.graph(gr):
-                        self._launch_k(nl, n0 & 1)
+                        self._launch_k(inK, n0 & 1)
                     self.graphs[key] = gr
                 gr.replay()
             else:
-                self._launch_k(nl, n0 & 1)
+                self._launch_k(inK, n0 & 1)
             for g in self._advancing():
                 g._cur = (g._cur + nl) % 2
-            n0, count = n0 + nl * K, count - nl * K
+            n0, count = n0 + inK, count - inK
             if count:
-                # the step counter is already there; later steps write snapshot slots from nl*K on
+                # the step counter is already there; later steps write snapshot slots from inK on
                 self._sync_descs(n0, total - count)
         rem = count
         if self.pairs and count >= 2:

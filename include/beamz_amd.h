@@ -35,6 +35,7 @@
  *   bz_yee2d_run .......... fused multi-step 2D engine for many independent simulations at once:
  *                           per step numpy_backend.py:34-88 (H, E), helper.py:96-118 (source),
  *                           helper.py:231-256 (monitor samples + DFT), helper.py:120-187 (power)
+ *   bz_yee2d_runk_steps ... bz_yee2d_runk launches and a last one of the steps left, from one call
  *   bz_yee2d_hz_run(k) .... the (Hz, Ex, Ey) polarisation of bz_yee2d_run: the reference's 3D update
  *                           fdtd.py:200-310 restricted to d/dz = 0 (its 2D path numpy_backend.py:34-88 has
  *                           only the (Ez, Hx, Hy) family)
@@ -300,6 +301,13 @@ int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntil
                      int* step, int rd0, int nlaunch, const int* ent_start, const int* ents, float* stage, int npts,
                      const int* slot, const int* grp, int nslot, int nrow, float* series, int nfreq,
                      const double* phasor, double* dft, int src_sel, void* stream);
+
+/* nsteps steps by bz_yee2d_runk (hz nonzero: bz_yee2d_hz_runk) launches on the same lists: nsteps / ksteps launches of
+ * ksteps steps and, where steps are left, one that advances those. Launch q reads buffer (rd0 + q) & 1. */
+int bz_yee2d_runk_steps(int hz, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
+                        int ksteps, int* step, int rd0, int nsteps, const int* ent_start, const int* ents, float* stage,
+                        int npts, const int* slot, const int* grp, int nslot, int nrow, float* series, int nfreq,
+                        const double* phasor, double* dft, int src_sel, void* stream);
 
 /* ---------------- reverse-time 2D adjoint ----------------
  * No reference counterpart (the reference's gradient is the overlap heuristic of

@@ -89,3 +89,50 @@ def test_zero_weights_inside_a_source_box(hip, value, shape, pol):
     for n in out[0]:
         assert np.any(out[0][n]) and np.array_equal(out[0][n], out[1][n], equal_nan=True), n
     assert np.isfinite(value) or not np.all(np.isfinite(out[0][s.grid.names[0]]))
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("shape", [(16, 4, 16), (12, 8, 8), (31, 8, 16)])
+def test_runs_in_pieces_give_the_bits_of_single_steps(hip, shape, graph, pol):
+    """Runs of whole launches and of last steps that take a launch of their own (8 to K - 1 steps, also alone), one
+    after the other, with monitors; with graphs each piece twice (captured, then replayed)."""
+    K = shape[0]
+    pieces = [9, 2 * K, K - 1, 3, K + 8, 9, K + 8, K - 1, 1, 2 * K + 9]
+    steps = sum(pieces)
+    ref = run(steps, True, pol, kstep=0, pairs=False)
+    mem = [world(nx, ny, steps, True, q, pol) for q, (nx, ny) in enumerate(SIZES)]
+    batch = FDTDBatch([s for s, _ in mem], kstep=K, krows=shape[1], kwaves=shape[2], pairs=False, graph=graph)
+    batch.initialize()
+    for n in pieces:
+        batch.advance(n)
+    for size, (s, mons), b in zip(SIZES, mem, ref):
+        s.finalize_simulation()
+        a = {k: np.real(getattr(s, k)).copy() for k in s.grid.names}
+        for m in mons:
+            a.update({m.name + k: np.array(v) for k, v in m.dft.items()})
+            a.update({m.name + "series" + k: np.array(v) for k, v in m.fields.items() if len(v)})
+        assert set(a) == set(b)
+        for k in b:
+            assert np.array_equal(a[k], b[k]), (size, k)
+
+
+@pytest.mark.parametrize("count", [12, 28, 47])
+def test_snapshots_of_the_last_steps_follow_the_launches(hip, count):
+    """Snapshot boxes of a run of whole launches and a last one of fewer steps equal those of single steps."""
+    import torch
+    from beamz_amd.simulation.engine import Fused2D
+    got = []
+    for K in (0, 16):
+        s, _ = world(160, 145, 64, True, 2, "Ez")
+        s.initialize_simulation(save=False, live=False)
+        buf = torch.full((count, 3, 70, 90), -7.0, dtype=torch.float32, device="cuda")
+        eng = Fused2D([s.grid], seg=8, monitors=False, snapshots=[(10, 12, 90, 70, buf)], pairs=False, kstep=K, krows=4,
+                      kwaves=16)
+        s.grid._f2d = False
+        eng.run(0, 5)
+        eng.run(5, count)
+        got.append([buf.cpu().numpy()] + [s.field(k).cpu().numpy() for k in s.grid.names])
+    assert not np.any(got[0][0] == -7.0)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

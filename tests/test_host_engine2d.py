@@ -46,3 +46,29 @@ def test_coefficients_are_held_by_engines_that_run_k_steps(calls, pol):
     e.run(7, 8)
     assert e.descs[0].coef == e.coefs[0].data_ptr() and e.descs[0].gc == e.gcs[0].data_ptr()
     assert [c[0] for c in calls].count("bz_yee2d_coef") == 1
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+@pytest.mark.parametrize("count", [1, 7, 9, 10, 15, 16, 17, 18, 24, 31, 40, 48])
+def test_steps_short_of_a_launch_take_one_of_their_own(calls, pol, count):
+    """The steps of a run that are fewer than K go in one launch on the same tile list, from two on after whole
+    launches and from ten on alone; fewer go one by one. The buffers' parity moves once per launch."""
+    e = Fused2D([grid(pol)])
+    assert e.kstep == 16 and not e.pairs
+    e.run(0, count)
+    nl, left = divmod(count, 16)
+    single = left if left < (2 if nl else 10) else 0
+    made = {n: a for n, a in calls}
+    assert ("bz_yee2d_runk_steps" in made) == (count > single)
+    if count > single:
+        a = made["bz_yee2d_runk_steps"]
+        assert (a[0], a[7], a[9], a[10]) == (int(pol == "Hz"), 16, 0, count - single) and "bz_yee2d_coef" in made
+    assert made.get("bz_yee2d_hz_run" if pol == "Hz" else "bz_yee2d_run", [0] * 7)[6] == single
+    assert e.grids[0]._cur == (nl + (left > single) + single) % 2
+
+
+def test_pairs_take_the_steps_short_of_a_launch(calls):
+    e = Fused2D([grid("Ez")], kstep=12, krows=8, kwaves=8, pairs=True)
+    e.run(0, 23)
+    assert [n for n, _ in calls] == ["bz_yee2d_coef", "bz_yee2d_runk_steps", "bz_yee2d_run2", "bz_yee2d_run"]
+    assert calls[1][1][10] == 12
