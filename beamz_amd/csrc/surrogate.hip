@@ -1515,16 +1515,23 @@ __global__ void k_head(const uint16_t* __restrict__ a, const float* __restrict__
     }
 }
 
-// The head with 8 channels per thread: a workgroup of 1024 threads per sample splits its pixels into S = 1024 / (C / 8)
-// interleaved slices (thread t: channels 8 (t % (C / 8)) .. +7 by 16-byte loads, pixels t / (C / 8) + S k); the
-// slices' sums are added in slice order in LDS, and 32 lanes share an output (deterministic). C % 8 == 0 and
-// 256 % (C / 8) == 0. Bound by the latency of its dependent passes, at any batch: 256 threads with one lane per output
-// took 17 us at 256 pixels x 256 channels, this 7.5.
+// The head with 8 channels per thread: a workgroup of 1024 threads per sample splits its pixels into S interleaved
+// slices (thread t: channels 8 (t % (C / 8)) .. +7 by 16-byte loads, pixels t / (C / 8) + S k); the slices' sums are
+// added in slice order in LDS, and 32 lanes share an output (deterministic). C % 8 == 0 and 256 % (C / 8) == 0. Bound by
+// the latency of its dependent passes, at any batch: 256 threads with one lane per output took 17 us at 256 pixels x 256
+// channels, this 7.5. S balances HW / S loads in a row, eight in flight, against S additions in a row: the power of two
+// from 4 sqrt(HW) on, within the threads and the pixels. With as many as the threads hold, one pixel x 8 channels took
+// 15 us (now 4.0), 1000 x 16 9.6 (5.5).
+inline int head_slices(int HW, int C) {
+    int s = 1;
+    while (s < 1024 / (C / 8) && (long)s * s < 16L * HW) s *= 2;
+    return s < HW ? s : HW;
+}
 __global__ __launch_bounds__(1024) void k_head8(const uint16_t* __restrict__ a, const float* __restrict__ fw,
                                                 const float* __restrict__ fb, float* __restrict__ gap,
-                                                float* __restrict__ out, int HW, int C, int nout) {
+                                                float* __restrict__ out, int HW, int C, int nout, int S) {
     extern __shared__ float sh[];
-    const int G = C / 8, S = 1024 / G;
+    const int G = C / 8;
     float* red = sh;             // [S][C]
     float* sg = sh + S * C;      // [C]
     const int b = blockIdx.x, t = threadIdx.x, cg = t % G, sl = t / G;
@@ -1533,14 +1540,15 @@ __global__ __launch_bounds__(1024) void k_head8(const uint16_t* __restrict__ a, 
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
     const uint16_t* ab = a + (long)b * HW * C + 8 * cg;
 #pragma unroll 8
-    for (int p = sl; p < HW; p += S) {     // unrolled: the loads of 8 pixels in flight, added in pixel order
+    for (int p = sl < S ? sl : HW; p < HW; p += S) {     // unrolled: the loads of 8 pixels in flight, added in pixel order
         const uint4 v = *reinterpret_cast<const uint4*>(ab + (long)p * C);
         const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] += b2f(h[e]);
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) red[sl * C + 8 * cg + e] = acc[e];
+    for (int e = 0; e < 8; ++e)
+        if (sl < S) red[sl * C + 8 * cg + e] = acc[e];
     __syncthreads();
     for (int c = t; c < C; c += 1024) {
         float v = 0.0f;
@@ -2124,12 +2132,14 @@ extern "C" int bz_nn_head(const uint16_t* a, const float* fw, const float* fb, f
                           int C, int nout, void* stream) {
     BZ_REQUIRE(a && fw && fb && gap && out && B > 0 && HW > 0 && C > 0 && C <= 4096 && nout > 0,
                "bz_nn_head: bad arguments");
-    if (C % 8 == 0 && 256 % (C / 8) == 0)
-        hipLaunchKernelGGL(k_head8, dim3(B), dim3(1024), (1024 / (C / 8) + 1) * C * sizeof(float), (hipStream_t)stream,
-                           a, fw, fb, gap, out, HW, C, nout);
-    else
+    if (C % 8 == 0 && 256 % (C / 8) == 0) {
+        const int S = head_slices(HW, C);
+        hipLaunchKernelGGL(k_head8, dim3(B), dim3(1024), (S + 1) * C * sizeof(float), (hipStream_t)stream, a, fw, fb, gap,
+                           out, HW, C, nout, S);
+    } else {
         hipLaunchKernelGGL(k_head, dim3(B), dim3(256), C * sizeof(float), (hipStream_t)stream, a, fw, fb, gap, out, HW,
                            C, nout);
+    }
     BZ_CHECK_LAUNCH("bz_nn_head");
     return BZ_OK;
 }
