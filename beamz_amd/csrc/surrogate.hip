@@ -209,7 +209,7 @@ __device__ __forceinline__ void to_lds(__amdgpu_buffer_rsrc_t r, uint16_t* lds, 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
 }
 
-template <int WM, int WN, int MI, int NI, int ST>
+template <int WM, int WN, int MI, int NI, int ST, bool CF>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* __restrict__ src,
                                                             const uint16_t* __restrict__ wk,
                                                             const float* __restrict__ bias, uint16_t* __restrict__ out,
@@ -224,10 +224,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
     __shared__ __attribute__((aligned(16))) uint16_t A2[ST == 4 ? BM * 64 : 8], A3[ST == 4 ? BM * 64 : 8],
         B2[ST == 4 ? BN * 64 : 8], B3[ST == 4 ? BN * 64 : 8];
     // consecutive pixel tiles, which share input rows, on one XCD
-    const int tile = ((int)blockIdx.x % 8) * per_xcd + (int)blockIdx.x / 8;
+    // (CF: the channel blocks of a pixel tile one after the other, so that its input rows are read from memory once)
+    const int q = CF ? (int)(blockIdx.y * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x / 8;
+    const int tile = ((int)blockIdx.x % 8) * per_xcd + (CF ? q / (int)gridDim.y : q);
     if (tile >= mtiles) return;
     const int P = g.B * g.H * g.W, K = 9 * Cs;
-    const int m0 = tile * BM, n0 = blockIdx.y * BN;
+    const int m0 = tile * BM, n0 = (CF ? q % (int)gridDim.y : (int)blockIdx.y) * BN;
     const int t = threadIdx.x, l = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(src), 0, (int)((uint32_t)P * (uint32_t)Cs * 2u),
                                                       0x00020000);
@@ -1707,12 +1709,12 @@ static bool conv_march(const uint16_t* src, const uint16_t* wk, const float* bia
     return true;
 }
 
-template <int WM, int WN, int MI, int NI, int ST>
+template <int WM, int WN, int MI, int NI, int ST, bool CF = false>
 static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out,
                         const uint16_t* mask, const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
     const long P = (long)g.B * g.H * g.W;
     const int mt = (int)((P + 32 * MI * WM - 1) / (32 * MI * WM)), per_xcd = (mt + 7) / 8;
-    hipLaunchKernelGGL((k_conv_tile<WM, WN, MI, NI, ST>), dim3(per_xcd * 8, Cout / (32 * NI * WN)), dim3(64 * WM * WN), 0,
+    hipLaunchKernelGGL((k_conv_tile<WM, WN, MI, NI, ST, CF>), dim3(per_xcd * 8, Cout / (32 * NI * WN)), dim3(64 * WM * WN), 0,
                        st, src, wk, bias, out, mask, g, Cin, Cout, sign, relu, mt, per_xcd);
 }
 
@@ -1720,7 +1722,8 @@ static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bi
 // offsets. Tiles of 128 x 128 while they give every CU one (16 x 16 x 256 -> 256: batch 128 43 us, 64-wide ones 55;
 // at batch 16, 64 tiles, 21 against 15), then 128 x 64 on the same terms (64 x 64 x 64 -> 64, batch 128: 60 us,
 // 64 x 64 tiles 67), then 64 x 64 (16 x 16 x 256 -> 256, batch 16: 14 us, 128 x 64 tiles 15). 32-channel remainders
-// take 128 x 32, except 64-pixel rows in numbers that fill the row march (64 -> 32 channels: batch 128 36 us against
+// take 128 x 32 with the channel blocks of a pixel tile one after the other (past 4 MB of input per XCD each block read
+// the whole input from memory again: 32 x 32 256 -> 288, batch 128, 681 us, so 268), except 64-pixel rows in numbers that fill the row march (64 -> 32 channels: batch 128 36 us against
 // 42 here, batch 16 30 against 9). Where a CU gets one tile at most, nothing runs beside its barriers: three slices
 // in flight there (16 x 16 256 -> 256, batch 16: 15 -> 11 us, 256 -> 128, batch 128: 30 -> 23), one where two or more
 // tiles share a CU and the LDS (64 x 64 64 -> 64, batch 128: 63 us, 93 with three).
@@ -1731,7 +1734,7 @@ static bool conv_tile(const uint16_t* src, const uint16_t* wk, const float* bias
     const long P = (long)g.B * g.H * g.W, mt = (P + 127) / 128;
     if (Cout % 64) {
         if (g.W == 64 && Cin == 64 && (long)g.B * g.H / 16 * (Cout / 32) >= 512) return false;
-        launch_tile<4, 1, 1, 1, 2>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
+        launch_tile<4, 1, 1, 1, 2, true>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     } else if (Cout % 128 == 0 && mt * (Cout / 128) >= 256) {
         (mt * (Cout / 128) > 256 ? launch_tile<2, 4, 2, 1, 2> : launch_tile<2, 4, 2, 1, 4>)(
             src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
