@@ -1723,17 +1723,21 @@ static void launch_tile(const uint16_t* src, const uint16_t* wk, const float* bi
 // at batch 16, 64 tiles, 21 against 15), then 128 x 64 on the same terms (64 x 64 x 64 -> 64, batch 128: 60 us,
 // 64 x 64 tiles 67), then 64 x 64 (16 x 16 x 256 -> 256, batch 16: 14 us, 128 x 64 tiles 15). 32-channel remainders
 // take 128 x 32 with the channel blocks of a pixel tile one after the other (past 4 MB of input per XCD each block read
-// the whole input from memory again: 32 x 32 256 -> 288, batch 128, 681 us, so 268), except 64-pixel rows in numbers that fill the row march (64 -> 32 channels: batch 128 36 us against
-// 42 here, batch 16 30 against 9). Where a CU gets one tile at most, nothing runs beside its barriers: three slices
-// in flight there (16 x 16 256 -> 256, batch 16: 15 -> 11 us, 256 -> 128, batch 128: 30 -> 23), one where two or more
-// tiles share a CU and the LDS (64 x 64 64 -> 64, batch 128: 63 us, 93 with three).
+// the whole input from memory again: 32 x 32 256 -> 288, batch 128, 681 us, so 268). The row march keeps 64-pixel rows of
+// 64 input channels where they fill it and the output is a remainder (64 -> 160, batch 16 x 100 rows: 37.8 us, 39.6
+// here; batch 16 x 64 rows 35.9 and 26.4), and 64 -> 64 once the tensors outgrow the 256 MB Infinity Cache (64 rows:
+// batch 256, 268 MB, 124 us against 114 here, batch 400, 420 MB, 190 against 204).
+// Where a CU gets one tile at most, nothing runs beside its barriers: three slices in flight there (16 x 16 256 -> 256,
+// batch 16: 15 -> 11 us, 256 -> 128, batch 128: 30 -> 23), one where two or more tiles share a CU and the LDS (64 x 64
+// 64 -> 64, batch 128: 63 us, 93 with three).
 static bool conv_tile(const uint16_t* src, const uint16_t* wk, const float* bias, uint16_t* out, const uint16_t* mask,
                       const Geo& g, int Cin, int Cout, int sign, int relu, hipStream_t st) {
     const uintptr_t all = (uintptr_t)src | (uintptr_t)wk | (uintptr_t)out | (uintptr_t)mask;
     if (Cin % 64 || (all & 15) || 18L * Cin * Cout >= (1L << 31)) return false;
     const long P = (long)g.B * g.H * g.W, mt = (P + 127) / 128;
+    if (g.W == 64 && Cin == 64 && Cout == 64 && 2 * P * (Cin + Cout * (mask ? 2 : 1)) > 300000000L) return false;
     if (Cout % 64) {
-        if (g.W == 64 && Cin == 64 && (long)g.B * g.H / 16 * (Cout / 32) >= 512) return false;
+        if (g.W == 64 && Cin == 64 && (long)g.B * g.H / 16 * (Cout / 32) >= 448) return false;
         launch_tile<4, 1, 1, 1, 2, true>(src, wk, bias, out, mask, g, Cin, Cout, sign, relu, st);
     } else if (Cout % 128 == 0 && mt * (Cout / 128) >= 256) {
         (mt * (Cout / 128) > 256 ? launch_tile<2, 4, 2, 1, 2> : launch_tile<2, 4, 2, 1, 4>)(
