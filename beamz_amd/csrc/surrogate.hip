@@ -1894,8 +1894,8 @@ static void tree_sum2(const SumSeg& a, const SumSeg& b, float* scratch, hipStrea
 // sums to write and read back (about 2048 workgroups, at most 8 M (64- and 128-pixel rows) or 16 M partial floats,
 // measured at batch 128, us with the sums, before / after: 16 x 16 256 -> 256 97 / 80, 128 -> 256 63 / 49, 32 x 32
 // 128 -> 128 83 / 68). Fewer blocks keep that older count, whose partial rows the tests of the ordered sums are
-// written for, raised to one workgroup per place with bands of 4 rows for rows of 64 and more pixels (64 x 64
-// 64 -> 64, batch 16: 30 us with 16-row bands, 25 with 4). Halving some bands so that every place gets the same
+// written for, raised to one workgroup per place, at most 256, with bands of 4 rows for rows of 64 and more pixels
+// (64 x 64 64 -> 64, batch 16: 30 us with 16-row bands, 25 with 4; 32 -> 32, batch 64: 28 us, 34 with 512 bands). Halving some bands so that every place gets the same
 // number of rows measured slower than equal ones (56 -> 59 us at 32 x 32 64 -> 128).
 struct MarchPlan {
     bool ok;
@@ -1919,7 +1919,7 @@ inline MarchPlan march_plan(int B, int H, int W, int Ci, int Co) {
     } else {
         nz = std::min(2048 / nblk, std::max(1L, rows / 16));
         nz = std::min(nz, std::max(1L, (W >= 64 ? 8L << 20 : 16L << 20) / nw));
-        if (W >= 64) nz = std::max(nz, std::min(places, rows / 4));
+        if (W >= 64) nz = std::max(nz, std::min({places, 256L, rows / 4}));
     }
     long band = (rows + nz - 1) / nz;
     band = (band + R - 1) / R * R;

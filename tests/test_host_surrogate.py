@@ -38,3 +38,14 @@ def test_chunk_density_generator_equals_the_per_map_one():
         assert b.dtype == bool and b.shape == (m, n, n)
         assert np.array_equal(a, b)
         assert np.array_equal(r1.random(4), r2.random(4))
+
+
+def test_weight_gradient_bands_of_one_channel_block():
+    """32 -> 32 channels on rows of 64 and more pixels: at most 256 bands where the map's rows are fewer than 16 times
+    that (512, a partial sum each, took 20 % longer), and one per four rows on small maps."""
+    from beamz_amd import _native as N
+    nw = 9 * 32 * 32
+    bands = lambda B, H, W: N.lib().bz_nn_wgrad_work(B, H, W, 32, 32, 32) / nw      # (and a few rows of the sums' tree)
+    for B, H, W in ((64, 64, 64), (32, 64, 64), (64, 48, 64), (24, 128, 128), (16, 128, 128)):
+        assert 256 <= bands(B, H, W) < 300, (B, H, W)
+    assert 16 <= bands(1, 64, 64) < 20 and 32 <= bands(1, 128, 128) < 40
