@@ -1119,7 +1119,7 @@ __global__ __launch_bounds__(256) void k_conv_first_wgrad8(const uint16_t* __res
 __global__ __launch_bounds__(256) void k_conv_first_rows(const uint16_t* __restrict__ x, const float* __restrict__ w,
                                                          const float* __restrict__ b, uint16_t* __restrict__ y,
                                                          Geo g, int Co, int RB) {
-    extern __shared__ float xs[];
+    extern __shared__ __attribute__((aligned(16))) float xs[];
     const int G = Co / 8, R = 256 / G;
     const int t = threadIdx.x, gi = t % G, r = t / G;
     const int c = 8 * gi;
@@ -1131,16 +1131,20 @@ __global__ __launch_bounds__(256) void k_conv_first_rows(const uint16_t* __restr
         const int yy = y0 + ry - 1, xx = rx - 1;
         xs[q] = (yy >= 0 && yy < g.H && xx >= 0 && xx < W) ? b2f(x[((long)bi * g.H + yy) * W + xx]) : 0.0f;
     }
-    float* wl = xs + (RB + 2) * WP;           // the weights once through LDS: a thread's 72 lie 9 apart in memory
-    for (int q = t; q < 9 * Co; q += 256) wl[q] = b2f(f2b(w[q]));
+    // the weights once through LDS, by tap: a thread's 72 lie 9 apart in memory, and there each tap's 8 in a row
+    float* wl = xs + (((RB + 2) * WP + 3) & ~3);
+    for (int q = t; q < 9 * Co; q += 256) wl[q % 9 * Co + q / 9] = b2f(f2b(w[q]));
     float wv[8][9], bv[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) bv[e] = b[c + e];
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap) wv[e][tap] = wl[(c + e) * 9 + tap];
+    for (int tap = 0; tap < 9; ++tap) {
+        const float4 lo = *reinterpret_cast<const float4*>(wl + tap * Co + c);
+        const float4 hi = *reinterpret_cast<const float4*>(wl + tap * Co + c + 4);
+        wv[0][tap] = lo.x, wv[1][tap] = lo.y, wv[2][tap] = lo.z, wv[3][tap] = lo.w;
+        wv[4][tap] = hi.x, wv[5][tap] = hi.y, wv[6][tap] = hi.z, wv[7][tap] = hi.w;
+    }
     uint16_t* __restrict__ yc = y + (long)row0 * W * Co + c;
     int ly = r / W, lx = r - (r / W) * W;
     for (int q = r; q < RB * W; q += R) {
@@ -2005,14 +2009,16 @@ extern "C" int bz_nn_conv_first(const uint16_t* x, const float* w, const float* 
                                 int Co, void* stream) {
     BZ_REQUIRE(x && w && b && y && B > 0 && H > 0 && W > 0 && Co > 0, "bz_nn_conv_first: bad arguments");
     Geo g{B, H, W};
-    // chunks of whole rows of one image take the row-staged kernel
-    // about 2048 pixels, or fewer where that gives less than four workgroups per CU (with the weights through LDS, batch 16: 18 ->
-    // 9.4 us, batch 128: 39 -> 36)
+    // chunks of whole rows of one image take the row-staged kernel: about 2048 pixels, or fewer where that gives less
+    // than four workgroups per CU (128 x 128 -> 32 channels, with the weights through LDS: batch 16 18 -> 8.3 us, batch
+    // 128 36 -> 32)
     int rb = std::max(1, std::min(H, 2048 / W));
     while (rb > 2 && (long)B * H / rb < 1024) rb /= 2;
     while (H % rb) --rb;
-    const size_t lds = ((size_t)(rb + 2) * (W + 2) + 9L * Co) * sizeof(float);
-    const bool rows_ok = Co % 8 == 0 && 256 % (Co / 8) == 0 && lds - 36L * Co <= 32768 && lds <= 65536 && ((uintptr_t)y & 15) == 0;
+    const size_t lds = ((((size_t)(rb + 2) * (W + 2) + 3) & ~(size_t)3) + 9L * Co) * sizeof(float);
+    // (2048 channels, whose weights do not fit: the kernel below, 258 us at 4 x 64 x 64 where this one took 560)
+    const bool rows_ok = Co % 8 == 0 && 256 % (Co / 8) == 0 && lds - 36L * Co <= 32768 && lds <= 65536 &&
+                         ((uintptr_t)y & 15) == 0;
     if (rows_ok)
         hipLaunchKernelGGL(k_conv_first_rows, dim3((unsigned)((long)B * H / rb)), dim3(256), lds, (hipStream_t)stream,
                            x, w, b, y, g, Co, rb);
