@@ -2076,11 +2076,13 @@ extern "C" int bz_nn_conv_first_bwd(const uint16_t* x, const uint16_t* gz, const
     BZ_CHECK_LAUNCH("bz_nn_conv_first_bwd(w)");
     if (gx) {
         // 32 channels, bands of up to 8 rows whose products leave room for three workgroups per CU (one row: up to 604
-        // pixels)
+        // pixels), and fewer rows than would leave a CU without a band: one map of 128 x 128, the whole call, 22 us with
+        // bands of 8 rows, 18 with one
         int rb = 8;
+        while (rb > 1 && (long)B * H / rb < 256) --rb;
         while (rb > 1 && (H % rb || 36L * (rb + 2) * (W + 2) > 49152)) --rb;
         const size_t lds = 36L * ((long)(rb + 2) * (W + 2) | 1);
-        if (Co == 32 && lds <= 65536 && ((uintptr_t)gz & 15) == 0)
+        if (Co == 32 && lds <= 65536 && ((uintptr_t)gz & 15) == 0 && (long)B * H / rb < (1L << 24))
             hipLaunchKernelGGL(k_conv_first_dgrad32, dim3((unsigned)((long)B * H / rb)), dim3(256), lds, st, gz, w, gx,
                                g, rb);
         else if (Co % 8 == 0 && Co <= 64 && ((uintptr_t)gz & 15) == 0)

@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,H,W", [(1, 1, 1), (2, 1, 5), (3, 3, 16), (2, 7, 17), (2, 16, 64), (1, 24, 128), (1, 6, 130),
-                                   (1, 5, 401), (1, 4, 604), (1, 4, 605)])
+                                   (1, 5, 401), (1, 4, 604), (1, 4, 605), (20, 128, 9), (300, 7, 3), (257, 8, 20),
+                                   (90, 18, 33)])
 def test_first_layer_input_gradient(hip, B, H, W):
     import torch
     C = 32
