@@ -19,8 +19,9 @@ extern "C" int bz_version(void) { return 100; }
 
 extern "C" int bz_abi_sizes(int* out, int n) {
     BZ_REQUIRE(out && n >= 0, "bz_abi_sizes: null pointer");
-    const int sizes[3] = {(int)sizeof(bz_sim2d), (int)sizeof(bz_adj2d), (int)sizeof(bz_box_source)};
-    for (int q = 0; q < n && q < 3; ++q) out[q] = sizes[q];
+    const int sizes[4] = {(int)sizeof(bz_sim2d), (int)sizeof(bz_adj2d), (int)sizeof(bz_box_source),
+                          (int)sizeof(bz_gather_table)};
+    for (int q = 0; q < n && q < 4; ++q) out[q] = sizes[q];
     return BZ_OK;
 }
 

@@ -274,7 +274,8 @@ int bz_yee2d_run2(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles,
 int bz_yee2d_coef(const bz_sim2d* sims, int nsims, int max_cells, void* stream);
 
 /* Sizes of the descriptor structs as this library was compiled: out[0] = sizeof(bz_sim2d),
- * out[1] = sizeof(bz_adj2d), out[2] = sizeof(bz_box_source) (bindings check their own layouts). */
+ * out[1] = sizeof(bz_adj2d), out[2] = sizeof(bz_box_source), out[3] = sizeof(bz_gather_table), the first n of them
+ * (bindings check their own layouts). */
 int bz_abi_sizes(int* out, int n);
 
 /* K steps per pass: nlaunch launches of ksteps steps of the bz_yee2d_run step each (same results, bit for

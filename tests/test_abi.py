@@ -68,6 +68,14 @@ def test_descriptor_struct_layouts_match_the_library():
     assert list(out) == [C.sizeof(N.Sim2D), C.sizeof(N.Adj2D), C.sizeof(N.BoxSource)]
 
 
+def test_gather_table_layout_matches_the_library():
+    """The fourth size, of the monitor tables of a 3D run; entries past the known structs stay as they were."""
+    import ctypes as C
+    out = (C.c_int * 5)(*[-7] * 5)
+    N.call("bz_abi_sizes", out, 5)
+    assert list(out) == [C.sizeof(N.Sim2D), C.sizeof(N.Adj2D), C.sizeof(N.BoxSource), C.sizeof(N.GatherTable), -7]
+
+
 def test_kstep_owner_tables_give_each_point_one_owner():
     """Host tables of the K-step kernel: every monitor point is listed once, by the tile whose inner cells
     hold it, and its packed (region row, region column, component) decodes back to its grid cell."""
