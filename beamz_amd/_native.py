@@ -95,7 +95,7 @@ SIGNATURES = {
     "bz_yee2d_hz_runk": [vp, i32, vp, i32, i32, i32, i32, vp, i32, i32, vp, vp, vp, i32, vp, vp, i32, i32, vp, i32, vp,
                       vp, i32, vp],
     "bz_yee2d_runk_steps": [i32, vp, i32, vp, i32, i32, i32, i32, vp, i32, i32, vp, vp, vp, i32, vp, vp, i32, i32, vp,
-                            i32, vp, vp, i32, vp],
+                            i32, vp, vp, i32, i32, vp],
     "bz_adj2d_run": [vp, i32, vp, i32, i32, i32, i32, vp],
     "bz_adj2d_run2": [vp, i32, vp, i32, i32, vp, i32, i32, i32, i32, i32, vp],
     "bz_adj2d_runk": [vp, i32, vp, i32, i32, i32, i32, vp, i32, i32, i32, i32, i32, vp],

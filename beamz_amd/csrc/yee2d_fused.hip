@@ -706,7 +706,7 @@ __device__ __forceinline__ float src_term(float v, float amp) {
     return __float_as_uint(v) == 0x80000000u ? v : a;
 }
 
-constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further ones are read again every step)
+constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further ones are looked for again every step)
 
 // SEL: some simulation's source box holds several sources (bz_sim2d.src_sel); without it the per-cell
 // source lookup is compiled out.
@@ -719,21 +719,26 @@ constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further 
 // HZ: the (Hz, Ex, Ey) polarisation in the slots of (Ez, Hx, Hy). Its H update reads Ex of the next row and Ey of
 // the next column, its E update Hz of the previous row and column: the bands exchange Ex of the first row and Ex,
 // Ey of the last, and each keeps the Hz of the row above (with its source, which this family adds to Hz).
-template <int B, int KW, bool SEL, bool HZ>
-__global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)) void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
+// DENSE: many monitor points in a region: its waves leave their rows of all three components in LDS and, behind one
+// more barrier, the workgroup's threads share the entries (an instantiation of its own: it needs more registers, and its
+// 48 KB of samples allow two workgroups per CU). Otherwise the wave whose rows hold them takes them, without a barrier.
+template <int B, int KW, bool SEL, bool HZ, bool DENSE>
+__global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ || DENSE ? 4 : 6) : 1))
+void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                                                         const int* __restrict__ tiles, int ntiles, int P, int K,
                                                         const int* __restrict__ step, int q, int rd,
                                                         const int* __restrict__ ent_start,
                                                         const int* __restrict__ ents, float* __restrict__ stage_all,
                                                         Gather2D G) {
     constexpr int RH = KW * B;
-    __shared__ float xe[2][HZ ? 3 : 2][KW][LANES];   // [step parity][first, last row of a band]: its Ez (HZ: Ex;
+    __shared__ float xe[2][HZ ? 3 : 2][DENSE ? KW - 1 : KW][LANES];   // [step parity][first, last row of a band]: its Ez (HZ: Ex;
                                                      // and its last row's Ey)
     __shared__ float amps[32];              // the signal's K <= 31 samples of this launch
     __shared__ float wsrc[KW][B + HZ][LANES];   // source weights of the cells of the waves that meet the box (HZ:
                                                 // row B is the row above the band)
     __shared__ SnapBox snq;
-    extern __shared__ float smp_all[];      // with monitor points: samples [KW][B][LANES], entries [KW][ELIST][2]
+    extern __shared__ float smp_all[];      // with monitor points: samples [KW][B][LANES], entries [KW][ELIST][2], or
+                                            // with dense ones samples [3][RH][LANES]
     const int npts = G.npts;
     const int t = blockIdx.x;
     if (t >= ntiles) {
@@ -810,7 +815,11 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
         }
         return seen;
     };
-    if (e1 > e0)
+    const bool many = DENSE && e1 > e0;         // (uniform over the workgroup)
+    const int ef = e0 + tid;
+    const int epnt = many && ef < e1 ? ents[2 * ef] : -1, ecode = many && ef < e1 ? ents[2 * ef + 1] : 0;
+    auto sample = [&](int code) { return smp_all[((code & 3) * RH + (code >> 10)) * LANES + ((code >> 2) & 255)]; };
+    if (!DENSE && e1 > e0)
         nmine = entries([&](int pos, int pnt, int loc) {
             if (pos < ELIST) list[pos] = make_int2(pnt, loc);
         });
@@ -854,7 +863,9 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
         }
     }
 
-    const int wd = min(w + 1, KW - 1), wu = max(w - 1, 0);   // edge waves read their own slot (stale rows)
+    // where a wave reads the next and the previous band's rows; edge waves read a slot of stale rows. (DENSE: without
+    // the two slots that no other wave reads, so that two workgroups of 64 x 64 regions fit a CU's LDS)
+    const int wd = DENSE ? min(w, KW - 2) : min(w + 1, KW - 1), wu = max(w - 1, 0);
     auto steps = [&](auto lossy_c, auto edge_c) {
         constexpr bool L = decltype(lossy_c)::value;
         constexpr int E = decltype(edge_c)::value;
@@ -916,9 +927,11 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
         }
         for (int k = 0; k < K; ++k) {
             auto x = xe[k & 1];
-            x[0][w][l] = HZ ? hx[0] : ez[0];
-            x[1][w][l] = HZ ? hx[B - 1] : ez[B - 1];
-            if (HZ) x[2][w][l] = hy[B - 1];
+            if (!DENSE || w > 0) x[0][DENSE ? w - 1 : w][l] = HZ ? hx[0] : ez[0];
+            if (!DENSE || w < KW - 1) {
+                x[1][w][l] = HZ ? hx[B - 1] : ez[B - 1];
+                if (HZ) x[2][w][l] = hy[B - 1];
+            }
             __syncthreads();
             if (k < klive) {
                 const float ezb = x[0][wd][l], ezg = x[1][wu][l];
@@ -1043,10 +1056,25 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
                     }
                 }
             }
+            if (DENSE && many) {
+                float* __restrict__ stage = stage_all + ((long)(q & 1) * P + k) * npts;
+                if (k < klive)
+#pragma unroll
+                    for (int r = 0; r < B; ++r) {
+                        const int o = (w * B + r) * LANES + l;
+                        smp_all[o] = ez[r];
+                        smp_all[RH * LANES + o] = hx[r];
+                        smp_all[2 * RH * LANES + o] = hy[r];
+                    }
+                // (the next step's writes come after its barrier, which every thread reaches after these reads)
+                __syncthreads();
+                if (epnt >= 0) gstore(stage, epnt, sample(ecode));
+                for (int e = ef + LANES * KW; e < e1; e += LANES * KW) gstore(stage, ents[2 * e], sample(ents[2 * e + 1]));
+            }
             // monitor samples of step n0+k: the wave's rows of one component after the other go through its own LDS
             // rows, and the lanes read their entries' cells back between them (no workgroup barrier and no wait in
             // between: a wave's LDS operations complete in order)
-            if (E == 2 && nmine > 0) {
+            if (!DENSE && E == 2 && nmine > 0) {
                 float* __restrict__ stage = stage_all + ((long)(q & 1) * P + k) * npts;
                 for (int eb = 0; eb < min(nmine, ELIST); eb += LANES) {
                     const int2 ent = list[min(eb + l, nmine - 1)];
@@ -1110,17 +1138,20 @@ __global__ __launch_bounds__(LANES* KW, B == 4 ? 8 : (B == 8 ? (HZ ? 4 : 6) : 1)
 // nlaunch launches of P steps, then one of `part` (0: none).
 template <int B, int KW, bool HZ>
 int runk(const bz_sim2d* sims, const int* tiles, int ntiles, int P, int* step, int rd0, int nlaunch, int part,
-         const int* ent_start, const int* ents, float* stage, const Gather2D& G, bool sel, hipStream_t st) {
+         const int* ent_start, const int* ents, float* stage, const Gather2D& G, bool sel, bool dense, hipStream_t st) {
     const dim3 b(LANES, KW);
-    // sample staging and entry lists in LDS, only when there are monitor points
-    const size_t lds = G.npts > 0 ? (size_t)KW * (B * LANES * sizeof(float) + ELIST * sizeof(int2)) : 0;
+    // sample staging (and entry lists) in LDS, only when there are monitor points
+    const size_t lds = G.npts == 0 ? 0
+                       : dense     ? 3u * KW * B * LANES * sizeof(float)
+                                   : (size_t)KW * (B * LANES * sizeof(float) + ELIST * sizeof(int2));
     const long gather_threads = (long)G.npts * (G.nfreq > 0 ? G.nfreq : 1);
     const int gather_blocks = (int)((gather_threads + LANES * KW - 1) / (LANES * KW));
     const int total = nlaunch + (part > 0);
     // the gather of launch q-1 runs as extra workgroups of launch q; the last launch's gets a launch of its own
     for (int q = 0; q < total; ++q) {
         const dim3 g(ntiles + (q > 0 && G.npts > 0 ? gather_blocks : 0));
-        const auto kern = sel ? k_yee2d_tbk<B, KW, true, HZ> : k_yee2d_tbk<B, KW, false, HZ>;
+        const auto kern = dense ? (sel ? k_yee2d_tbk<B, KW, true, HZ, true> : k_yee2d_tbk<B, KW, false, HZ, true>)
+                                : (sel ? k_yee2d_tbk<B, KW, true, HZ, false> : k_yee2d_tbk<B, KW, false, HZ, false>);
         hipLaunchKernelGGL(kern, g, b, lds, st, sims, tiles, ntiles, P, q < nlaunch ? P : part, step, q, (rd0 + q) & 1,
                            ent_start, ents, stage, G);
         BZ_CHECK_LAUNCH("bz_yee2d_runk(steps)");
@@ -1246,7 +1277,7 @@ template <bool HZ>
 static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows,
                      int waves, int ksteps, int* step, int rd0, int nlaunch, int part, const int* ent_start,
                      const int* ents, float* stage, int npts, const int* slot, const int* grp, int nslot, int nrow,
-                     float* series, int nfreq, const double* phasor, double* dft, int src_sel, void* stream) {
+                     float* series, int nfreq, const double* phasor, double* dft, int src_sel, int dense, void* stream) {
     BZ_REQUIRE(sims && nsims > 0 && tiles && ntiles > 0 && step && nlaunch >= 0 && (rd0 == 0 || rd0 == 1),
                name + ": bad arguments");
     const int shape = rows * 100 + waves;
@@ -1275,7 +1306,8 @@ static int runk_call(const std::string& name, const bz_sim2d* sims, int nsims, c
     const hipStream_t st = (hipStream_t)stream;
     if (npts == 0) ent_start = ents = nullptr;
 #define BZ_RUNK(R, W) \
-    runk<R, W, HZ>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, part, ent_start, ents, stage, G, src_sel != 0, st)
+    runk<R, W, HZ>(sims, tiles, ntiles, ksteps, step, rd0, nlaunch, part, ent_start, ents, stage, G, src_sel != 0, \
+                   dense && npts > 0, st)
     switch (shape) {
         case 804: return BZ_RUNK(8, 4);
         case 808: return BZ_RUNK(8, 8);
@@ -1294,7 +1326,7 @@ extern "C" int bz_yee2d_runk(const bz_sim2d* sims, int nsims, const int* tiles, 
                              void* stream) {
     return runk_call<false>("bz_yee2d_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, 0,
                             ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
-                            stream);
+                            1, stream);
 }
 
 extern "C" int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
@@ -1304,19 +1336,19 @@ extern "C" int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tile
                                 void* stream) {
     return runk_call<true>("bz_yee2d_hz_runk", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nlaunch, 0,
                            ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
-                           stream);
+                           1, stream);
 }
 
 extern "C" int bz_yee2d_runk_steps(int hz, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows,
                                    int waves, int ksteps, int* step, int rd0, int nsteps, const int* ent_start,
                                    const int* ents, float* stage, int npts, const int* slot, const int* grp, int nslot,
                                    int nrow, float* series, int nfreq, const double* phasor, double* dft, int src_sel,
-                                   void* stream) {
+                                   int dense, void* stream) {
     BZ_REQUIRE(ksteps >= 1 && nsteps >= 0, "bz_yee2d_runk_steps: bad step counts");
     return (hz ? runk_call<true> : runk_call<false>)(
         "bz_yee2d_runk_steps", sims, nsims, tiles, ntiles, rows, waves, ksteps, step, rd0, nsteps / ksteps,
         nsteps % ksteps, ent_start, ents, stage, npts, slot, grp, nslot, nrow, series, nfreq, phasor, dft, src_sel,
-        stream);
+        dense != 0, stream);
 }
 
 extern "C" int bz_yee2d_coef(const bz_sim2d* sims, int nsims, int max_cells, void* stream) {

@@ -860,6 +860,7 @@ class Fused2D:
         self._pts_host = pts if plans else None
         self.kstep, self.krows, self.kwaves = 0, 8, 8
         self.tilesk = self.ent_start = self.ents = self.stagek = None
+        self.dense = False
         self.coefs = self.gcs = None
         self._coef_done = False
         if kstep is None and self.kstep_applies():
@@ -983,6 +984,10 @@ class Fused2D:
     # 800 x 400, 8 steps 84 / 58; alone (with the pass over the coefficients) 10 steps 50 / 36, at 1000 x 990 8 steps
     # 67 / 68 ((Hz, Ex, Ey): 69 / 79), 10 steps 82 / 71 (85 / 84)
     PART_MIN, PART_ALONE = 2, 10
+    # Most monitor entries (point and component) in the rows of one wave for which that wave takes the samples; above, the
+    # workgroup does. us/step by wave / by workgroup: 1024 x 1024, 3 columns (72 entries) 3.0 / 2.4, 12 (288) 21.9 / 3.0;
+    # 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two, not three, on many grids
+    DENSE_MIN = 64
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
     # (K, rows, waves) candidates of tune_kstep. Forward sweeps: 64 grids of 256 x 256 cells 4.95 / 5.05 us/step
     # for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 4.49 / 4.45; 16 grids of 600 x 600 cells
@@ -1059,9 +1064,12 @@ class Fused2D:
         self.tilesk = T.from_numpy(tiles.ravel()).to(self.dev)
         self.ntilesk = len(tiles)
         self.ent_start = self.ents = self.stagek = None
+        self.dense = False
         if self.npts:
             dims = np.array([(g.nx, g.ny, g.ld) for g in self.grids], np.int64)
             start, ents = kstep_owner_tables(tiles, self._pts_host, dims, K, rows * waves)
+            wave = np.repeat(np.arange(len(tiles)) * waves, np.diff(start)) + (ents[:, 1] >> 10) // rows
+            self.dense = bool(np.bincount(wave, minlength=1).max() > self.DENSE_MIN)
             self.ents = T.from_numpy(ents.ravel()).to(self.dev)
             self.ent_start = T.from_numpy(start).to(self.dev)
             self.stagek = T.zeros(2 * K * self.npts, dtype=T.float32, device=self.dev)   # two slots: q & 1
@@ -1224,7 +1232,7 @@ class Fused2D:
                self.tilesk.data_ptr(), self.ntilesk, self.krows, self.kwaves, self.kstep, self.step.data_ptr(), rd0,
                count, ptr(self.ent_start), ptr(self.ents), ptr(self.stagek), self.npts, ptr(self.slot), ptr(self.grp),
                self.nslot, self.nrow, ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft),
-               int(self.multi_src), self.grids[0].stream)
+               int(self.multi_src), int(self.dense), self.grids[0].stream)
 
     def _launch(self, count):
         ptr = lambda t: t.data_ptr() if t is not None else None

@@ -304,11 +304,13 @@ int bz_yee2d_hz_runk(const bz_sim2d* sims, int nsims, const int* tiles, int ntil
                      const double* phasor, double* dft, int src_sel, void* stream);
 
 /* nsteps steps by bz_yee2d_runk (hz nonzero: bz_yee2d_hz_runk) launches on the same lists: nsteps / ksteps launches of
- * ksteps steps and, where steps are left, one that advances those. Launch q reads buffer (rd0 + q) & 1. */
+ * ksteps steps and, where steps are left, one that advances those. Launch q reads buffer (rd0 + q) & 1. dense: how the
+ * samples are taken, with the same results: 0 by the wave whose rows hold them (fastest up to 64 entries of `ents` in
+ * one wave's rows, slow past 192), else by the whole workgroup (as bz_yee2d_runk and bz_yee2d_hz_runk do). */
 int bz_yee2d_runk_steps(int hz, const bz_sim2d* sims, int nsims, const int* tiles, int ntiles, int rows, int waves,
                         int ksteps, int* step, int rd0, int nsteps, const int* ent_start, const int* ents, float* stage,
                         int npts, const int* slot, const int* grp, int nslot, int nrow, float* series, int nfreq,
-                        const double* phasor, double* dft, int src_sel, void* stream);
+                        const double* phasor, double* dft, int src_sel, int dense, void* stream);
 
 /* ---------------- reverse-time 2D adjoint ----------------
  * No reference counterpart (the reference's gradient is the overlap heuristic of

@@ -136,3 +136,47 @@ def test_snapshots_of_the_last_steps_follow_the_launches(hip, count):
     assert not np.any(got[0][0] == -7.0)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+@pytest.mark.parametrize("dense", [0, 10 ** 9])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 4, 16), (12, 4, 8), (8, 8, 4), (3, 16, 4), (20, 8, 16)])
+def test_both_ways_of_sampling_give_the_bits_of_single_steps(hip, monkeypatch, shape, dense, pol):
+    """Monitor samples taken by the whole workgroup, and by the wave that holds them (here with more entries than its
+    list keeps), also in a launch of fewer steps than the list's."""
+    from beamz_amd.simulation.engine import Fused2D
+    monkeypatch.setattr(Fused2D, "DENSE_MIN", dense)
+    K, rows, waves = shape
+    steps = 2 * K + max(2, K - 1)
+    ref = run(steps, True, pol, kstep=0, pairs=False)
+    got = run(steps, True, pol, kstep=K, krows=rows, kwaves=waves, pairs=False)
+    for size, a, b in zip(SIZES, got, ref):
+        assert set(a) == set(b)
+        for k in b:
+            assert np.array_equal(a[k], b[k]), (size, k)
+
+
+def test_neighbouring_monitor_rows_are_not_slow(hip):
+    """Eight neighbouring rows of monitor points take no more than twice the time of one (once five times: entries past a
+    wave's list were looked for in the tile's again every step)."""
+    import time
+
+    import torch
+    best = []
+    for rows in (1, 8):
+        s, _ = world(400, 300, 1200, False, 1, "Ez")
+        s.monitors = [bz.Monitor(design=s.design, start=(0, (90 + q) * DX), end=(399 * DX, (90 + q) * DX),
+                                 dft_frequencies=[1.9e14], record_fields=False, accumulate_power=False)
+                      for q in range(rows)]
+        batch = FDTDBatch([s])
+        batch.initialize()
+        batch.advance(192)
+        times = []
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            batch.advance(192)
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+    assert best[1] < 2 * best[0], best

@@ -72,3 +72,17 @@ def test_pairs_take_the_steps_short_of_a_launch(calls):
     e.run(0, 23)
     assert [n for n, _ in calls] == ["bz_yee2d_coef", "bz_yee2d_runk_steps", "bz_yee2d_run2", "bz_yee2d_run"]
     assert calls[1][1][10] == 12
+
+
+@pytest.mark.parametrize("points,dense", [((), False), ([(j, 30) for j in range(40)], False),
+                                          ([(20, i) for i in range(21)], False), ([(20, i) for i in range(22)], True),
+                                          ([(j, i) for j in (20, 21) for i in range(70)], True)])
+def test_dense_monitor_points_are_those_past_one_entry_per_lane(points, dense):
+    """More than 64 entries (points times components) in the rows of one wave: the workgroup takes the samples."""
+    g = grid("Ez")
+    if points:
+        off = np.array([g.offset(0, j, i) for j, i in points])
+        comps = np.repeat(np.arange(3), len(off))
+        g.add_gather(comps, np.tile(off, 3), np.arange(8), np.arange(9.0), None)
+    e = Fused2D([g], kstep=8, krows=4, kwaves=16)
+    assert e.dense == dense
