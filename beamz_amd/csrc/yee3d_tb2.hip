@@ -47,6 +47,7 @@ namespace {
 constexpr int LANES = 64;
 constexpr int OXT = LANES - 4;   // stored columns per wave
 constexpr int NXCD = 8;
+constexpr int MANY_BOXES = 3;
 #define BZ_GLOBAL __attribute__((address_space(1)))
 
 struct Fields6 {
@@ -104,22 +105,34 @@ __device__ __forceinline__ void ecoef(float sig, float eps, const Coef& c, float
     cb = c.kbe * ie * r;
 }
 
+__device__ __forceinline__ void add_box(float& ex, float& ey, float& ez, int i, int j, int k, const bz_box_source& b,
+                                        float amp) {
+    const int a = i - b.x0, bb = j - b.y0, cc = k - b.z0;
+    if (a >= 0 && a < b.sx && bb >= 0 && bb < b.sy && cc >= 0 && cc < b.sz) {
+        const long rr = ((long)cc * b.sy + bb) * b.sx + a;
+        // (global, not flat, accesses, also where the pointers come from LDS)
+        const float m = b.mul ? ((const BZ_GLOBAL float*)b.mul)[rr] : 1.0f;
+        const float v = ((const BZ_GLOBAL float*)b.add)[rr] * amp;
+        // selects, not a component-indexed write (which would place ex, ey, ez in scratch memory)
+        ex = b.comp == 0 ? m * ex + v : ex;
+        ey = b.comp == 1 ? m * ey + v : ey;
+        ez = b.comp == 2 ? m * ez + v : ez;
+    }
+}
+
+// MANY: the boxes as kernel arguments, unrolled; else from LDS, one after the other.
+template <bool MANY>
 __device__ __forceinline__ void add_sources(float& ex, float& ey, float& ez, int i, int j, int k, const Boxes2& src,
                                             bool second) {
-#pragma unroll 1
-    for (int q = 0; q < src.n; ++q) {
-        const bz_box_source& b = src.b[q];
-        const int a = i - b.x0, bb = j - b.y0, cc = k - b.z0;
-        if (a >= 0 && a < b.sx && bb >= 0 && bb < b.sy && cc >= 0 && cc < b.sz) {
-            const long rr = ((long)cc * b.sy + bb) * b.sx + a;
-            // (global, not flat, accesses: the pointers come from LDS)
-            const float m = b.mul ? ((const BZ_GLOBAL float*)b.mul)[rr] : 1.0f;
-            const float v = ((const BZ_GLOBAL float*)b.add)[rr] * (second ? src.amp1[q] : b.amp);
-            // selects, not a component-indexed write (which would place ex, ey, ez in scratch memory)
-            ex = b.comp == 0 ? m * ex + v : ex;
-            ey = b.comp == 1 ? m * ey + v : ey;
-            ez = b.comp == 2 ? m * ez + v : ez;
+    if (MANY) {
+#pragma unroll
+        for (int q = 0; q < BZ_MAX_BOX; ++q) {
+            if (q >= src.n) break;
+            add_box(ex, ey, ez, i, j, k, src.b[q], second ? src.amp1[q] : src.b[q].amp);
         }
+    } else {
+#pragma unroll 1
+        for (int q = 0; q < src.n; ++q) add_box(ex, ey, ez, i, j, k, src.b[q], second ? src.amp1[q] : src.b[q].amp);
     }
 }
 
@@ -170,7 +183,7 @@ __device__ __forceinline__ void gather_prev(const Gather3D& G, const Fields6& S,
     a[1] = im;
 }
 
-template <int R, int W>
+template <int R, int W, bool MANY>
 __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, const float* __restrict__ eps,
                                                        const float* __restrict__ sig, int nx, int ny, int nz, int ld,
                                                        int kseg, int gx, int gy, int gz, int per_xcd, Coef c,
@@ -187,12 +200,16 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
 
     // the source boxes and the staging box, written before the first barrier and read after it by the few waves
     // and planes that meet them: as kernel arguments their 80 values sat in spilled scalar registers in every wave
-    __shared__ Boxes2 src;
+    // (MANY, three and more boxes: as arguments all the same, since one after the other from LDS each costs a chain of its
+    // own: us per pair with 4 boxes on one line, 39 from LDS and 35 as arguments at 120x72x40, 149 and 140 at 240x160x100
+    // with boxes of 31 cells a side; with 2 boxes 28 and 28, 72 and 82)
+    __shared__ Boxes2 src_lds;
     __shared__ Stage stg;
     if (threadIdx.x == 0 && threadIdx.y == 0) {
-        src = src_arg;
+        if (!MANY) src_lds = src_arg;
         stg = stg_arg;
     }
+    const Boxes2& src = MANY ? src_arg : src_lds;
 
     const int h = blockIdx.x;
     const int tile = (h % NXCD) * per_xcd + h / NXCD;
@@ -329,7 +346,7 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
                                ? ca * C.ey0[r] + cb * ((h1x[r] - C.h1x[r]) * rdz - (h1z[r] - hzL) * rdx)
                                : C.ey0[r];
                 float ezz = (kz && yin && xin) ? ca * ez[r] + cb * ((h1y[r] - hyL) * rdx - (h1x[r] - hxU) * rdy) : ez[r];
-                if (k >= sz0 && k < sz1) add_sources(ex, ey, ezz, i, j, k, src, false);
+                if (k >= sz0 && k < sz1) add_sources<MANY>(ex, ey, ezz, i, j, k, src, false);
                 e1x[r] = ex;
                 e1y[r] = ey;
                 e1z[r] = ezz;
@@ -402,7 +419,7 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
                 float ezz = (kz && yin && xin) ? ca * C.f1z[r] + cb * ((C.h2y[r] - hyL) * rdx - (C.h2x[r] - hxU) * rdy)
                                                : C.f1z[r];
                 if (kst && lane_out && j >= J0 + 2 && j < J0 + T - 2 && j < ny) {
-                    if (m2 >= sz0 && m2 < sz1) add_sources(ex, ey, ezz, i, j, m2, src, true);
+                    if (m2 >= sz0 && m2 < sz1) add_sources<MANY>(ex, ey, ezz, i, j, m2, src, true);
                     const uint32_t o = mp + ro[r];
                     put(D.p[0], o, ex);
                     put(D.p[1], o, ey);
@@ -456,7 +473,8 @@ int launch(const Fields6& S, const Fields6& D, const float* eps, const float* si
     const int per_xcd = (n + NXCD - 1) / NXCD;
     const long gt = (long)G.n * (G.nfreq > 0 ? G.nfreq : 1);
     const dim3 grid(per_xcd * NXCD + (unsigned)((gt + LANES * W - 1) / (LANES * W)));
-    hipLaunchKernelGGL((k_yee3d_tb2<R, W>), grid, dim3(LANES, W), 0, st, S, D, eps, sig, nx, ny, nz, ld, kseg, gx, gy,
+    const auto kern = bs.n >= MANY_BOXES ? k_yee3d_tb2<R, W, true> : k_yee3d_tb2<R, W, false>;
+    hipLaunchKernelGGL(kern, grid, dim3(LANES, W), 0, st, S, D, eps, sig, nx, ny, nz, ld, kseg, gx, gy,
                        gz, per_xcd, c, rdx, rdy, rdz, bs, stg, G);
     BZ_CHECK_LAUNCH("bz_yee3d_step2");
     return BZ_OK;
