@@ -202,7 +202,7 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
     // and planes that meet them: as kernel arguments their 80 values sat in spilled scalar registers in every wave
     // (MANY, three and more boxes: as arguments all the same, since one after the other from LDS each costs a chain of its
     // own: us per pair with 4 boxes on one line, 39 from LDS and 35 as arguments at 120x72x40, 149 and 140 at 240x160x100
-    // with boxes of 31 cells a side; with 2 boxes 28 and 28, 72 and 82)
+    // with wide boxes; with 3 boxes of a few cells 34 and 32, 84 and 92)
     __shared__ Boxes2 src_lds;
     __shared__ Stage stg;
     if (threadIdx.x == 0 && threadIdx.y == 0) {
