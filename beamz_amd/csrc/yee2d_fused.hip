@@ -731,9 +731,17 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                                                         const int* __restrict__ ents, float* __restrict__ stage_all,
                                                         Gather2D G) {
     constexpr int RH = KW * B;
+    // several sources in a box: a region that meets few of them stages their samples in LDS and takes its cells' from
+    // there. STAGED: not where eight rows of Ez a wave are bound by vector issue (1200 x 1200 cells, 8 sources: 6.6
+    // us/step staged, 6.4 read at each cell; 800 x 400 cells, 4 rows: 2.0 and 2.8; 256 x 256, Hz: 2.0 and 2.7).
+    // RBITS a row name a cell's source in one register; 15 sources in the dense form would keep two workgroups off a CU
+    constexpr bool STAGED = SEL && (B == 4 || (HZ && B == 8));
+    constexpr int RBITS = B == 4 && !DENSE ? 4 : 3, SRCS = STAGED ? (1 << RBITS) - 1 : 1;
     __shared__ float xe[2][HZ ? 3 : 2][DENSE ? KW - 1 : KW][LANES];   // [step parity][first, last row of a band]: its Ez (HZ: Ex;
                                                      // and its last row's Ey)
-    __shared__ float amps[32];              // the signal's K <= 31 samples of this launch
+    __shared__ float amps[SRCS][32];         // the signal's K <= 31 samples of this launch (STAGED: of each source that
+                                                // the region meets, in their order)
+    __shared__ uint32_t met[STAGED ? 8 : 1];       // those sources, one bit each
     __shared__ float wsrc[KW][B + HZ][LANES];   // source weights of the cells of the waves that meet the box (HZ:
                                                 // row B is the row above the band)
     __shared__ SnapBox snq;
@@ -793,7 +801,35 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
     // step loop would wait behind the snapshot and staging stores of the previous step (the vector memory
     // counter retires in order)
     const int tid = w * LANES + l;
-    if (tid < K) amps[tid] = S.signal ? gload(S.signal, n0 + tid) : 0.0f;
+    auto src_cell = [&](int r) {
+        const int a = i - S.src_x0, b = jb + r - S.src_y0;
+        return a >= 0 && a < S.src_sx && b >= 0 && b < S.src_sy ? (long)b * S.src_sx + a : -1L;
+    };
+    const bool sel = STAGED && S.src_sel;
+    int nsrc = 1;
+    if (sel) {                              // (uniform over the workgroup, as its barriers need)
+        if (tid < 8) met[tid] = 0;
+        __syncthreads();
+        if (src_band)
+#pragma unroll
+            for (int r = 0; r < B + HZ; ++r) {
+                const long o = src_cell(r < B ? r : -1);
+                if (o < 0) continue;
+                const int s = gload(S.src_sel, o), s0 = __builtin_amdgcn_readfirstlane(s);
+                const bool first = __builtin_amdgcn_mbcnt_hi((uint32_t)(__ballot(1) >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)__ballot(1), 0)) == 0;
+                if (first || s != s0)   // (one lane for the many with the first one's source)
+                    atomicOr(&met[s >> 5], 1u << (s & 31));
+            }
+        __syncthreads();
+        nsrc = 0;
+        for (int a = 0; a < 8; ++a)
+            for (uint32_t m = __builtin_amdgcn_readfirstlane(met[a]); m; m &= m - 1, ++nsrc)
+                if (nsrc < SRCS && nsrc % KW == w && l < K)
+                    amps[nsrc][l] = gload(S.signal, (long)(a * 32 + __builtin_ctz(m)) * S.src_sig_len + n0 + l);
+    } else if (tid < K) {
+        amps[0][tid] = S.signal ? gload(S.signal, n0 + tid) : 0.0f;
+    }
 
     // the monitor entries of the tile whose rows are this wave's, compacted into its LDS list: (sample slot,
     // (row * LANES + column) | comp << 16)
@@ -913,16 +949,21 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
         }
         // the source's weights of this wave's cells, loaded once, in LDS: -0, which as an addend changes no value,
         // outside its box, and a weight of zero as +0 (its product is added, NaN at an infinite amplitude)
-        const bool plain_src = E == 2 && src_band && !SEL && !S.src_mul;
-        auto src_cell = [&](int r) {
-            const int a = i - S.src_x0, b = jb + r - S.src_y0;
-            return a >= 0 && a < S.src_sx && b >= 0 && b < S.src_sy ? (long)b * S.src_sx + a : -1L;
-        };
+        const bool plain_src = E == 2 && src_band && nsrc <= SRCS && !S.src_mul && (!SEL || STAGED);
+        uint32_t ranks = 0;                 // STAGED: RBITS a row, the cell's source among the staged ones
         if (E == 2 && src_band) {
 #pragma unroll
             for (int r = 0; r < B + HZ; ++r) {
+                if (STAGED) __builtin_amdgcn_sched_barrier(0);  // (few registers at a time)
                 const long o = src_cell(r < B ? r : -1);
                 wsrc[w][r][l] = o >= 0 ? gload(S.src_add, o) + 0.0f : -0.0f;
+                if (sel && plain_src) {
+                    const int s = o >= 0 ? gload(S.src_sel, o) : 0;
+                    uint32_t n = __popc(met[s >> 5] & ((1u << (s & 31)) - 1));
+#pragma unroll 1
+                    for (int a = 0; a < 7; ++a) n += a < s >> 5 ? __popc(met[a]) : 0;
+                    ranks |= (o >= 0 ? n : 0) << RBITS * r;
+                }
             }
         }
         for (int k = 0; k < K; ++k) {
@@ -941,17 +982,20 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                 // a step's latency counts) read and multiplied here, off the step's chain
                 float add[B], amp = 0.0f;
                 // (four LDS reads at a time, then selects: no wait for each read in turn)
+                if (STAGED && E == 2) asm volatile("" : "+v"(ranks));  // (no row's LDS address is kept over the steps)
+                auto amp_of = [&](int r) { return amps[ranks >> RBITS * r & SRCS][k]; };
+                constexpr int AT = STAGED && (B > 4 || HZ) ? 1 : 4;
                 auto src_adds = [&](int r0) {
-                    float v[4];
+                    float v[AT];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = wsrc[w][r0 + r][l];
+                    for (int r = 0; r < AT; ++r) v[r] = wsrc[w][r0 + r][l];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        add[r0 + r] = src_term(v[r], amp);
+                    for (int r = 0; r < AT; ++r) {
+                        add[r0 + r] = src_term(v[r], STAGED ? amp_of(r0 + r) : amp);
                     }
                 };
-                if (E == 2 && src_band) amp = amps[k];
-                if (plain_src && B <= 4) src_adds(0);
+                if (E == 2 && src_band) amp = amps[0][k];
+                if (plain_src && B == AT) src_adds(0);
                 // H: the row above the band (its Hy, or Hz, only), then the band
                 if (HZ) {
                     const float hg = computed(upd_hz(L ? fag : 1.0f, L ? gbg : gb0, rdx, rdy, hyg, from_right(eyg), eyg,
@@ -1041,10 +1085,11 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                 if (plain_src) {
 #pragma unroll
                     for (int r = 0; r < B; ++r) {
-                        if (B > 4 && r % 4 == 0) src_adds(r);
+                        if (STAGED && B > AT) __builtin_amdgcn_sched_barrier(0);
+                        if (B > AT && r % AT == 0) src_adds(r);
                         ez[r] += add[r];
                     }
-                    if (HZ) hyg += src_term(wsrc[w][B][l], amp);
+                    if (HZ) hyg += src_term(wsrc[w][B][l], STAGED ? amp_of(B) : amp);
                 } else if (E == 2 && src_band) {
 #pragma unroll
                     for (int r = 0; r < B + HZ; ++r) {

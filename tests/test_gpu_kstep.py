@@ -180,3 +180,62 @@ def test_neighbouring_monitor_rows_are_not_slow(hip):
             times.append(time.perf_counter() - t0)
         best.append(min(times))
     assert best[1] < 2 * best[0], best
+
+
+@pytest.mark.parametrize("pol", ["Ez", "Hz"])
+@pytest.mark.parametrize("dense", [0, 10 ** 9])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 4, 16), (12, 4, 8)])
+@pytest.mark.parametrize("count", [2, 7, 8, 15, 16, 40])
+def test_several_sources_in_a_region(hip, monkeypatch, count, shape, dense, pol):
+    """Up to as many sources as a region stages in LDS, one more, and many: cells of all of them, of weight 0 and of no
+    source side by side, one signal with an infinite sample, over two launches."""
+    from beamz_amd.simulation.engine import Fused2D
+    monkeypatch.setattr(Fused2D, "DENSE_MIN", dense)
+    steps, K = 32, shape[0]
+    rng = np.random.default_rng(count)
+    cells = np.array([(j, i) for j in range(3, 30) for i in range(50, 90)])
+    own = rng.integers(0, count + 1, len(cells))              # count: no source
+    own[:count] = np.arange(count)
+    w = np.where(rng.random(len(cells)) < 0.2, 0.0, 0.1 + rng.random(len(cells)))
+    sigs = np.cos(0.3 * np.arange(steps) + np.arange(count)[:, None])
+    sigs[count - 1, 2 * K - 1] = np.inf
+    out = []
+    for k in (0, K):
+        s, mons = world(113, 64, steps, True, 3, pol)
+        s.initialize_simulation(save=False, live=False)
+        g = s.grid
+        g.kstep2d, g.krows2d, g.kwaves2d = k, shape[1], shape[2]
+        g.sources = []
+        for q in range(count):
+            g.add_point_source(g.names[0], cells[own == q], w[own == q], None, sigs[q])
+        g.run(0, 2 * K)
+        out.append({n: np.real(getattr(s, n)).copy() for n in g.names})
+        assert bool(g._f2d.kstep) == bool(k)
+    for n in out[0]:
+        assert np.any(out[0][n]) and np.array_equal(out[0][n], out[1][n], equal_nan=True), n
+
+
+def test_several_sources_are_not_slow(hip):
+    """Eight sources over a grid take no more than 1.45 times one (once 1.7: each cell read its own source's sample from
+    memory at the end of every step)."""
+    import time
+
+    import torch
+    batches = []
+    for n in (1, 8):
+        s, _ = world(800, 400, 2200, False, 1, "Ez")
+        s.monitors = []
+        s.sources = [bz.GaussianSource(position=((20 + 105 * (q % 7)) * DX, (20 + 45 * (q // 7)) * DX), width=DX / 4,
+                                       signal=np.cos(0.05 * np.arange(2200))) for q in range(n)]
+        batches.append(FDTDBatch([s]))
+        batches[-1].initialize()
+        batches[-1].advance(192)
+    best = [1e9, 1e9]
+    for _ in range(8):
+        for q, b in enumerate(batches):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            b.advance(192)
+            torch.cuda.synchronize()
+            best[q] = min(best[q], time.perf_counter() - t0)
+    assert best[1] < 1.45 * best[0], best
