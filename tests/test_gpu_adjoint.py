@@ -455,3 +455,52 @@ def test_the_k_step_sweep_reads_the_injection_table(hip, monkeypatch, shape, lin
         out.append(prob.gradient().cpu().numpy())
         assert prob._rs["tabled"]
     assert np.abs(out[0]).max() > 0 and np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("line", [((120, 20), (120, 150)), ((40, 140), (150, 30))])
+@pytest.mark.parametrize("wide", [1.0, 1.25])
+@pytest.mark.parametrize("shape", [(8, 8, 8), (12, 8, 8), (16, 4, 16), (12, 4, 8)])
+def test_k_step_gradients_over_several_regions_give_the_bits_of_single_steps(hip, shape, wide, line):
+    """180 x 170 cells, three regions and more along both axes and most of them without conductivity; the design box and
+    the monitor (a column, a diagonal) cross their seams, cells are square or not, the run is no whole number of launches:
+    forward and reverse sweeps of every K-step shape give the single steps' gradient, with the full history and with
+    checkpoints, with and without the gradient pass and the injection table."""
+    torch = hip
+    nx, ny, steps, box = 180, 170, 203, (50, 45, 80, 75)
+    K, rows, waves = shape
+    rng = np.random.default_rng(11)
+    eps = 1.5 + 3.0 * rng.random((ny, nx))
+    sig = np.zeros((ny, nx))
+    sig[:, :5] = sig[:, -5:] = 2e4
+    e_box = torch.from_numpy(eps[box[1]:box[1] + box[3], box[0]:box[0] + box[2]]).float().cuda()[None]
+    ref = None
+    for k, mode, gp, tab in ((0, "full", True, True),) + tuple(
+            (K, m, g, t) for m in ("full", "checkpoint") for g in (True, False) for t in (True, False)):
+        d = bz.Design(nx * DX * (1 + 1e-9), ny * DX * (1 + 1e-9), material=bz.Material(1.0), auto_pml=False)
+        t = np.arange(steps) * 0.99 * DX / (bz.LIGHT_SPEED * np.sqrt(2))
+        d += bz.GaussianSource(position=(60 * wide * DX, 62 * DX), width=DX / 4, signal=np.cos(0.1 * np.arange(steps)))
+        mon = bz.Monitor(design=d, start=(line[0][0] * wide * DX, line[0][1] * DX),
+                         end=(line[1][0] * wide * DX, line[1][1] * DX), dft_frequencies=[F0, 1.1 * F0],
+                         record_fields=False, accumulate_power=False)
+        d += mon
+        mesh = RegularGrid.from_arrays(d, eps, sig, DX)
+        mesh.dx = wide * DX
+        sim = bz.FDTD(mesh, time=t)
+        npts = len(mon.get_grid_points_2d(sim.dx, sim.dy))
+        c = np.exp(1j * np.arange(2 * npts)).reshape(2, npts)
+        prob = AdjointProblem2D([sim], [mon], c, box, checkpoint_every=51, pairs=False, kstep=k, snapshots=mode,
+                                gradient_pass=gp)
+        if not tab:
+            prob.INJ_TABLE_BYTES = 0
+        prob.forward(e_box)
+        if k:
+            prob.fwd.set_kstep(K, rows, waves)
+            prob.rec.set_kstep(K, rows, waves)
+            prob.forward(e_box)
+        g = prob.gradient().cpu().numpy()
+        assert prob._rs["tabled"] == tab and (prob.l2hist is not None) == gp
+        assert (prob.sims[0].grid.dx != prob.sims[0].grid.dy) == (wide != 1.0)
+        assert (prob.rec.kstep, prob.fwd.kstep) == (k, k)
+        ref = g if ref is None else ref
+        # (the diagonal's field reaches every design cell; the sweeps' seams are inside the box)
+        assert np.count_nonzero(g) > 0.9 * g.size and np.array_equal(g, ref), (k, mode, gp, tab)
