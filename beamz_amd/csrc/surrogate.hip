@@ -191,16 +191,16 @@ __device__ __forceinline__ uint4 keep_positive(uint4 v, const uint4& y) {
 // A workgroup of WM x WN waves computes TM = 32 MI WM pixels x TN = 32 NI WN channels, each wave MI x NI blocks of
 // 32 x 32, in slices of 64 input channels of one tap. Both operands of a slice go from memory into LDS without
 // registers (16 bytes per lane, 8 rows of 128 bytes per wave and instruction), those of the next ST - 1 slices in
-// flight while the current one's MFMAs run (ST 2 or 4 slots); a tap outside the image, or a pixel past the last, is an offset past the end of the buffer, which
-// the hardware reads as zeros. Rows are not padded (such a load writes 1 KB in a row): chunk c of row r sits in
-// place c ^ ((r >> 1) & 7), which puts the 16 rows of an operand read on distinct banks.
-// The MFMA takes the weights as its first operand: a lane holds one pixel and 4 consecutive channels in 4
-// accumulators; after an exchange with lane +-32 it stores 8 channels, 16 bytes, at once.
-// Bound by the matrix units' issue with 2 to 4 waves per SIMD (850 to 910 TFLOP/s on 16- and 32-pixel rows at 256 and
-// 128 channels, where a library's 8192^3 product reaches 1118); with 64 channels, whose 9 slices are soon over, by
-// filling and draining the pipeline. Batch 128, us, against 64 x 64 tiles staged through registers (the same bits):
-// 16 x 16, 256 -> 256 78 -> 43, 128 -> 256 38 -> 23; 32 x 32, 128 -> 128 69 -> 46, 64 -> 128 39 -> 28; 64 x 64,
-// 64 -> 64 73 -> 60 (row march). 8 waves of 64 x 32 per 128 x 128 tile rather than 4 of 64 x 64 (46 on the first).
+// flight while the current one's MFMAs run (ST 2 or 4 slots); a tap outside the image, or a pixel past the last, is an
+// offset past the end of the buffer, which the hardware reads as zeros. Rows are not padded (such a load writes 1 KB
+// in a row): chunk c of row r sits in place c ^ ((r >> 1) & 7), which puts the 16 rows of an operand read on distinct
+// banks. The MFMA takes the weights as its first operand: a lane holds one pixel and 4 consecutive channels in 4
+// accumulators; after an exchange with lane +-32 it stores 8 channels, 16 bytes, at once. Bound by the matrix units'
+// issue with 2 to 4 waves per SIMD (850 to 910 TFLOP/s on 16- and 32-pixel rows at 256 and 128 channels, where a
+// library's 8192^3 product reaches 1118); with 64 channels, whose 9 slices are soon over, by filling and draining the
+// pipeline. Batch 128, us, against 64 x 64 tiles staged through registers (the same bits): 16 x 16, 256 -> 256 78 ->
+// 43, 128 -> 256 38 -> 23; 32 x 32, 128 -> 128 69 -> 46, 64 -> 128 39 -> 28; 64 x 64, 64 -> 64 73 -> 60 (row march). 8
+// waves of 64 x 32 per 128 x 128 tile rather than 4 of 64 x 64 (46 on the first).
 constexpr uint32_t OUTSIDE = 0xFFFFFFF0u;      // past every buffer: their sizes are multiples of 128 bytes
 
 __device__ __forceinline__ uint32_t f2b2(float lo, float hi) { return (uint32_t)f2b(lo) | ((uint32_t)f2b(hi) << 16); }
@@ -263,7 +263,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
         for (int h = 0; h < NA; ++h)
             to_lds(rs, a + (wave * NA + h) * 512, (tapok[h] >> tap) & 1u ? pofs[h] + shift : OUTSIDE);
 #pragma unroll
-        for (int h = 0; h < NB; ++h) to_lds(rw, b + (wave * NB + h) * 512, s < slices ? wofs[h] + 128u * (uint32_t)s : OUTSIDE);
+        for (int h = 0; h < NB; ++h)
+            to_lds(rw, b + (wave * NB + h) * 512, s < slices ? wofs[h] + 128u * (uint32_t)s : OUTSIDE);
     };
     f32x16 acc[MI][NI];
 #pragma unroll
@@ -403,8 +404,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_conv_tile(const uint16_t* _
 // once per band and channel block. Wave w computes the 32-pixel block w % (W / 32) and the 32-channel block
 // w / (W / 32) of every row: MFMAs with M = pixels, N = output channels, K = input channels, nine taps of
 // CIN / 16 steps. With a mask (the forward input of a backward-data step, an activation after ReLU), outputs
-// where the mask is not positive are stored as 0: the ReLU derivative of the layer below, fused. A tap shifts whole pixels, so every fragment is one aligned 16-byte LDS read; pixel strides
-// of CIN + 8 and weight rows of 9 CIN + 8 elements put the 16 rows of a read on distinct banks.
+// where the mask is not positive are stored as 0: the ReLU derivative of the layer below, fused. A tap shifts whole
+// pixels, so every fragment is one aligned 16-byte LDS read; pixel strides of CIN + 8 and weight rows of 9 CIN + 8
+// elements put the 16 rows of a read on distinct banks.
 template <int W, int CIN, int CB, bool MASK>
 __global__ __launch_bounds__(64 * (W / 32) * (CB / 32)) void k_conv_march(const uint16_t* __restrict__ src,
                                                                           const uint16_t* __restrict__ wk,
@@ -1311,7 +1313,8 @@ __global__ __launch_bounds__(256) void k_conv_first_dgrad32(const uint16_t* __re
     uint16_t wb[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) wb[e] = col < 9 ? f2b(w[(kg + e) * 9 + col]) : (uint16_t)0;
-    const bf16x8 bw = __builtin_bit_cast(bf16x8, make_uint4(pack2(wb[0], wb[1]), pack2(wb[2], wb[3]), pack2(wb[4], wb[5]), pack2(wb[6], wb[7])));
+    const bf16x8 bw = __builtin_bit_cast(bf16x8, make_uint4(pack2(wb[0], wb[1]), pack2(wb[2], wb[3]),
+                                                            pack2(wb[4], wb[5]), pack2(wb[6], wb[7])));
     __syncthreads();
     const int ya = max(y0 - 1, 0), yb = min(y0 + RB, g.H - 1);       // the band's rows and those beside it
     const int n = (yb - ya + 1) * W;
@@ -1899,8 +1902,9 @@ static void tree_sum2(const SumSeg& a, const SumSeg& b, float* scratch, hipStrea
 // measured at batch 128, us with the sums, before / after: 16 x 16 256 -> 256 97 / 80, 128 -> 256 63 / 49, 32 x 32
 // 128 -> 128 83 / 68). Fewer blocks keep that older count, whose partial rows the tests of the ordered sums are
 // written for, raised to one workgroup per place, at most 256, with bands of 4 rows for rows of 64 and more pixels
-// (64 x 64 64 -> 64, batch 16: 30 us with 16-row bands, 25 with 4; 32 -> 32, batch 64: 28 us, 34 with 512 bands). Halving some bands so that every place gets the same
-// number of rows measured slower than equal ones (56 -> 59 us at 32 x 32 64 -> 128).
+// (64 x 64 64 -> 64, batch 16: 30 us with 16-row bands, 25 with 4; 32 -> 32, batch 64: 28 us, 34 with 512 bands).
+// Halving some bands so that every place gets the same number of rows measured slower than equal ones (56 -> 59 us at
+// 32 x 32 64 -> 128).
 struct MarchPlan {
     bool ok;
     int nco, nci, rows_per_step, nz, band;

@@ -737,8 +737,8 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
     // RBITS a row name a cell's source in one register; 15 sources in the dense form would keep two workgroups off a CU
     constexpr bool STAGED = SEL && (B == 4 || (HZ && B == 8));
     constexpr int RBITS = B == 4 && !DENSE ? 4 : 3, SRCS = STAGED ? (1 << RBITS) - 1 : 1;
-    __shared__ float xe[2][HZ ? 3 : 2][DENSE ? KW - 1 : KW][LANES];   // [step parity][first, last row of a band]: its Ez (HZ: Ex;
-                                                     // and its last row's Ey)
+    // [step parity][first, last row of a band]: its Ez (HZ: Ex; and its last row's Ey)
+    __shared__ float xe[2][HZ ? 3 : 2][DENSE ? KW - 1 : KW][LANES];
     __shared__ float amps[SRCS][32];         // the signal's K <= 31 samples of this launch (STAGED: of each source that
                                                 // the region meets, in their order)
     __shared__ uint32_t met[STAGED ? 8 : 1];       // those sources, one bit each
@@ -1114,7 +1114,8 @@ void k_yee2d_tbk(const bz_sim2d* __restrict__ sims,
                 // (the next step's writes come after its barrier, which every thread reaches after these reads)
                 __syncthreads();
                 if (epnt >= 0) gstore(stage, epnt, sample(ecode));
-                for (int e = ef + LANES * KW; e < e1; e += LANES * KW) gstore(stage, ents[2 * e], sample(ents[2 * e + 1]));
+                for (int e = ef + LANES * KW; e < e1; e += LANES * KW)
+                    gstore(stage, ents[2 * e], sample(ents[2 * e + 1]));
             }
             // monitor samples of step n0+k: the wave's rows of one component after the other go through its own LDS
             // rows, and the lanes read their entries' cells back between them (no workgroup barrier and no wait in

@@ -200,9 +200,9 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
 
     // the source boxes and the staging box, written before the first barrier and read after it by the few waves
     // and planes that meet them: as kernel arguments their 80 values sat in spilled scalar registers in every wave
-    // (MANY, three and more boxes: as arguments all the same, since one after the other from LDS each costs a chain of its
-    // own: us per pair with 4 boxes on one line, 39 from LDS and 35 as arguments at 120x72x40, 149 and 140 at 240x160x100
-    // with wide boxes; with 3 boxes of a few cells 34 and 32, 84 and 92)
+    // (MANY, three and more boxes: as arguments all the same, since one after the other from LDS each costs a chain of
+    // its own: us per pair with 4 boxes on one line, 39 from LDS and 35 as arguments at 120x72x40, 149 and 140 at
+    // 240x160x100 with wide boxes; with 3 boxes of a few cells 34 and 32, 84 and 92)
     __shared__ Boxes2 src_lds;
     __shared__ Stage stg;
     if (threadIdx.x == 0 && threadIdx.y == 0) {
@@ -238,7 +238,8 @@ __global__ __launch_bounds__(LANES* W) void k_yee3d_tb2(Fields6 S, Fields6 D, co
 
     // planes on which this wave's rows and columns can meet a source, or the staging box (empty: never)
     const int wr = __builtin_amdgcn_readfirstlane(jb), wx = tx * OXT - 2;
-    const bool src_xy = src_arg.n > 0 && wr < src_arg.y1 && wr + R > src_arg.y0 && wx < src_arg.x1 && wx + LANES > src_arg.x0;
+    const bool src_xy = src_arg.n > 0 && wr < src_arg.y1 && wr + R > src_arg.y0 && wx < src_arg.x1 &&
+                        wx + LANES > src_arg.x0;
     const int sz0 = src_xy ? src_arg.z0 : 0, sz1 = src_xy ? src_arg.z1 : 0;
     const bool stg_xy = stg_arg.p && wr < stg_arg.y0 + stg_arg.sy && wr + R > stg_arg.y0 &&
                         wx < stg_arg.x0 + stg_arg.sx && wx + LANES > stg_arg.x0;
@@ -620,8 +621,9 @@ extern "C" int bz_yee3d_run2(float* const src[6], float* const dst[6], const flo
                           G.phasor0, G.phasor1, G.dft, stream);
     };
     // One call, since a pair on a small grid is shorter than its two Python calls were (33 us at 120x72x40; now 20 per
-    // pair with the samples). With one table, pair q - 1's samples are taken by extra workgroups of pair q's launch: its first step sits in
-    // the staging slot that launch does not write, its second step in the buffer that launch only reads
+    // pair with the samples). With one table, pair q - 1's samples are taken by extra workgroups of pair q's launch:
+    // its first step sits in the staging slot that launch does not write, its second step in the buffer that launch
+    // only reads
     for (int q = 0; q < npairs; ++q) {
         for (int k = 0; k < nbox; ++k) {
             bs.b[k].amp = amps[(long)2 * q * nbox + k];

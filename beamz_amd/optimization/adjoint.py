@@ -411,9 +411,9 @@ class AdjointProblem2D:
                         e1.record()
                         T.cuda.synchronize(self.dev)
                         ms[shape] = min(ms.get(shape, 1e30), e0.elapsed_time(e1))
-                # within 3 % of the fastest, the most steps per launch wins: on 16 designs of 600 x 600 cells,
-                # 192-step windows time K = 6 about 1.5 % faster than K = 8, while whole 3000-step sweeps with
-                # K = 8 took 68.0-69.3 ms per gradient against 68.8-72.8 ms with K = 6
+                # within 3 % of the fastest, the most steps per launch wins: a window of 192 steps favours fewer steps
+                # per launch a little against whole sweeps (16 designs of 600 x 600 cells: about 1.5 % between two
+                # shapes of which the other was 0 to 5 % faster over 3000 steps)
                 best = min(ms.values())
                 self.rec.set_kstep(*max((c for c in ms if ms[c] <= 1.03 * best), key=lambda c: (c[0], -ms[c])))
                 self.rev_timings = ms

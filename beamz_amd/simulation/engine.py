@@ -138,7 +138,9 @@ class Grid:
             if self.kernel == "fused" and self.tb2:
                 return (f"bz_yee3d_step2 (two steps per pass, {self.waves2} waves x {self.rows2} rows, "
                         f"{self.kseg2_eff()}-plane segments)")
-            return f"bz_yee3d_step (fused z-march, {self.rows} rows/wave)" if self.kernel == "fused" else "bz_update_3d (two-pass)"
+            if self.kernel != "fused":
+                return "bz_update_3d (two-pass)"
+            return f"bz_yee3d_step (fused z-march, {self.rows} rows/wave)"
         hz = "hz_" if self.pol == "Hz" else ""
         f = self._f2d
         if f and f.kstep and (hz or self.kernel == "fused"):
@@ -427,8 +429,8 @@ class Grid:
                 n += 1
 
     # ---------------- two-step 3D path ----------------
-    # workgroups of the two-step kernel one CU holds at once, by (rows, waves): VGPRs 112 -> 4 waves per
-    # SIMD (two 8-wave groups); 151 and 202 VGPRs, or 16 waves -> one group
+    # workgroups of the two-step kernel one CU holds at once, by (rows, waves): 97 VGPRs, 123 with three sources and
+    # more -> 4 waves per SIMD (two 8-wave groups); three and four rows (134 to 215 VGPRs), or 16 waves -> one group
     _RESIDENT = {(2, 8): 2, (3, 8): 1, (4, 8): 1, (2, 16): 1}
 
     def kseg2_eff(self):
@@ -1237,7 +1239,8 @@ class Fused2D:
     def _launch(self, count):
         ptr = lambda t: t.data_ptr() if t is not None else None
         g0 = self.grids[0]
-        N.call("bz_yee2d_hz_run" if self.pol == "Hz" else "bz_yee2d_run", self.desc_dev.data_ptr(), len(self.grids), self.tiles.data_ptr(), self.ntiles,
+        N.call("bz_yee2d_hz_run" if self.pol == "Hz" else "bz_yee2d_run", self.desc_dev.data_ptr(), len(self.grids),
+               self.tiles.data_ptr(), self.ntiles,
                self.seg, self.step.data_ptr(), count, ptr(self.pts), self.npts, ptr(self.slot), ptr(self.grp),
                self.nslot, self.nrow, ptr(self.series), self.nfreq, ptr(self.phasor), ptr(self.dft), g0.stream)
 
