@@ -715,7 +715,8 @@ constexpr int ELIST = 192;    // monitor entries of a wave kept in LDS (further 
 // step (LDS round trip, barrier, eight dependent operations) and the launch itself. Measured, whole calls, with
 // 4-value coefficients, two barriers per step, unanchored regions and 128 registers before: 64 grids of 256 x 256
 // cells 15.6 -> 10.7 ms, twelve of 256..1024 a side 4.6 -> 3.2 ms; one grid of 800 x 400 cells with a 16-frequency
-// line 1.33 (K = 12) -> 1.1 us/step (K = 16). HZ, 701 x 403 cells, 1500 steps: 10.0 ms at one step per launch, 3.1.
+// line, 4000 steps 9.2 (K = 12) -> 6.7 ms (K = 16; a launch 21.7 us). HZ, 701 x 403 cells, 1500 steps: 10.0 ms at one
+// step per launch, 3.2.
 // HZ: the (Hz, Ex, Ey) polarisation in the slots of (Ez, Hx, Hy). Its H update reads Ex of the next row and Ey of
 // the next column, its E update Hz of the previous row and column: the bands exchange Ex of the first row and Ex,
 // Ey of the last, and each keeps the Hz of the row above (with its source, which this family adds to Hz).

@@ -25,10 +25,11 @@
 // (clamped in-grid reads) only feed values that are not stored.
 // HBM traffic per two cell-updates: 8 reads + 6 writes of FP32 (56 B) plus
 // the halo columns, rows and planes.
-// What bounds it: on a large grid the issue of about 260 vector operations per halo-inclusive cell pair (20% of the
-// rows and 6% of the columns are halo), at two workgroups of 512 per CU (95 VGPRs); on a small one the serial march
-// of a segment of kseg + 3 planes. Sources and staging box sit in LDS, with the planes on which a wave can meet them
-// worked out once: as kernel arguments tested on every plane they cost 130 spilled scalar registers and 120 VGPRs.
+// What bounds it: on a large grid HBM (480x240x160: 1.228 GB a pair, 1.19 times one pass, at 4.35 TB/s, 0.89 of a large
+// copy; vector ALUs 40% busy, waves waiting 64% of their time), at two workgroups of 512 per CU (97 VGPRs); on a small
+// one the serial march of a segment of kseg + 3 planes. Sources and staging box sit in LDS, with the planes on which a
+// wave can meet them worked out once: as kernel arguments tested on every plane they cost 130 spilled scalar registers
+// and 120 VGPRs.
 // us per pair before / after: 480x240x160 295 / 286, 300x200x100 112 / 97, 200x120x64 46 / 37, 120x72x40 24 / 20.
 // Tried and slower: 80 VGPRs for three workgroups per CU (20 spills: 609 at 480x240x160, 31 at 120x72x40), loads one
 // plane ahead (378 at 480x240x160), three rows per wave (322), 16 waves (22 at 120x72x40).

@@ -991,10 +991,10 @@ class Fused2D:
     # 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two, not three, on many grids
     DENSE_MIN = 64
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
-    # (K, rows, waves) candidates of tune_kstep. Forward sweeps: 64 grids of 256 x 256 cells 4.95 / 5.05 us/step
-    # for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 4.49 / 4.45; 16 grids of 600 x 600 cells
-    # 5.81 / 5.79 against 6.47 for (12, 4, 16); one 800 x 400 grid 1.16 for (16, 4, 16), 1.42 for (8, 4, 8), 1.33
-    # for (12, 4, 16); one 256 x 256 grid 1.07 for (12, 4, 8), 1.11 for (16, 4, 16), 1.28 for (16, 8, 8)
+    # (K, rows, waves) candidates of tune_kstep. Forward sweeps with one monitor line, us/step: 64 grids of 256 x 256 cells
+    # 5.2 / 5.7 for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 6.1 / 6.3; 16 grids of 600 x 600
+    # cells 6.5 / 6.5 against 7.5 for (12, 4, 16); one 800 x 400 grid 1.51 for (16, 4, 16), 1.53 for (8, 4, 8), 1.45 for
+    # (12, 4, 16); one 256 x 256 grid 1.15 for (12, 4, 8), 1.24 for (16, 4, 16), 1.35 for (16, 8, 8)
     KCANDIDATES = ((8, 8, 8), (12, 8, 8), (8, 4, 8), (12, 4, 8), (16, 4, 16))
 
     def kstep_applies(self):
