@@ -213,29 +213,3 @@ def test_several_sources_in_a_region(hip, monkeypatch, count, shape, dense, pol)
         assert bool(g._f2d.kstep) == bool(k)
     for n in out[0]:
         assert np.any(out[0][n]) and np.array_equal(out[0][n], out[1][n], equal_nan=True), n
-
-
-def test_several_sources_are_not_slow(hip):
-    """Eight sources over a grid take no more than 1.45 times one (once 1.7: each cell read its own source's sample from
-    memory at the end of every step)."""
-    import time
-
-    import torch
-    batches = []
-    for n in (1, 8):
-        s, _ = world(800, 400, 2200, False, 1, "Ez")
-        s.monitors = []
-        s.sources = [bz.GaussianSource(position=((20 + 105 * (q % 7)) * DX, (20 + 45 * (q // 7)) * DX), width=DX / 4,
-                                       signal=np.cos(0.05 * np.arange(2200))) for q in range(n)]
-        batches.append(FDTDBatch([s]))
-        batches[-1].initialize()
-        batches[-1].advance(192)
-    best = [1e9, 1e9]
-    for _ in range(8):
-        for q, b in enumerate(batches):
-            torch.cuda.synchronize()
-            t0 = time.perf_counter()
-            b.advance(192)
-            torch.cuda.synchronize()
-            best[q] = min(best[q], time.perf_counter() - t0)
-    assert best[1] < 1.45 * best[0], best
