@@ -988,8 +988,12 @@ class Fused2D:
     PART_MIN, PART_ALONE = 2, 10
     # Most monitor entries (point and component) in the rows of one wave for which that wave takes the samples; above, the
     # workgroup does. us/step by wave / by workgroup: 1024 x 1024, 3 columns (72 entries) 3.0 / 2.4, 12 (288) 21.9 / 3.0;
-    # 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two, not three, on many grids
-    DENSE_MIN = 64
+    # 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two regions, not three: with more
+    # regions than are resident at once, only where a wave's list (DENSE_LIST) or a region (DENSE_TILE) has too many:
+    # 16 x 600 x 600, a row (192 in one wave) 6.2 / 7.1, 3 columns (432 in a region) 7.1 / 7.3, 6 (864) 8.4 / 7.8; 64 x 256 x
+    # 256 5.4 / 5.8, 6.2 / 5.9, 7.3 / 6.3; 1200 x 1200 3.0 / 3.2, 3.4 / 3.2, 4.1 / 3.3
+    DENSE_MIN, DENSE_LIST, DENSE_TILE = 64, 192, 576
+    RESIDENT = 512          # regions that 256 CUs hold at two per CU
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
     # (K, rows, waves) candidates of tune_kstep. Forward sweeps with one monitor line, us/step: 64 grids of 256 x 256 cells
     # 5.2 / 5.7 for (8, 8, 8) / (12, 8, 8); twelve grids of 256..1024 cells a side 6.1 / 6.3; 16 grids of 600 x 600
@@ -1071,7 +1075,9 @@ class Fused2D:
             dims = np.array([(g.nx, g.ny, g.ld) for g in self.grids], np.int64)
             start, ents = kstep_owner_tables(tiles, self._pts_host, dims, K, rows * waves)
             wave = np.repeat(np.arange(len(tiles)) * waves, np.diff(start)) + (ents[:, 1] >> 10) // rows
-            self.dense = bool(np.bincount(wave, minlength=1).max() > self.DENSE_MIN)
+            tight = len(tiles) <= self.RESIDENT or np.diff(start).max() > self.DENSE_TILE
+            limit = self.DENSE_MIN if tight else max(self.DENSE_MIN, self.DENSE_LIST)
+            self.dense = bool(np.bincount(wave, minlength=1).max() > limit)
             self.ents = T.from_numpy(ents.ravel()).to(self.dev)
             self.ent_start = T.from_numpy(start).to(self.dev)
             self.stagek = T.zeros(2 * K * self.npts, dtype=T.float32, device=self.dev)   # two slots: q & 1

@@ -86,3 +86,17 @@ def test_dense_monitor_points_are_those_past_one_entry_per_lane(points, dense):
         g.add_gather(comps, np.tile(off, 3), np.arange(8), np.arange(9.0), None)
     e = Fused2D([g], kstep=8, krows=4, kwaves=16)
     assert e.dense == dense
+
+
+@pytest.mark.parametrize("points,dense", [([(20, i) for i in range(50)], False),
+                                          ([(j, i) for j in (20, 30) for i in range(50)], False),
+                                          ([(j, i) for j in (20, 21) for i in range(50)], True),
+                                          ([(j, i) for j in (4, 8, 20, 30) for i in range(50)], True)])
+def test_dense_monitor_points_of_many_regions(monkeypatch, points, dense):
+    """More regions than are resident at once: the workgroup takes the samples where a wave has more than 192 entries,
+    or a region more than 576 and some wave more than 64."""
+    monkeypatch.setattr(Fused2D, "RESIDENT", 0)
+    g = grid("Ez")
+    off = np.array([g.offset(0, j, i) for j, i in points])
+    g.add_gather(np.repeat(np.arange(3), len(off)), np.tile(off, 3), np.arange(8), np.arange(9.0), None)
+    assert Fused2D([g], kstep=8, krows=4, kwaves=16).dense == dense
