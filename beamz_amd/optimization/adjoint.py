@@ -411,9 +411,10 @@ class AdjointProblem2D:
                         e1.record()
                         T.cuda.synchronize(self.dev)
                         ms[shape] = min(ms.get(shape, 1e30), e0.elapsed_time(e1))
-                # within 3 % of the fastest, the most steps per launch wins: a window of 192 steps favours fewer steps
-                # per launch a little against whole sweeps (16 designs of 600 x 600 cells: about 1.5 % between two
-                # shapes of which the other was 0 to 5 % faster over 3000 steps)
+                # within 3 % of the fastest, the most steps per launch wins: windows of 192 steps timed an earlier
+                # kernel's 6 steps 1.5 % ahead of its 8, which over 3000 steps were as fast or faster. (Now, 16 designs
+                # of 600 x 600 cells: 8 steps 2 to 3 % ahead of 12, and 26.1 against 27.2 ms a gradient: either may
+                # be taken there)
                 best = min(ms.values())
                 self.rec.set_kstep(*max((c for c in ms if ms[c] <= 1.03 * best), key=lambda c: (c[0], -ms[c])))
                 self.rev_timings = ms
