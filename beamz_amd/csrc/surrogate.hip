@@ -525,7 +525,8 @@ __global__ __launch_bounds__(64 * (W / 32) * (CB / 32)) void k_conv_march(const 
 // replace (92 -> 125 us), so those layers take k_conv_tile.
 template <int CC>
 __global__ __launch_bounds__(256) void k_conv_halo(const uint16_t* __restrict__ src, const uint16_t* __restrict__ wk,
-                                                   const float* __restrict__ bias, uint16_t* __restrict__ out, const uint16_t* __restrict__ mask, Geo g,
+                                                   const float* __restrict__ bias, uint16_t* __restrict__ out,
+                                                   const uint16_t* __restrict__ mask, Geo g,
                                                    int Cs, int N, int sign, int relu) {
     constexpr int SLD = CC + 8;              // halfwords per halo slot (16-byte pad: conflict-free reads)
     constexpr int KS = CC / 16;              // MFMA k-steps per tap and chunk

@@ -986,12 +986,13 @@ class Fused2D:
     # 800 x 400, 8 steps 84 / 58; alone (with the pass over the coefficients) 10 steps 50 / 36, at 1000 x 990 8 steps
     # 67 / 68 ((Hz, Ex, Ey): 69 / 79), 10 steps 82 / 71 (85 / 84)
     PART_MIN, PART_ALONE = 2, 10
-    # Most monitor entries (point and component) in the rows of one wave for which that wave takes the samples; above, the
-    # workgroup does. us/step by wave / by workgroup: 1024 x 1024, 3 columns (72 entries) 3.0 / 2.4, 12 (288) 21.9 / 3.0;
-    # 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two regions, not three: with more
-    # regions than are resident at once, only where a wave's list (DENSE_LIST) or a region (DENSE_TILE) has too many:
-    # 16 x 600 x 600, a row (192 in one wave) 6.2 / 7.1, 3 columns (432 in a region) 7.1 / 7.3, 6 (864) 8.4 / 7.8; 64 x 256 x
-    # 256 5.4 / 5.8, 6.2 / 5.9, 7.3 / 6.3; 1200 x 1200 3.0 / 3.2, 3.4 / 3.2, 4.1 / 3.3
+    # Most monitor entries (point and component) in the rows of one wave for which that wave takes the samples; above,
+    # the workgroup does. us/step by wave / by workgroup: 1024 x 1024, 3 columns (72 entries) 3.0 / 2.4, 12 (288) 21.9
+    # / 3.0; 800 x 400, 6 columns (72) 2.0 / 1.8, 3 rows (576) 5.1 / 1.7. By workgroup a CU holds two regions, not
+    # three: with more regions than are resident at once, only where a wave's list (DENSE_LIST) or a region
+    # (DENSE_TILE) has too many: 16 x 600 x 600, a row (192 in one wave) 6.2 / 7.1, 3 columns (432 in a region) 7.1 /
+    # 7.3, 6 (864) 8.4 / 7.8; 64 x 256 x 256 5.4 / 5.8, 6.2 / 5.9, 7.3 / 6.3; 1200 x 1200 3.0 / 3.2, 3.4 / 3.2, 4.1 /
+    # 3.3
     DENSE_MIN, DENSE_LIST, DENSE_TILE = 64, 192, 576
     RESIDENT = 512          # regions that 256 CUs hold at two per CU
     KSHAPES = ((8, 4), (8, 8), (8, 16), (4, 8), (4, 16), (16, 4))     # (rows per wave, waves per workgroup)
